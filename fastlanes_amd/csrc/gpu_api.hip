@@ -10,6 +10,7 @@
 #include "launch.hpp"
 #include "page_kernels.hpp"
 #include "gpu_internal.hpp"
+#include "rowgroup.hpp"
 
 namespace fls {
 
@@ -84,14 +85,15 @@ const Column& plan_column(const fls_gpu_plan* p) { return p->col; }
 const void*   plan_dictionary(const fls_gpu_plan* p, size_t page) {
     return page < p->dicts.size() ? p->dicts[page].values : nullptr;
 }
-int plan_decode_dictionaries(fls_gpu_plan* p, const uint8_t* dev_encoded, hipStream_t s) {
+void plan_dictionary_jobs(const fls_gpu_plan* p, uint64_t dev_off, std::vector<DictJob>& jobs) {
     for (size_t i = 0; i < p->col.pages.size(); ++i) {
-        const DevDict& d = p->dicts[i];
-        if (!d.n_chunks) continue;
-        hipError_t e = launch_hzl(p->DW, dev_encoded, d.chunks, d.n_chunks, d.values, d.exc, s);
-        if (e != hipSuccess) return hip_fail(e, "dictionary launch");
+        if (!p->dicts[i].n_chunks) continue;
+        bool exc = false;
+        for (HzlChunk ch : device_chunks(p->col.pages[i].hzl, exc, p->DW)) {
+            ch.src += dev_off;
+            jobs.push_back({ch, (uint64_t)(uintptr_t)p->dicts[i].values, p->DW, 0});
+        }
     }
-    return FLS_OK;
 }
 }  // namespace fls
 

@@ -1110,36 +1110,32 @@ __global__ __launch_bounds__(kMaxBlock) void k_page_dict(const uint8_t* __restri
 // order (the lane-major order of unffor); the raw tail is copied; exceptions are patched by a second launch.
 // ---------------------------------------------------------------------------------------------------------------
 
-// One block per chunk, one thread per (value row j, lane): every thread extracts its value straight from the two
+// A block decodes one chunk, one thread per (value row j, lane): every thread extracts its value straight from the two
 // packed words that hold it (word floor(j*bw/DW) and the next of its lane), so a chunk decodes with one round of
 // loads instead of a serial walk over its rows. Output in array order: out[j * L + lane] = value + base.
+template <typename D>
+__device__ __forceinline__ void hzl_chunk(const uint8_t* in, const HzlChunk& ch, D* out) {
+    const uint32_t n = ch.bw == 255 ? ch.n : 1024u;
+    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) out[k] = hzl_value<D>(in, ch, k);
+}
 template <int DW>
 __global__ __launch_bounds__(1024) void k_hzl_chunks(const uint8_t* __restrict__ enc, const HzlChunk* chunks,
                                                      uint32_t n_chunks, uint8_t* __restrict__ dict) {
-    using D                = typename uint_of<DW>::type;
-    constexpr unsigned L   = 1024 / DW;
+    using D = typename uint_of<DW>::type;
     for (uint32_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
-        const HzlChunk ch  = chunks[c];
-        D*             out = reinterpret_cast<D*>(dict + ch.dst * sizeof(D));
-        const uint8_t* in  = enc + ch.src;
-        if (ch.bw == 255) {
-            for (uint32_t k = threadIdx.x; k < ch.n; k += blockDim.x) out[k] = load_t<D>(in + (uint64_t)k * sizeof(D));
-            continue;
-        }
-        const unsigned bw   = ch.bw;
-        const D        base = (D)ch.base;
-        const D        mask = bw >= DW ? (D)~(D)0 : (D)(((D)1 << bw) - 1);
-        for (uint32_t k = threadIdx.x; k < 1024; k += blockDim.x) {
-            const unsigned j = k / L, lane = k % L;
-            D              v = 0;
-            if (bw) {
-                const unsigned bit = j * bw, w = bit / DW, sh = bit % DW;
-                v                  = load_t<D>(in + ((uint64_t)w * L + lane) * sizeof(D)) >> sh;
-                if (sh + bw > DW) v |= load_t<D>(in + ((uint64_t)(w + 1) * L + lane) * sizeof(D)) << (DW - sh);
-                v &= mask;
-            }
-            out[k] = (D)(v + base);
-        }
+        const HzlChunk ch = chunks[c];
+        hzl_chunk<D>(enc + ch.src, ch, reinterpret_cast<D*>(dict) + ch.dst);
+    }
+}
+// Exceptions of an FFOR chunk: positions (u16), then values, behind its packed rows.
+template <typename D>
+__device__ __forceinline__ void hzl_chunk_exceptions(const uint8_t* in, const HzlChunk& ch, D* out) {
+    if (ch.bw == 255 || ch.exc_c == 0) return;
+    const uint8_t* pos = in + 128ull * ch.bw;
+    const uint8_t* val = pos + 2ull * ch.exc_c;
+    for (uint32_t e = threadIdx.x; e < ch.exc_c; e += blockDim.x) {
+        const uint32_t p = *reinterpret_cast<const u16_ua*>(pos + 2ull * e);
+        if (p < 1024) out[p] = load_t<D>(val + (uint64_t)e * sizeof(D));
     }
 }
 template <int DW>
@@ -1148,14 +1144,7 @@ __global__ __launch_bounds__(256) void k_hzl_exceptions(const uint8_t* __restric
     using D = typename uint_of<DW>::type;
     for (uint32_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
         const HzlChunk ch = chunks[c];
-        if (ch.bw == 255 || ch.exc_c == 0) continue;
-        const uint8_t* pos = enc + ch.src + 128ull * ch.bw;
-        const uint8_t* val = pos + 2ull * ch.exc_c;
-        D*             out = reinterpret_cast<D*>(dict) + ch.dst;
-        for (uint32_t e = threadIdx.x; e < ch.exc_c; e += blockDim.x) {
-            const uint32_t p = *reinterpret_cast<const u16_ua*>(pos + 2ull * e);
-            if (p < 1024) out[p] = load_t<D>(val + (uint64_t)e * sizeof(D));
-        }
+        hzl_chunk_exceptions<D>(enc + ch.src, ch, reinterpret_cast<D*>(dict) + ch.dst);
     }
 }
 

@@ -64,6 +64,14 @@ constexpr unsigned kRgDump       = 16;    // LDS bytes at the end of a wave slot
 // every 256 (the threads' 16-byte words land on different banks), read back lane-consecutively for the stores.
 constexpr unsigned rg_out_lds(unsigned W) { return 128 * W + 8 * W; }
 
+// A chunk of one of a row-group's dictionaries: `ch.src` counts from the row-group's encoded buffer, `dict` is the
+// device address of the dictionary's first value.
+struct DictJob {
+    HzlChunk ch;
+    uint64_t dict;
+    uint32_t dw, pad;  // value width, 32 or 64
+};
+
 // Element width (bits) of a kind's decoded values.
 unsigned rg_kind_bits(int kind);
 

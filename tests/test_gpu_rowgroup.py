@@ -217,3 +217,44 @@ def test_rowgroup_large_single_page_columns(torch_cuda, oracle):
         rg.decode(d_enc.data_ptr(), d_out.data_ptr(), 0, fa.stream_ptr())
         verify(torch, rg, d_out, want, f"large columns, run {rep}")
 
+
+
+@pytest.mark.parametrize("dtype", [np.uint32, np.uint64])
+def test_rowgroup_dictionary_chunks(torch_cuda, oracle, dtype):
+    """Dictionaries of one launch: a chunk with exceptions (hand-built: bit width 3 with two exceptions, as the
+    reference's HZL compressor writes them, src/cor/eng/hzl_cmp.cpp), a raw tail alone, whole chunks and a tail, and a
+    column without a dictionary between them, decoded twice into other buffers."""
+    torch = torch_cuda
+    ddt = np.dtype(dtype)
+    print(f"rowgroup dictionary chunks {ddt.name}", flush=True)
+    x = np.tile((np.arange(1024, dtype=np.uint64) * 1000 + 5).astype(dtype), 4)
+    enc = fa.encode_from_memory(x, 17)
+    dict_len = 8 + 12 + 128 * int(1023 * 1000).bit_length() + 12
+    want = (100 + np.arange(1024) % 8).astype(dtype)
+    hdr, tail = np.zeros(12, np.uint8), np.zeros(12, np.uint8)
+    hdr[0], hdr[2], tail[0] = 3, 2, 255
+    hdr[4:12] = np.frombuffer(np.uint64(100).tobytes(), np.uint8)
+    blob = np.concatenate([enc[:8], hdr, oracle.ffor(want, 3, ddt.type(100)).view(np.uint8),
+                           np.array([7, 1000], np.uint16).view(np.uint8), np.array([123456, 42], dtype).view(np.uint8),
+                           tail, enc[dict_len:]])
+    want[7], want[1000] = 123456, 42
+    g = np.random.default_rng(3)
+    few = g.integers(0, 1 << 30, 5).astype(dtype)[g.integers(0, 5, 3 * 1024)]
+    many = g.permutation(1 << 20)[:2500].astype(dtype)
+    many = np.concatenate([many, many[g.integers(0, 2500, 5 * 1024 - 2500)]])
+    plain = np.arange(2048, dtype=dtype)
+    cols = [(blob, np.tile(want, 4)), (fa.encode_from_memory(few, 17), few), (fa.encode_from_memory(plain, 1), plain),
+            (fa.encode_from_memory(many, 22), many)]
+    offs, pos = [], 64  # the first column does not start at byte 0
+    for e, _ in cols:
+        offs.append(pos)
+        pos = (pos + e.size + 255) // 256 * 256
+    host = np.zeros(pos + 16, np.uint8)
+    for o, (e, _) in zip(offs, cols):
+        host[o: o + e.size] = e
+    rg = fa.RowGroup([e for e, _ in cols], [ddt] * len(cols), offs)
+    for _ in range(2):
+        d_enc = torch.from_numpy(host).cuda()
+        d_out = torch.full((rg.total_bytes,), 0xA5, dtype=torch.uint8, device="cuda")
+        rg.decode(d_enc.data_ptr(), d_out.data_ptr(), 0, fa.stream_ptr())
+        verify(torch, rg, d_out, [w for _, w in cols], "dictionary chunks")
