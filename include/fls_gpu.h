@@ -89,14 +89,14 @@ int fls_gpu_selection_and(const uint64_t* dev_a, const uint64_t* dev_b, uint64_t
  * of src/cor/eng/compressor.cpp:41-86): encodes n device-resident values (n a multiple of 1024) of `type` with
  * pool expression 0 (UNCOMPRESSED), 1 (FFOR), 11 (DELTA), 6 or 7 (RLE) into dev_out, the same bytes encode_from_memory writes
  * for those values. *out_size receives the encoded size (also when it exceeds `capacity`, which returns
- * FLS_E_CAPACITY and writes nothing). Reads the per-vector bit widths back to lay out the pages, so it returns
- * after `stream` has completed. */
+ * FLS_E_CAPACITY and writes nothing). The pages are laid out on the device and only the size is read back, so it
+ * returns after `stream` has completed. */
 int fls_gpu_encode(const void* dev_values, uint64_t n, enum data_t type, uint8_t expr_id, uint8_t* dev_out,
                    uint64_t capacity, uint64_t* out_size, void* stream);
 /* fls_gpu_encode without device allocation. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
- * The encoder's scratch (per-vector bit widths, bases, buffer offsets and the page table) is a fixed device array
- * of about 1.1 MiB per GPU, kept until the process ends, instead of stream allocations; n is at most 2^24 values
+ * The encoder's scratch (per-vector bit widths, bases, their sums and the page table) is a fixed device array
+ * of about 160 KiB per GPU, kept until the process ends, instead of stream allocations; n is at most 2^24 values
  * (FLS_E_CAPACITY beyond). Every call on one GPU shares that GPU's array: calls that overlap on one GPU race.
  * Same bytes, errors and synchronization as fls_gpu_encode. */
 int fls_gpu_encode_noalloc(const void* dev_values, uint64_t n, enum data_t type, uint8_t expr_id, uint8_t* dev_out,

@@ -685,3 +685,49 @@ def test_gpu_encoder_multi_page_and_capacity(torch_cuda):
         del d_out
     with pytest.raises(fa.FlsError):
         fa.gpu_encode(d_x.data_ptr(), x.size, np.int64, 11, d_x.data_ptr(), 100)
+
+
+@pytest.mark.parametrize("eid", [1, 11])
+@pytest.mark.parametrize("dtype", [np.uint8, np.uint16, np.uint32, np.uint64, np.int64])
+def test_gpu_encoder_every_bit_width(torch_cuda, dtype, eid):
+    """One vector of every bit width 0 .. W (W = 64: parts of a lane that end inside a word, and words that several
+    parts share), full-range values among them, from an input that is aligned to its element type only."""
+    torch = torch_cuda
+    print(f"gpu encode every bit width dtype={np.dtype(dtype).name} expr={eid}", flush=True)
+    W = np.dtype(dtype).itemsize * 8
+    g = np.random.default_rng(W + eid)
+    rows = []
+    for w in range(W + 1):
+        top = (1 << w) - 1
+        r = g.integers(0, top, 1024, dtype=np.uint64, endpoint=True)
+        r[g.permutation(1024)[:2]] = (0, top)  # exactly w bits
+        rows.append(np.cumsum(r, dtype=np.uint64) if eid == 11 else r + np.uint64((1 << W) - 1 - top) // np.uint64(2))
+    x = np.concatenate(rows).astype(np.dtype(f"u{W // 8}")).view(dtype)
+    want = fa.encode_from_memory(x, eid)
+    buf = torch.zeros(x.nbytes + W // 8, dtype=torch.uint8, device="cuda")
+    buf[W // 8:] = torch.from_numpy(x.view(np.uint8)).cuda()
+    d_out = torch.full((want.size + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    size = fa.gpu_encode(buf.data_ptr() + W // 8, x.size, dtype, eid, d_out.data_ptr(), want.size)
+    assert size == want.size
+    np.testing.assert_array_equal(d_out[:size].cpu().numpy(), want)
+    assert bool((d_out[size:] == 0x5A).all())  # nothing past the encoded bytes
+
+
+def test_gpu_encoder_pages_of_runs(torch_cuda):
+    """A page that reaches 128 MiB inside its even split, by run values and by packed rows, with a small odd rest; and
+    one vector more than the page limit."""
+    torch = torch_cuda
+    g = np.random.default_rng(5)
+    x = np.repeat(g.integers(0, 1 << 62, 20_003 * 512, dtype=np.int64), 2)  # 512 runs a vector: 4 KB + 2 KB
+    x = np.concatenate([x, x[: 1024 * 5_000]])
+    for eid, v in ((7, x), (1, x), (6, np.zeros(65_536 * 1024, np.uint8))):
+        want = fa.encode_from_memory(v, eid)
+        d_x = dev(torch, v)
+        d_out = torch.zeros(want.size, dtype=torch.uint8, device="cuda")
+        size = fa.gpu_encode(d_x.data_ptr(), v.size, v.dtype, eid, d_out.data_ptr(), want.size)
+        assert size == want.size
+        assert torch.equal(d_out.cpu(), torch.from_numpy(want)), eid
+        with pytest.raises(fa.FlsError):  # one byte short: nothing is written
+            d_out.fill_(7)
+            fa.gpu_encode(d_x.data_ptr(), v.size, v.dtype, eid, d_out.data_ptr(), want.size - 1)
+        assert bool((d_out == 7).all())
