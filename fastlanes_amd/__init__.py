@@ -157,7 +157,7 @@ class Plan:
               "decode_strings")
 
     def decode_strings_fused(self, dev_encoded_ptr, dev_offsets_ptr, dev_bytes_ptr, cap, stream: int = 0) -> None:
-        """Offsets and bytes in one pass (one launch per page)."""
+        """Offsets and bytes in one call."""
         check(lib().fls_gpu_plan_decode_strings_fused(self.h, dev_encoded_ptr, dev_offsets_ptr, dev_bytes_ptr, cap,
                                                       stream), "decode_strings_fused")
 
@@ -270,7 +270,7 @@ class RowGroup:
         check(lib().fls_gpu_rowgroup_check(self.h, stream), "rowgroup_check")
 
     def decode_strings_fused(self, dev_encoded_ptr, dev_offsets_ptr, dev_bytes_ptr, cap, stream: int = 0) -> None:
-        """Offsets and bytes in one pass (one launch per page)."""
+        """Offsets and bytes in one call."""
         check(lib().fls_gpu_plan_decode_strings_fused(self.h, dev_encoded_ptr, dev_offsets_ptr, dev_bytes_ptr, cap,
                                                       stream), "decode_strings_fused")
 

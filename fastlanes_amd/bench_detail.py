@@ -102,7 +102,7 @@ def cascade(dev, stream, log2n=26, log2_strings=24, verbose=True):
     d_bytes = torch.empty(data.size + 64, dtype=torch.uint8, device=dev)
     sp = int(stream.cuda_stream)
 
-    def fn():  # offsets and bytes in one pass
+    def fn():  # offsets and bytes in one call
         plan.decode_strings_fused(d_in.data_ptr(), d_off.data_ptr(), d_bytes.data_ptr(), data.size, sp)
 
     t = _events_time(fn, stream, reps=3)

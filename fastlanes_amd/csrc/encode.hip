@@ -53,7 +53,7 @@ __device__ __forceinline__ void enc_wave_sync() {
 // A block of the analyze and pack kernels takes a group of 32 consecutive vectors, a wave an equal run of them (their
 // small metadata stores share cache lines); prefix sums are kept per group, and a wave scans a group's widths with one
 // lane per vector. Large columns run 4 waves of 8 vectors; while the groups are too few to fill the device, 16 waves
-// of 2, because a wave's vectors follow one another: 64 vectors of uint32 37 us with 8 in a row, 25 us with 2.
+// of 2, because a wave's vectors follow one another: 64 vectors of uint32 37 us with 8 in a row, 31 us with 2.
 constexpr unsigned kEncGroup = 32, kEncMaxWaves = 16;
 __host__ __device__ constexpr unsigned enc_waves(uint32_t n_vec) {
     return (n_vec + kEncGroup - 1) / kEncGroup < 1024 ? kEncMaxWaves : 4;

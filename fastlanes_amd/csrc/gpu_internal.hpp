@@ -15,14 +15,19 @@ int hip_fail(hipError_t e, const char* what);
 // Device-side FSST symbol table (include/fls/cor/prm/fsst/fsst.h:92-98 without the version/terminator fields).
 struct FsstTableDev {
     uint64_t symbol[256];
+    uint64_t packed[256];  // kind 0 (symbols of at most 3 bytes): symbol, 8 len above bit 32; 1 (at most 7): symbol, len
+                           // above bit 56; 2: symbol
     uint8_t  len[256];
+    uint32_t kind;
 };
 
 struct StringPlan {
     FsstTableDev* d_tables = nullptr;  // one per page entry
-    uint64_t*     d_status = nullptr;  // look-back status word per half-vector segment (zeroed once)
-    uint64_t*     d_ticket = nullptr;  // look-back tickets: counter (never reset), the call's base, its epoch
-    uint32_t*     d_err    = nullptr;  // error bits: capacity, look-back
+    void*         d_segs   = nullptr;  // FsstSeg of every segment (k_fsst.hip)
+    uint64_t*     d_vecs   = nullptr;  // every vector's decoded bytes, then the sums before each
+    uint32_t*     d_ends   = nullptr;  // every string's end within its segment
+    uint16_t*     d_sizes  = nullptr;  // decoded bytes of every 32 compressed bytes (k_fsst.hip)
+    uint32_t*     d_err    = nullptr;  // error bits: capacity
     uint64_t      n_vec    = 0;
 };
 

@@ -6,21 +6,25 @@
 // with fsst_decompress (include/fls/cor/prm/fsst/fsst.h:152-258): code < 255 emits symbol[code] (len[code] bytes),
 // code 255 emits the next byte literally.
 //
-// One kernel, one pass over the compressed bytes. A block of 512 threads owns one half-vector segment (512
-// strings). Its compressed bytes are split into equal 32-byte-aligned shares, one per thread, read straight from
-// HBM into registers:
-//   1. count: each thread adds up the decoded length of its share (a byte is a literal when it follows an odd run
-//      of 255 bytes inside its string; an escape emits one byte, a code c emits len[c]);
-//   2. one block scan of (bytes, string starts) gives every share its output position and the rank of its first
-//      string start;
-//   3. walk: each thread walks its share again, records the output position of every string start it passes, and
-//      ORs its decoded bytes, 8 at a time, into a zeroed LDS image of the segment's output;
-//   4. the segment's output base comes from a decoupled look-back over the column's segments (a status word per
-//      segment: aggregate, then inclusive prefix; blocks take segments in dispatch order from a ticket counter so
-//      every segment they wait on is already running), or from the caller's offsets;
-//   5. the LDS image is copied out with coalesced 16-byte stores, and the string end offsets are written.
-// Segments that are malformed (non-monotone offsets), larger than the LDS image, or whose compressed bytes exceed
-// the start bitmap, take a per-string path that reads and writes global memory byte by byte.
+// A block of 256 threads owns one segment (256 strings of a vector), whose compressed bytes it takes in chunks of 8 KiB, 32
+// bytes (a granule) per thread, read straight from HBM into registers. Launches:
+//   k_fsst_count  every granule's and segment's decoded size, and the strings' ends in order;
+//   k_fsst_scan   the vectors' output bases, when they are too many for each block to sum them itself;
+//   k_fsst        per chunk: one block scan of the granules' sizes; each thread joins its symbols into 8-byte words of the
+//                 LDS image of the output (44 of its 76 vector instructions per four codes), which is copied out with
+//                 16-byte stores aligned to the output, and leaves the packed exclusive prefix of its codes' lengths in
+//                 LDS: a string's end is its granule's base plus one byte of it.
+// The bases came from a decoupled look-back in one pass over the compressed bytes before: its dispatch-order tickets (one
+// same-address atomic per segment) and waits took 48 of 135 us for 2^21 strings of 36 bytes. Every symbol was OR-ed into
+// a zeroed image by an LDS atomic; now a word is stored by the one thread that has its last byte, and threads that have
+// only earlier bytes of it OR them in after a barrier. (Writing each symbol's 8 bytes at its own unaligned place, two
+// instructions per code, measured 135 us: unaligned LDS writes take about one cycle per lane.) 2^21 strings: 151 -> 71 us
+// a call, k_fsst 42, bound by its vector instructions. No variable of k_fsst may spill: a build whose registers did gave
+// wrong bytes in a hundredth of the segments.
+// Segments that are malformed (non-monotone offsets) take a per-string path that reads and writes global memory byte by
+// byte.
+#include <algorithm>
+
 #include "../../include/fls_gpu.h"
 #include "gpu_internal.hpp"
 #include "page_kernels.hpp"
@@ -29,195 +33,62 @@ namespace fls {
 
 namespace {
 
-constexpr unsigned kSeg      = 512;        // strings per segment (= threads per block)
+constexpr unsigned kSeg      = 256;         // strings per segment (= threads per block)
 constexpr unsigned kSegPerV  = 1024 / kSeg;
 constexpr unsigned kWaves    = kSeg / 64;
-constexpr uint32_t kMaxComp  = 32 * 1024;  // compressed bytes of a segment on the byte-parallel path
-constexpr uint32_t kOutLds   = 24 * 1024;  // decoded bytes of a segment assembled in LDS
-constexpr uint32_t kShare    = 32;         // share granule: one word of the start bitmap
-
-constexpr unsigned kCallBase = 16;  // u64 index of the call state, 128 bytes past the ticket counter
+constexpr uint32_t kShare    = 32;          // compressed bytes per thread and chunk
+constexpr uint32_t kChunk    = kShare * kSeg;
+constexpr uint32_t kOutLds   = 12 * 1024;   // bytes of the LDS image of decoded output
+constexpr uint32_t kMaxComp  = 1u << 28;    // compressed bytes of a segment whose decoded size is below 2^32
+constexpr unsigned kWideCount = 1024;       // vectors of a page that k_fsst_count takes with 1024 threads each
+constexpr unsigned kDirect   = 1024;        // vectors of a column whose sizes each block sums itself (4 loads per thread)
 
 // error bits (StringPlan::d_err)
-constexpr uint32_t kErrCap = 4, kErrSpin = 16, kErrTicket = 32;
-
-// Segment status word of the look-back: [63:48] call epoch, [47:46] flag, [45:0] decoded bytes.
-constexpr uint64_t kFlagAgg = 1, kFlagPrefix = 2, kValMask = (1ull << 46) - 1;
-
-struct SegCtl {
-    uint64_t* status;       // one word per segment of the column
-    uint64_t* ticket;       // [0] dispatch-order ticket counter (never reset); [kCallBase] its value when the call
-                            // began, [kCallBase + 1] the call's epoch (1..65535), on a cache line of their own: set on
-                            // the device by k_begin_call, so a captured graph of a call stays valid on replay
-    uint64_t  ticket_off;   // tickets taken by the call's earlier page launches
-    uint64_t  seg0;         // column-wide index of the page's first segment
-    uint32_t  spin_limit;   // look-back polls before giving up (error bit kErrSpin)
-};
-
-__device__ __forceinline__ uint64_t status_word(uint32_t epoch, uint64_t flag, uint64_t v) {
-    return ((uint64_t)epoch << 48) | (flag << 46) | (v & kValMask);
-}
+constexpr uint32_t kErrCap = 4;
 
 enum : int { FS_OFFSETS = 0, FS_BYTES = 1, FS_ALL = 2 };
 
-// transposed index of original position i (inverse of untranspose_i): i = r + 8*ORDER[b] + 64c -> 128r + 16b + c
-__device__ __forceinline__ unsigned transposed_of(unsigned i) {
-    const unsigned c = i >> 6, b = order8((i >> 3) & 7), r = i & 7;
-    return 128 * r + 16 * b + c;
-}
+// Place in LDS of the end offset of string i, which is transposed: i = r + 8*ORDER[b] + 64c sits at 128r + 16b + c. Rows
+// of 140 dwords and runs of 17 keep 32 consecutive strings on 16 banks; unpadded they share two.
+constexpr unsigned kEndRow = 140;
+__device__ __forceinline__ unsigned end_place(unsigned i) { return (i & 7) * kEndRow + order8((i >> 3) & 7) * 17 + (i >> 6); }
 
-// Exclusive scan of one u64 per thread over the block; returns the block total in *total.
-__device__ __forceinline__ uint64_t block_exclusive_scan(uint64_t x, uint64_t* total) {
-    __shared__ uint64_t wsum[kWaves];
-    const unsigned      lane = threadIdx.x % 64, w = threadIdx.x / 64;
-    uint64_t            inc  = x;
+// Exclusive scan of one value per thread over the block; returns the block total in *total.
+template <typename U>
+__device__ __forceinline__ U block_exclusive_scan(U x, U* wsum, U* total) {
+    const unsigned lane = threadIdx.x % 64, w = threadIdx.x / 64;
+    U              inc  = x;
     for (unsigned d = 1; d < 64; d <<= 1) {
-        const uint64_t y = __shfl_up(inc, d, 64);
+        const U y = __shfl_up(inc, d, 64);
         if (lane >= d) inc += y;
     }
     if (lane == 63) wsum[w] = inc;
     __syncthreads();
-    uint64_t before = 0, all = 0;
+    U before = 0, all = 0;
     for (unsigned k = 0; k < kWaves; ++k) {
-        const uint64_t s = wsum[k];
+        const U s = wsum[k];
         if (k < w) before += s;
         all += s;
     }
-    __syncthreads();
     *total = all;
     return before + inc - x;
 }
 
-// 32 bytes of a share into registers: two 16-byte loads, or byte loads for the last, partial granule of a segment
-// (nothing at or past `avail` is read).
+// 32 bytes of a granule into registers: two 16-byte loads; the last, partial granule of a segment by dwords and its
+// last bytes (nothing at or past `avail` is read).
 __device__ __forceinline__ void load_granule(const uint8_t* p, uint32_t avail, uint32_t (&wd)[8]) {
     if (avail >= kShare) {
         const v4u a = *reinterpret_cast<const v4u_ua*>(p), b = *reinterpret_cast<const v4u_ua*>(p + 16);
         wd[0] = a[0], wd[1] = a[1], wd[2] = a[2], wd[3] = a[3], wd[4] = b[0], wd[5] = b[1], wd[6] = b[2], wd[7] = b[3];
     } else {
-        static_for<8>([&](auto d) { wd[d.value] = 0u; });
-        static_for<32>([&](auto J) {
-            constexpr unsigned j = decltype(J)::value;
-            if (j < avail) wd[j / 4] |= (uint32_t)p[j] << (8 * (j % 4));
+        uint32_t rest = 0;
+        for (uint32_t k = avail & ~3u; k < avail; ++k) rest |= (uint32_t)p[k] << (8 * (k & 3u));
+        static_for<8>([&](auto d) {
+            wd[d.value] = 4 * d.value == (avail & ~3u) ? rest : 0u;
+            if (4 * d.value + 4 <= avail) wd[d.value] = *reinterpret_cast<const u32_ua*>(p + 4 * d.value);
         });
     }
 }
-
-// Per-thread walk state over its share.
-struct Walk {
-    uint32_t lit;   // 1: the next byte is a literal consumed by an escape
-    uint32_t run;   // decoded bytes so far (segment-relative in the second pass)
-    uint32_t rk;    // rank of the next string start (second pass)
-    uint32_t w;     // LDS output word
-    uint32_t ab;    // pending bytes in acc
-    uint64_t acc;   // bytes of word w not yet complete
-};
-
-// The granule passes below run as a loop of 4 rounds over 8 positions each. Between rounds the registers rotate:
-// the round's bytes are always wd[0..1], the byte after them the low byte of wd[2], their start bits (and the next
-// one) the low 9 bits of sb, their packed lengths kp[0]. Per-byte decisions are integer arithmetic (0/1 values), so
-// no lane masks pile up across the unrolled steps.
-__device__ __forceinline__ void rotate(uint32_t (&wd)[8], uint32_t (&kp)[4], uint64_t& sb, uint32_t fill) {
-    static_for<6>([&](auto d) { wd[d.value] = wd[d.value + 2]; });
-    wd[6] = fill, wd[7] = 0u;
-    kp[0] = kp[1], kp[1] = kp[2], kp[2] = kp[3], kp[3] = 0u;
-    sb >>= 8;
-}
-
-// Pass 1 over one granule (32 positions; `sb` holds their start bits and the next one; positions at or past `lim`
-// are outside the share): decoded bytes into st.run and each position's length, in 4 bits, into kp. len[255] is 1
-// (an escape emits one byte) and a literal emits nothing. Each round issues its 8 table loads together.
-__device__ __forceinline__ void count_granule(const uint32_t (&wd_in)[8], uint64_t sb, uint32_t lim,
-                                              const uint8_t* len, Walk& st, uint32_t (&kp)[4]) {
-    uint32_t wd[8], unused[4] = {0u, 0u, 0u, 0u};
-    static_for<8>([&](auto d) { wd[d.value] = wd_in[d.value]; });
-#pragma unroll 1
-    for (uint32_t r = 0; r < 4; ++r) {
-        const int32_t lr = (int32_t)lim - (int32_t)(8 * r);
-        uint32_t      lc[8];
-        static_for<8>([&](auto J) { lc[J.value] = len[(wd[J.value / 4] >> (8 * (J.value % 4))) & 255u]; });
-        uint32_t kw = 0;
-        static_for<8>([&](auto J) {
-            constexpr unsigned j   = decltype(J)::value;
-            const uint32_t     c   = (wd[j / 4] >> (8 * (j % 4))) & 255u;
-            const uint32_t     is  = (c + 1u) >> 8;                      // 1 for an escape byte
-            const uint32_t     s1  = (uint32_t)(sb >> (j + 1)) & 1u;
-            const uint32_t     in  = (uint32_t)((int32_t)j - lr) >> 31;  // j < lr
-            const uint32_t     act = in & (st.lit ^ 1u);                 // a code or an escape inside the share
-            const uint32_t     k   = lc[j] & (0u - act);
-            st.lit                 = act & is & (s1 ^ 1u);
-            st.run += k;
-            kw |= k << (4 * j);
-        });
-        kp[0] = kp[1], kp[1] = kp[2], kp[2] = kp[3], kp[3] = kw;  // after 4 rounds kp[r] holds round r
-        rotate(wd, unused, sb, 0u);
-    }
-}
-
-// Pass 2 over one granule: records the output position of every string start (ostart by rank; a lane-private
-// dummy slot takes the write where none starts) and, with EMIT, ORs the decoded bytes into obuf 8 at a time.
-// Lengths come from pass 1 (HAVE_K: kp) or are recomputed with the literal chain. `nb` is the byte after the
-// granule.
-template <bool EMIT, bool HAVE_K>
-__device__ __forceinline__ void walk_granule(const uint32_t (&wd_in)[8], uint32_t nb, uint64_t sb, uint32_t lim,
-                                             const uint32_t (&kp_in)[4], const uint64_t* sym, const uint8_t* len,
-                                             uint32_t* ostart, uint32_t dummy, uint64_t* obuf, Walk& st) {
-    uint32_t wd[8], kp[4];
-    static_for<8>([&](auto d) { wd[d.value] = wd_in[d.value]; });
-    static_for<4>([&](auto d) { kp[d.value] = kp_in[d.value]; });
-#pragma unroll 1
-    for (uint32_t r = 0; r < 4; ++r) {
-        const int32_t lr = (int32_t)lim - (int32_t)(8 * r);
-        uint64_t      sv[8];
-        uint32_t      lc[8];
-        static_for<8>([&](auto J) {
-            const uint32_t c = (wd[J.value / 4] >> (8 * (J.value % 4))) & 255u;
-            if constexpr (EMIT) sv[J.value] = sym[c];  // sym[255] = 0; symbols are zero beyond their length
-            if constexpr (!HAVE_K) lc[J.value] = len[c];
-        });
-        static_for<8>([&](auto J) {
-            constexpr unsigned j  = decltype(J)::value;
-            const uint32_t     c  = (wd[j / 4] >> (8 * (j % 4))) & 255u;
-            const uint32_t     is = (c + 1u) >> 8;
-            const uint32_t     s1 = (uint32_t)(sb >> (j + 1)) & 1u;
-            const uint32_t     in = (uint32_t)((int32_t)j - lr) >> 31;
-            uint32_t           k;
-            if constexpr (HAVE_K) {
-                k = (kp[0] >> (4 * j)) & 15u;
-            } else {
-                const uint32_t act = in & (st.lit ^ 1u);
-                k                  = lc[j] & (0u - act);
-                st.lit             = act & is & (s1 ^ 1u);
-            }
-            const uint32_t s0 = in & (uint32_t)(sb >> j) & 1u;
-            ostart[dummy + s0 * (st.rk - dummy)] = st.run;
-            st.rk += s0;
-            if constexpr (EMIT) {
-                const uint32_t nxt = j < 7 ? (wd[(j + 1) / 4] >> (8 * ((j + 1) % 4))) & 255u : wd[2] & 255u;
-                // k != 0: a code (its symbol) or an escape (the next byte, or 0 when its string ends first)
-                const uint64_t eb   = (uint64_t)(nxt * (is & (s1 ^ 1u)));
-                const uint32_t kz   = (k + 15u) >> 4;  // 1 when k != 0
-                const uint64_t keep = 0ull - (uint64_t)kz;
-                const uint64_t x    = (sv[j] | eb) & keep;
-                const uint32_t sh   = 8 * st.ab;
-                const uint64_t lo   = st.acc | (x << sh);
-                const uint64_t hi   = (x >> 1) >> (63 - sh);  // the bytes past the word (none when sh = 0)
-                atomicOr(reinterpret_cast<unsigned long long*>(obuf + st.w), (unsigned long long)lo);
-                const uint32_t all  = st.ab + k;
-                const uint64_t full = (uint64_t)(all >> 3);
-                st.w += (uint32_t)full;
-                st.acc = lo ^ ((lo ^ hi) & (0ull - full));
-                st.ab  = all & 7u;
-                __builtin_amdgcn_sched_barrier(0);  // one byte at a time: interleaving steps only adds registers
-            }
-            st.run += k;
-        });
-        rotate(wd, kp, sb, nb);
-        nb = 0u;
-    }
-}
-
-// -- granules of codes only: no 0xFF byte, no literal at the start, all 32 positions inside the share ---------------
 __device__ __forceinline__ bool has_ff(const uint32_t (&wd)[8]) {
     uint32_t z = 0;
     static_for<8>([&](auto d) {
@@ -226,433 +97,510 @@ __device__ __forceinline__ bool has_ff(const uint32_t (&wd)[8]) {
     });
     return z != 0;
 }
-
-__device__ __forceinline__ uint32_t nib_sum(uint32_t v) {  // sum of the 8 nibbles of v (each <= 8)
-    const uint32_t t = (v & 0x0F0F0F0Fu) + ((v >> 4) & 0x0F0F0F0Fu);
-    return (t * 0x01010101u) >> 24;
+template <unsigned J>
+__device__ __forceinline__ uint32_t byte_of(const uint32_t (&wd)[8]) {
+    return (wd[J / 4] >> (8 * (J % 4))) & 255u;
 }
 
-// Pass 1: every byte is a code; its length goes to kp and the total to st.run.
-__device__ __forceinline__ void count_codes(const uint32_t (&wd)[8], const uint8_t* len, Walk& st, uint32_t (&kp)[4]) {
-    static_for<4>([&](auto R) {
-        constexpr unsigned r = decltype(R)::value;
-        uint32_t           lc[8];
-        static_for<8>([&](auto J) { lc[J.value] = len[(wd[2 * r + J.value / 4] >> (8 * (J.value % 4))) & 255u]; });
-        uint32_t kw = 0;
-        static_for<8>([&](auto J) { kw |= lc[J.value] << (4 * J.value); });
-        kp[r] = kw;
-        st.run += nib_sum(kw);
-    });
-}
+// What k_fsst_count leaves for k_fsst per segment: decoded bytes, those of the vector's segments before it (kMalformed:
+// its offsets are not monotone), and the place of its compressed bytes in the vector's.
+struct FsstSeg {
+    uint64_t total, before;
+    uint32_t s0, n;
+};
+constexpr uint64_t kMalformed = 1ull << 63;
 
-// Pass 2, bytes: OR each code's symbol into the LDS image (st.w / st.ab / st.acc as in walk_granule).
-__device__ __forceinline__ void emit_codes(const uint32_t (&wd)[8], const uint32_t (&kp)[4], const uint64_t* sym,
-                                           uint64_t* obuf, Walk& st) {
-    static_for<4>([&](auto R) {
-        constexpr unsigned r = decltype(R)::value;
-        uint64_t           sv[8];
-        static_for<8>([&](auto J) { sv[J.value] = sym[(wd[2 * r + J.value / 4] >> (8 * (J.value % 4))) & 255u]; });
-        static_for<8>([&](auto J) {
-            const uint32_t k  = (kp[r] >> (4 * J.value)) & 15u;
-            const uint64_t x  = sv[J.value];
-            const uint32_t sh = 8 * st.ab;
-            const uint64_t lo = st.acc | (x << sh);
-            const uint64_t hi = (x >> 1) >> (63 - sh);
-            atomicOr(reinterpret_cast<unsigned long long*>(obuf + st.w), (unsigned long long)lo);
-            const uint32_t all = st.ab + k;
-            const bool     full = all >= 8;
-            st.w += full;
-            st.acc = full ? hi : lo;
-            st.ab  = all & 7u;
-            __builtin_amdgcn_sched_barrier(0);
-        });
-    });
-}
+// A segment's compressed bytes `seg`, n of them, and the ends of its strings (LDS, from its start).
+struct Segment {
+    const uint8_t*  seg;
+    uint32_t        n;
+    const uint32_t* end;
+};
 
-// Pass 2, bytes, for any first granule (escapes, literals, positions past the share): lengths from pass 1 (a
-// literal or a position past the share has length 0); a code emits its symbol, an escape the byte after it (0 when
-// its string ends first).
-__device__ __forceinline__ void emit_first(const uint32_t (&wd)[8], uint32_t nb, uint64_t sb, const uint32_t (&kp)[4],
-                                           const uint64_t* sym, uint64_t* obuf, Walk& st) {
-    static_for<4>([&](auto R) {
-        constexpr unsigned r = decltype(R)::value;
-        uint64_t           sv[8];
-        static_for<8>([&](auto J) { sv[J.value] = sym[(wd[2 * r + J.value / 4] >> (8 * (J.value % 4))) & 255u]; });
-        static_for<8>([&](auto J) {
-            constexpr unsigned j   = 8 * r + decltype(J)::value;
-            const uint32_t     c   = (wd[j / 4] >> (8 * (j % 4))) & 255u;
-            const uint32_t     k   = (kp[r] >> (4 * J.value)) & 15u;
-            const uint32_t     s1  = (uint32_t)(sb >> (j + 1)) & 1u;
-            uint32_t           nxt;
-            if constexpr (j + 1 < 32) nxt = (wd[(j + 1) / 4] >> (8 * ((j + 1) % 4))) & 255u;
-            else nxt = nb;
-            const uint64_t eb = (uint64_t)(nxt * (((c + 1u) >> 8) & (s1 ^ 1u)));
-            const uint64_t x  = (sv[J.value] | eb) & (0ull - (uint64_t)((k + 15u) >> 4));
-            const uint32_t sh = 8 * st.ab;
-            const uint64_t lo = st.acc | (x << sh);
-            const uint64_t hi = (x >> 1) >> (63 - sh);
-            atomicOr(reinterpret_cast<unsigned long long*>(obuf + st.w), (unsigned long long)lo);
-            const uint32_t all  = st.ab + k;
-            const bool     full = all >= 8;
-            st.w += full;
-            st.acc = full ? hi : lo;
-            st.ab  = all & 7u;
-            __builtin_amdgcn_sched_barrier(0);
-        });
-    });
+// Place of a segment's first granule in StringPlan::d_sizes: granules of 32 bytes from the column's start, one more per
+// segment before it for the partial ones.
+__device__ __forceinline__ uint64_t sizes_at(uint64_t page_off, const uint8_t* page, const uint8_t* bytes, uint64_t seg) {
+    return (page_off + (uint64_t)(bytes - page)) / kShare + seg;
 }
+constexpr uint32_t kSpecial = 0x8000;  // in d_sizes: the granule holds, or starts with, part of an escape
 
-// Pass 2, positions: the output position of each string start among the granule's 32 positions (bits of sbm) is the
-// granule's first position run0 plus the lengths before it (nibble sums of kp).
-__device__ __forceinline__ void record_starts(uint32_t sbm, const uint32_t (&kp)[4], uint32_t run0, uint32_t* ostart,
-                                              Walk& st) {
-    const uint32_t s1 = nib_sum(kp[0]), s2 = s1 + nib_sum(kp[1]), s3 = s2 + nib_sum(kp[2]);
-    while (sbm) {
-        const uint32_t p = (uint32_t)__builtin_ctz(sbm), q = p >> 3;
-        sbm &= sbm - 1;
-        const uint32_t word   = q == 0 ? kp[0] : q == 1 ? kp[1] : q == 2 ? kp[2] : kp[3];
-        const uint32_t before = q == 0 ? 0u : q == 1 ? s1 : q == 2 ? s2 : s3;
-        ostart[st.rk++]       = run0 + before + nib_sum(word & ((1u << (4 * (p & 7))) - 1));
+// A thread's granule of the chunk at c0: its bytes (0 past the segment), its place in the segment, how many bytes the
+// segment has there.
+struct Granule {
+    uint32_t wd[8];
+    uint32_t q0, lim;
+};
+__device__ __forceinline__ Granule open_granule(const Segment& g, uint32_t c0, unsigned tid) {
+    Granule r;
+    r.q0  = c0 + tid * kShare;
+    r.lim = r.q0 < g.n ? (g.n - r.q0 < kShare ? g.n - r.q0 : kShare) : 0;
+    if (r.lim) {
+        load_granule(g.seg + r.q0, g.n - r.q0, r.wd);
+    } else {
+        static_for<8>([&](auto d) { r.wd[d.value] = 0u; });
     }
-    st.run = run0 + s3 + nib_sum(kp[3]);
+    return r;
 }
 
-// Wave 0 of the block: bytes decoded by all segments before g (decoupled look-back over their status words). Each
-// poll reads a window of 512 predecessors (8 per lane), so the frontier of known prefixes advances 512 segments per
-// memory round trip. Status words are read and written with relaxed agent-scope atomics: a block consumes only the
-// words' own values (no data that other blocks wrote), and acquire/release at agent scope would invalidate or write
-// back the whole L2 of the XCD at every poll.
-__device__ __forceinline__ uint64_t look_back(const SegCtl& sc, uint32_t epoch, uint64_t g, uint32_t* err) {
-    constexpr unsigned M     = 8;
-    const unsigned     lane  = threadIdx.x % 64;
-    uint64_t           excl  = 0;
-    int64_t            j     = (int64_t)g - 1;
-    uint32_t           spins = 0;
-    while (j >= 0) {
-        uint64_t val[M];
-        uint32_t fl[M];
-        static_for<M>([&](auto MM) {
-            constexpr unsigned m   = decltype(MM)::value;
-            const int64_t      idx = j - (int64_t)(lane + 64 * m);
-            fl[m] = (uint32_t)kFlagPrefix, val[m] = 0;  // before the first segment: a prefix of 0
-            if (idx >= 0) {
-                const uint64_t w = __hip_atomic_load(sc.status + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                fl[m]            = (uint32_t)(w >> 48) == epoch ? (uint32_t)((w >> 46) & 3u) : 0u;
-                val[m]           = w & kValMask;
-            }
+// Bit k of m as byte k, 0 or 255.
+__device__ __forceinline__ uint32_t spread4(uint32_t m) { return (((m & 15u) * 0x00204081u) & 0x01010101u) * 255u; }
+// Number of strings of the segment that end at or before p (the ends are sorted).
+__device__ __forceinline__ uint32_t ends_upto(const uint32_t* end, uint32_t p) {
+    uint32_t lo = 0;
+    for (uint32_t step = kSeg / 2; step; step /= 2)
+        if (end[lo + step - 1] <= p) lo += step;
+    return lo + (end[lo] <= p ? 1u : 0u);
+}
+// Escapes of a granule, bit j for its byte j: `esc` the escapes that emit the byte after them (one whose string ends
+// right after it emits 0), `none` the bytes that emit nothing (literals, and bytes past the segment).
+struct Escapes {
+    uint32_t esc, none;
+};
+__device__ __forceinline__ Escapes find_escapes(const Segment& g, const Granule& r) {
+    Escapes  x {0, r.lim >= kShare ? 0u : ~0u << r.lim};
+    uint32_t ff = 0;
+    static_for<32>([&](auto J) { ff |= ((byte_of<decltype(J)::value>(r.wd) + 1u) >> 8) << decltype(J)::value; });
+    ff &= ~x.none;
+    uint64_t lit = 0;  // literals; bit 32: the byte after the granule
+    uint32_t k   = ends_upto(g.end, r.q0);  // the first string that ends past q0
+    if (r.q0 && g.seg[r.q0 - 1] == 255 && !(k && g.end[k - 1] == r.q0)) {
+        // the granule starts on a literal when the run of 255 bytes before it has an odd length inside its string (a
+        // run begins with an escape code: after a code or a literal comes a code)
+        const uint32_t start = k ? g.end[k - 1] : 0u;
+        uint32_t       p     = r.q0 - 1;
+        while (p > start && g.seg[p - 1] == 255) --p;
+        lit = (r.q0 - p) & 1u;
+    }
+    // the escapes and the ends in the granule are both in order: one walk over them
+    uint32_t e = k < kSeg ? g.end[k] : ~0u;
+    while (ff) {
+        const uint32_t j = (uint32_t)__builtin_ctz(ff), p = r.q0 + j + 1;
+        ff &= ff - 1;
+        if ((lit >> j) & 1u) continue;
+        while (e < p) e = ++k < kSeg ? g.end[k] : ~0u;
+        if (e != p) x.esc |= 1u << j, lit |= 2ull << j;
+    }
+    x.none |= (uint32_t)lit;
+    return x;
+}
+
+// Values the compiler cannot carry over from before: it would take the table addresses out of all forms of emit_granule,
+// in registers that it then spills.
+__device__ __forceinline__ void forget(uint32_t (&w)[8]) {
+    asm volatile("" : "+v"(w[0]), "+v"(w[1]), "+v"(w[2]), "+v"(w[3]), "+v"(w[4]), "+v"(w[5]), "+v"(w[6]), "+v"(w[7]));
+}
+
+// Joins a thread's symbols into the 8-byte words of the LDS image. acc holds the bytes of the word not yet complete.
+struct Emit {
+    uint8_t* image;
+    uint64_t acc;
+    uint32_t at;  // bit position in the image
+    // x: `bits` bits, 0 above them. WIDE: bits may be 64
+    template <bool WIDE>
+    __device__ __forceinline__ void add(uint64_t x, uint32_t bits) {
+        const uint64_t lo = acc | (x << (at & 63u));
+        const uint64_t hi = WIDE ? (x >> 8) >> (~(at + 7u) & 63u) : x >> (-at & 63u);  // the bytes past the word
+        const uint32_t to   = at + bits;
+        const bool     full = (at ^ to) >= 64u;
+        if (full) *reinterpret_cast<uint64_t*>(image + ((at >> 3) & ~7u)) = lo;
+        acc = full ? hi : lo;
+        at  = to;
+    }
+};
+// Emits the granule's symbols and packs their lengths into lk. KIND 0 (symbols of at most 3 bytes): a table entry is the
+// symbol and its bits, two codes are one addition. KIND 1 (at most 7): the entry's top byte is the length. KIND 2: the
+// lengths are a table of their own. Bytes that emit nothing have been replaced by 255, whose symbol is empty, and
+// `none` (only then) drops their lengths.
+template <int KIND, bool NONE>
+__device__ __forceinline__ void emit_granule(const uint32_t (&wd_in)[8], uint32_t none, const uint64_t* sym,
+                                             const uint8_t* len, Emit& o, uint32_t (&lk)[8]) {
+    uint32_t wd[8];
+    static_for<8>([&](auto d) { wd[d] = wd_in[d]; });
+    forget(wd);
+    if constexpr (NONE) asm volatile("" : "+v"(none));
+    static_for<8>([&](auto D) {
+        constexpr unsigned d = decltype(D)::value;
+        const uint32_t     drop = NONE ? spread4(none >> (4 * d)) : 0u;
+        uint64_t           x[4];
+        uint32_t           l[4];  // KIND 0: bits
+        static_for<4>([&](auto k) {
+            const uint32_t c = byte_of<4 * d + decltype(k)::value>(wd);
+            x[k]             = sym[c];
+            if constexpr (KIND == 2) l[k] = len[c];
         });
-        // distance of the nearest inclusive prefix; every segment nearer must have published its aggregate
-        unsigned first = 64 * M;
-        bool     wait  = false;
-        static_for<M>([&](auto MM) {
-            constexpr unsigned m  = decltype(MM)::value;
-            const uint64_t     bp = __ballot(fl[m] == kFlagPrefix);
-            const uint64_t     bx = __ballot(fl[m] == 0);
-            if (first == 64 * M && !wait) {
-                const unsigned f    = bp ? (unsigned)__builtin_ctzll(bp) : 64u;
-                const uint64_t need = f >= 63 ? ~0ull : ((2ull << f) - 1);
-                if (bx & need) wait = true;
-                else if (bp) first = 64 * m + f;
-            }
+        static_for<4>([&](auto k) {
+            if constexpr (KIND == 0) l[k] = (uint32_t)(x[k] >> 32), x[k] &= 0xffffffffull;
+            if constexpr (KIND == 1) l[k] = (uint32_t)(x[k] >> 56), x[k] &= 0x00ffffffffffffffull;
+            if constexpr (NONE) l[k] &= ~(drop >> (8 * decltype(k)::value));
         });
-        if (wait) {
-            if (++spins > sc.spin_limit) {
-                if (lane == 0) atomicOr(err, kErrSpin);
-                return excl;
-            }
-            __builtin_amdgcn_s_sleep(1);
-            continue;
+        // (the asm keeps the packing here: sunk to its use it would hold every length in a register of its own)
+        if constexpr (KIND == 0) {
+            lk[d] = (l[0] | (l[1] << 8) | (l[2] << 16) | (l[3] << 24)) >> 3;  // at most 3 each: no bit crosses a byte
+            asm volatile("" : "+v"(lk[d]));
+            o.template add<false>(x[0] | (x[1] << l[0]), l[0] + l[1]);
+            o.template add<false>(x[2] | (x[3] << l[2]), l[2] + l[3]);
+        } else {
+            lk[d] = l[0] | (l[1] << 8) | (l[2] << 16) | (l[3] << 24);
+            asm volatile("" : "+v"(lk[d]));
+            static_for<4>([&](auto k) { o.template add<KIND == 2>(x[k], 8 * l[k]); });
         }
-        uint64_t part = 0;
-        static_for<M>([&](auto MM) {
-            constexpr unsigned m = decltype(MM)::value;
-            if (lane + 64 * m <= first) part += val[m];
-        });
-        for (unsigned d = 32; d >= 1; d >>= 1) part += __shfl_xor(part, d, 64);
-        excl += part;
-        if (first < 64 * M) break;
-        j -= 64 * M;
-    }
-    return excl;
+        if constexpr (d % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+    });
+}
+// Exclusive prefix of the granule's packed lengths into its 32 bytes of `pre` (at most 248: a byte each).
+__device__ __forceinline__ void granule_prefix(const uint32_t (&lk)[8], uint8_t* p) {
+    uint32_t run = 0, ex[8];
+    static_for<8>([&](auto d) {
+        uint32_t t = lk[d] + (lk[d] << 8);
+        t += t << 16;  // inclusive prefix within the dword
+        ex[d] = (t << 8) + __builtin_amdgcn_perm(run, run, 0u);  // run in every byte
+        run += t >> 24;
+    });
+    *reinterpret_cast<v4u*>(p)      = v4u {ex[0], ex[1], ex[2], ex[3]};
+    *reinterpret_cast<v4u*>(p + 16) = v4u {ex[4], ex[5], ex[6], ex[7]};
+}
+// Decoded bytes of the granule (codes and escapes alike; dropped bytes not).
+__device__ __forceinline__ uint32_t granule_size(const uint32_t (&wd)[8], uint32_t none, const uint8_t* len) {
+    uint32_t s = 0;
+    static_for<8>([&](auto d) {
+        uint32_t l[4];
+        static_for<4>([&](auto k) { l[k] = len[byte_of<4 * decltype(d)::value + decltype(k)::value>(wd)]; });
+        if (none)
+            static_for<4>([&](auto k) { l[k] = (none >> (4 * decltype(d)::value + decltype(k)::value)) & 1u ? 0u : l[k]; });
+        s += l[0] + l[1] + l[2] + l[3];
+        if constexpr (decltype(d)::value % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+    });
+    return s;
 }
 
+// Decoded length of one string, byte by byte from global memory.
+__device__ __forceinline__ uint32_t string_length(const uint8_t* cb, uint32_t s, uint32_t e, const uint8_t* len) {
+    uint32_t tot = 0;
+    for (uint32_t q = s; q < e;) {
+        const unsigned c = cb[q];
+        if (c == 255) tot += 1, q += 2;
+        else tot += len[c], q += 1;
+    }
+    return tot;
+}
 // One string decoded from global memory to global memory, byte by byte, into out[w, stop).
-__device__ __forceinline__ void decode_string_global(const uint8_t* cb, uint32_t s, uint32_t e, const uint64_t* sym,
-                                                     const uint8_t* len, uint8_t* out, uint64_t w, uint64_t stop) {
+__device__ __forceinline__ void decode_string_global(const uint8_t* cb, uint32_t s, uint32_t e, const FsstTableDev* table,
+                                                     uint8_t* out, uint64_t w, uint64_t stop) {
     for (uint32_t q = s; q < e && w < stop;) {
         const unsigned c = cb[q];
         if (c == 255) {
             out[w++] = q + 1 < e ? cb[q + 1] : 0;
             q += 2;
         } else {
-            const uint64_t x = sym[c];
-            const unsigned n = len[c];
+            const uint64_t x = table->symbol[c];
+            const unsigned n = table->len[c];
             for (unsigned b = 0; b < n && w < stop; ++b) out[w++] = (uint8_t)(x >> (8 * b));
             q += 1;
         }
     }
 }
 
-// MODE FS_OFFSETS writes the n+1 string end offsets; FS_BYTES writes the bytes at the caller's offsets; FS_ALL
-// writes both. `offsets` is indexed from the column's first string; `first_string` is the page's. The launch bound
-// asks for 6 waves per SIMD (at most 80 VGPRs): three 512-thread blocks per compute unit, which the ~38 KB of LDS
-// per block also allows; without it the compiler takes ~100 VGPRs and two blocks fit.
-template <int MODE>
-__global__ __launch_bounds__(kSeg, 6) void k_fsst(const uint8_t* __restrict__ page, const FsstTableDev* __restrict__ table,
-                                               uint64_t first_string, uint64_t* __restrict__ offsets,
-                                               uint8_t* __restrict__ out, uint64_t cap, uint32_t* err, SegCtl sc) {
-    constexpr bool LOOKBACK = MODE != FS_BYTES;
-    constexpr bool EMIT     = MODE != FS_OFFSETS;
-    __shared__ uint64_t sym[256];
+// One block per vector: its segments' decoded sizes and places (FsstSeg), every string's end within its segment, and every
+// granule's decoded size. Bound by the length reads from LDS and, per block, by the chain offsets -> bytes -> lengths.
+// GROUPS: segments at a time, 256 threads each. 4 (the chain once) while two rounds of such blocks, two per compute unit,
+// hold the page: 2^19 strings of 36 bytes decode in 27 us against 33 with 1; beyond that 1, whose eight small blocks per
+// compute unit overlap their chains: 2^21 strings count in 23 us against 31. (A block per segment, which reads the
+// vector's offsets four times, took 34 us.)
+template <unsigned GROUPS>
+__global__ __launch_bounds__(kSeg* GROUPS, 8) void k_fsst_count(const uint8_t* __restrict__ page, uint64_t page_off,
+                                                                const FsstTableDev* __restrict__ table, uint64_t seg0,
+                                                                FsstSeg* __restrict__ segs, uint64_t* __restrict__ vecs,
+                                                                uint32_t* __restrict__ str_end,
+                                                                uint16_t* __restrict__ sizes) {
     __shared__ uint8_t  len[256];
-    __shared__ uint32_t sbits[kMaxComp / 32 + 2];  // string starts over positions [0, n]
-    __shared__ uint32_t ostart[kSeg + 1 + 64];     // output position by start rank; then one dummy slot per lane
-    __shared__ uint16_t rank0[kSeg];               // start rank at each share's first position
-    __shared__ uint64_t obuf[EMIT ? kOutLds / 8 + 1 : 1];
-    __shared__ uint64_t bcast;
-    const unsigned      tid = threadIdx.x, lane = tid % 64;
-
-    uint64_t local = blockIdx.x;
-    uint32_t epoch = 0;
-    if constexpr (LOOKBACK) {
-        // one thread reads the call's state and takes the ticket; the block shares them through LDS
-        __shared__ uint32_t bepoch;
-        if (tid == 0) {
-            // written by k_begin_call, an earlier kernel of the stream: plain loads see it (and stay in the L2)
-            const uint64_t base = sc.ticket[kCallBase];
-            bepoch = (uint32_t)sc.ticket[kCallBase + 1];
-            bcast  = __hip_atomic_fetch_add(sc.ticket, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) -
-                    (base + sc.ticket_off);
-        }
-        __syncthreads();
-        local = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(bcast >> 32)) << 32) |
-                __builtin_amdgcn_readfirstlane((uint32_t)bcast);  // block-uniform: scalar registers
-        epoch = __builtin_amdgcn_readfirstlane(bepoch);
-        __syncthreads();
-        if (local >= gridDim.x) {  // the host's ticket count disagrees with the counter: stop, report
-            if (tid == 0) atomicOr(err, kErrTicket);
-            return;
-        }
+    __shared__ uint32_t ends[8 * kEndRow], end[1024];  // transposed from the vector's start, then in order from the segment's
+    __shared__ uint64_t wsum[kSegPerV][kWaves];
+    __shared__ uint32_t malformed;
+    const unsigned      t = threadIdx.x, tid = t % kSeg, lane = t % 64, v = blockIdx.x;
+    const unsigned      group = __builtin_amdgcn_readfirstlane(t / kSeg);
+    const uint8_t*      cb  = vbuf(page, 2, v, 0);
+    const uint64_t      seg = seg0 + (uint64_t)v * kSegPerV;
+    if (t < 256) {
+        const v4u q = *reinterpret_cast<const v4u_ua*>(vbuf(page, 2, v, 1) + 16 * t);  // transposed 4 t .. 4 t + 3
+        static_for<4>([&](auto k) { ends[(t >> 5) * kEndRow + ((t >> 2) & 7) * 17 + 4 * (t & 3) + k] = q[k.value]; });
+        len[t] = table->len[t];
     }
-    __shared__ uint32_t ends_l[1024];
-    const unsigned      v = (unsigned)(local / kSegPerV), h = (unsigned)(local % kSegPerV), i = h * kSeg + tid;
-    const uint8_t*      cb   = vbuf(page, 2, v, 0);
-    const uint8_t*      ends = vbuf(page, 2, v, 1);
-    // the table, and the vector's 1024 (transposed) end offsets with one coalesced 16-byte load per thread
-    if (tid < 256) {
-        sym[tid] = table->symbol[tid], len[tid] = table->len[tid];
-        *reinterpret_cast<v4u*>(ends_l + 4 * tid) = *reinterpret_cast<const v4u_ua*>(ends + 16 * tid);
+    if (t == 0) malformed = 0;
+    __syncthreads();
+    auto bound = [&](unsigned h) {  // of the segments
+        return h ? (uint32_t)__builtin_amdgcn_readfirstlane(ends[end_place(h * kSeg - 1)]) : 0u;
+    };
+    auto span = [&](unsigned h) {
+        const uint32_t a = bound(h), b = bound(h + 1);
+        return a <= b && b - a <= kMaxComp;
+    };
+    for (unsigned h = group; h < kSegPerV; h += GROUPS) {
+        const unsigned i = h * kSeg + tid;
+        const uint32_t e = ends[end_place(i)], s = i ? ends[end_place(i - 1)] : 0u, s0 = bound(h);
+        end[i]                          = e - s0;
+        str_end[(seg + h) * kSeg + tid] = e - s0;
+        if (!(span(h) && s0 <= s && s <= e && e <= bound(h + 1))) atomicOr(&malformed, 1u << h);
     }
     __syncthreads();
-    auto end_at = [&](int k) { return k < 0 ? 0u : ends_l[transposed_of((unsigned)k)]; };
-    const uint64_t  g    = sc.seg0 + local;  // column-wide segment
-    uint64_t* const oseg = offsets + first_string + (uint64_t)v * 1024 + h * kSeg;
-    const uint32_t  s0 = __builtin_amdgcn_readfirstlane(end_at((int)(h * kSeg) - 1));
-    const uint32_t  s1 = __builtin_amdgcn_readfirstlane(end_at((int)(h * kSeg + kSeg) - 1));
-    uint32_t        s = end_at((int)i - 1), e = end_at((int)i);
-    // byte-parallel shares: 32-byte granules, C bytes per thread
-    const bool     span_ok = s0 <= s1 && s1 - s0 <= kMaxComp;  // block-uniform
-    const uint32_t n       = span_ok ? s1 - s0 : 0;
-    const uint32_t C       = kShare * ((n + kShare * kSeg - 1) / (kShare * kSeg));
-    const uint32_t q0 = tid * C < n ? tid * C : n, q1 = q0 + C < n ? q0 + C : n;
-    const uint8_t* seg = cb + s0;
-    // the share's first granule, the byte after it and the byte before it, loaded ahead of the barriers below
-    // (every byte lies in [s0, s1], inside the vector's compressed bytes)
-    uint32_t wd0[8], nb0 = 0, prev = 0;
-    if (q0 < q1) {
-        load_granule(seg + q0, n - q0, wd0);
-        nb0  = q0 + kShare < n ? seg[q0 + kShare] : 0u;
-        prev = q0 ? seg[q0 - 1] : 0u;
+    for (unsigned h = group; h < kSegPerV; h += GROUPS) {
+        const uint32_t s0 = bound(h);
+        const Segment  g {cb + s0, span(h) ? bound(h + 1) - s0 : 0u, end + h * kSeg};
+        uint64_t       mine = 0;
+        if (!((malformed >> h) & 1u)) {
+            uint16_t* const at = sizes + sizes_at(page_off, page, g.seg, seg + h);
+            for (uint32_t c0 = 0; c0 < g.n; c0 += kChunk) {
+                const Granule r    = open_granule(g, c0, tid);
+                uint32_t      prev = (uint32_t)__shfl_up((int)r.wd[7], 1, 64) >> 24;  // the byte before the granule
+                if (lane == 0) prev = r.q0 && r.lim ? g.seg[r.q0 - 1] : 0u;
+                const bool special = r.lim && (prev == 255u || has_ff(r.wd));
+                uint32_t   none    = r.lim >= kShare ? 0u : ~0u << r.lim;
+                if (special) none = find_escapes(g, r).none;
+                const uint32_t size = r.lim ? granule_size(r.wd, none, len) : 0u;
+                if (r.lim) at[r.q0 / kShare] = (uint16_t)(size | (special ? kSpecial : 0u));
+                mine += size;
+            }
+        } else {
+            mine = string_length(cb, tid ? end[h * kSeg + tid - 1] + s0 : s0, end[h * kSeg + tid] + s0, len);
+        }
+        for (unsigned d = 32; d >= 1; d >>= 1) mine += __shfl_xor((unsigned long long)mine, d, 64);
+        if (lane == 0) wsum[h][tid / 64] = mine;
     }
-    const bool fast = __syncthreads_and(span_ok && s0 <= s && s <= e && e <= s1) != 0;
+    __syncthreads();
+    if (t == 0) {
+        uint64_t vec = 0;
+        for (unsigned k = 0; k < kSegPerV; ++k) {
+            uint64_t all = 0;
+            for (unsigned w = 0; w < kWaves; ++w) all += wsum[k][w];
+            segs[seg + k] = {all, (malformed >> k) & 1u ? vec | kMalformed : vec, bound(k), span(k) ? bound(k + 1) - bound(k) : 0u};
+            vec += all;
+        }
+        vecs[seg / kSegPerV] = vec;
+    }
+}
 
-    uint64_t seg_total;
-    uint32_t start_rel = 0, end_rel = 0;  // this thread's string, segment-relative output positions
-    uint32_t n_starts = 0;
-    Walk     st {};
-    uint32_t kp0[4] = {0u, 0u, 0u, 0u}, lit1 = 0;  // first granule: lengths, literal after it
-    bool     codes0 = false;                        // first granule holds codes only
-    if (fast) {
-        for (uint32_t k = tid; k <= n / 32 + 1; k += kSeg) sbits[k] = 0u;
+// Exclusive sums of n vectors' decoded sizes, one block.
+__global__ __launch_bounds__(1024) void k_fsst_scan(const uint64_t* __restrict__ vecs, uint64_t* __restrict__ bases,
+                                                    uint32_t n) {
+    __shared__ uint64_t wsum[16];
+    __shared__ uint64_t carry;
+    const unsigned      tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
+    uint64_t            base = 0;
+    constexpr unsigned  K    = 2;  // sizes per thread and round
+    for (uint32_t r = 0; r < n; r += 1024 * K) {
+        uint64_t x[K], s = 0;
+        static_for<K>([&](auto k) {
+            const uint32_t i = r + tid * K + k;
+            x[k]             = i < n ? vecs[i] : 0ull;
+        });
+        static_for<K>([&](auto k) { s += x[k]; });
+        uint64_t inc = s;
+        for (unsigned d = 1; d < 64; d <<= 1) {
+            const uint64_t y = __shfl_up((unsigned long long)inc, d, 64);
+            if (lane >= d) inc += y;
+        }
+        if (lane == 63) wsum[wave] = inc;
         __syncthreads();
-        atomicOr(&sbits[(s - s0) >> 5], 1u << ((s - s0) & 31));
-        if (tid == 0) atomicOr(&sbits[n >> 5], 1u << (n & 31));
+        uint64_t b = base + inc - s;
+        for (unsigned w = 0; w < wave; ++w) b += wsum[w];
+        if (tid == 1023) carry = b + s;
+        static_for<K>([&](auto k) {
+            const uint32_t i = r + tid * K + k;
+            if (i < n) bases[i] = b;
+            b += x[k];
+        });
         __syncthreads();
-        auto is_start = [&](uint32_t p) { return ((sbits[p >> 5] >> (p & 31)) & 1u) != 0; };
-        // a share that starts inside a run of 255 bytes starts on a literal when the run before it is odd (a run
-        // begins with an escape code: after a code or a literal comes a code)
-        uint32_t lit0 = 0;
-        if (q0 < q1 && !is_start(q0) && prev == 255u) {
-            uint32_t p = q0 - 1;
-            while (!is_start(p) && seg[p - 1] == 255) --p;
-            lit0 = (q0 - p) & 1u;
-        }
-        // string starts in the share (bit q1 excluded: it belongs to the next share or is the end bit n)
-        uint32_t ns = 0;
-        for (uint32_t b = q0; b < q1; b += kShare) {
-            const uint32_t m = q1 - b >= 32 ? ~0u : ((1u << (q1 - b)) - 1);
-            ns += __popc(sbits[b >> 5] & m);
-        }
-        // pass 1: decoded bytes of the share
-        st.lit = lit0;
-        if (q0 < q1) {
-            const uint64_t sb  = sbits[q0 >> 5] | ((uint64_t)sbits[(q0 >> 5) + 1] << 32);
-            const uint32_t lim = q1 - q0 < kShare ? q1 - q0 : kShare;
-            codes0             = lim == kShare && st.lit == 0 && !has_ff(wd0);
-            // one form per wave: the codes-only one when every lane of the wave can take it
-            if (__all(codes0)) count_codes(wd0, len, st, kp0);
-            else count_granule(wd0, sb, lim, len, st, kp0);
-            lit1 = st.lit;
-        }
-        for (uint32_t b = q0 + kShare; b < q1; b += kShare) {
-            uint32_t wd[8], kp_unused[4];
-            load_granule(seg + b, n - b, wd);
-            const uint64_t sb  = sbits[b >> 5] | ((uint64_t)sbits[(b >> 5) + 1] << 32);
-            const uint32_t lim = q1 - b < kShare ? q1 - b : kShare;
-            count_granule(wd, sb, lim, len, st, kp_unused);
-        }
-        uint64_t       all;
-        const uint64_t before = block_exclusive_scan((uint64_t)st.run | ((uint64_t)ns << 32), &all);
-        seg_total              = (uint32_t)all;
-        n_starts               = (uint32_t)(all >> 32);
-        rank0[tid]             = (uint16_t)(before >> 32);
-        if (tid == 0) ostart[n_starts] = (uint32_t)seg_total;
-        st = Walk {lit0, (uint32_t)before, (uint32_t)(before >> 32), (uint32_t)before >> 3, (uint32_t)before & 7u, 0ull};
-    } else {
-        // per-string lengths from global memory (offsets clamped so that every read stays inside the vector)
-        if (s > e) s = e;
-        uint32_t tot = 0;
-        for (uint32_t q = s; q < e;) {
-            const unsigned c = cb[q];
-            if (c == 255) tot += 1, q += 2;
-            else tot += len[c], q += 1;
-        }
-        uint64_t       all;
-        const uint64_t before = block_exclusive_scan(tot, &all);
-        seg_total             = all;
-        start_rel             = (uint32_t)before;
-        end_rel               = (uint32_t)before + tot;
+        base = carry;
     }
+}
 
-    // publish this segment's aggregate early, so that later segments can sum past it while it decodes
-    if constexpr (LOOKBACK) {
-        if (tid == 0)
-            __hip_atomic_store(sc.status + g, status_word(epoch, g == 0 ? kFlagPrefix : kFlagAgg, seg_total),
-                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    uint64_t seg_base = 0;
-    bool     given_ok = true;
-    if constexpr (!LOOKBACK) {
+// MODE FS_OFFSETS writes the n+1 string end offsets; FS_BYTES writes the bytes at the caller's offsets; FS_ALL writes
+// both. `offsets` is indexed from the column's first string; `first_string` is the page's. segs: the column's
+// segments; vecs / bases: its vectors' decoded sizes and the sums before each (nullptr: at most kDirect vectors, summed
+// here); seg0: the page's first segment.
+// About 24 KB of LDS and at most 80 VGPRs: six blocks of four waves per compute unit.
+template <int MODE>
+__global__ __launch_bounds__(kSeg, 6) void k_fsst(const uint8_t* __restrict__ page, uint64_t page_off,
+                                               const FsstTableDev* __restrict__ table, uint64_t first_string,
+                                               uint64_t* __restrict__ offsets, uint8_t* __restrict__ out, uint64_t cap,
+                                               uint32_t* err, const FsstSeg* __restrict__ segs,
+                                               const uint64_t* __restrict__ vecs, const uint64_t* __restrict__ bases, const uint32_t* __restrict__ str_end,
+                                               const uint16_t* __restrict__ sizes, uint64_t seg0) {
+    constexpr bool EMIT = MODE != FS_OFFSETS;
+    __shared__ uint64_t sym[256];  // FsstTableDev::packed
+    __shared__ uint8_t  len[256];
+    __shared__ __attribute__((aligned(16))) uint8_t pre[kChunk];  // per compressed byte of the chunk: decoded bytes
+                                                                  // before it in its granule
+    __shared__ uint32_t end[kSeg];                                // of each string, from the segment's start
+    __shared__ uint32_t sbase[kSeg];                              // decoded bytes of the chunk before each granule
+    __shared__ uint32_t wsum[kWaves];
+    __shared__ uint64_t wsum64[kWaves];
+    __shared__ uint32_t window;
+    __shared__ __attribute__((aligned(16))) uint8_t image[kOutLds + 32];
+    const unsigned  tid = threadIdx.x;
+    const uint64_t  seg = seg0 + blockIdx.x;
+    const FsstSeg   st  = segs[seg];
+    const uint32_t  kind = table->kind;
+    const uint8_t*  cb   = vbuf(page, 2, blockIdx.x / kSegPerV, 0);
+    const Segment   g {cb + st.s0, st.n, end};
+    const uint16_t* size_at = sizes + sizes_at(page_off, page, g.seg, seg);
+    Granule         r  = open_granule(g, 0, tid);
+    uint32_t        sz = r.lim ? size_at[r.q0 / kShare] : 0u;
+    const uint64_t  vec = seg / kSegPerV, seg_total = st.total;
+    uint64_t* const oseg     = offsets + first_string + (uint64_t)blockIdx.x * kSeg;
+    uint64_t        seg_base = 0, before = 0;
+    bool            given_ok = true;
+    if constexpr (MODE == FS_BYTES) {
         seg_base = oseg[0];
         given_ok = oseg[kSeg] >= seg_base && oseg[kSeg] - seg_base == seg_total;
+    } else {
+        seg_base = st.before & ~kMalformed;
+        if (bases) seg_base += bases[vec];
+        else
+            for (uint64_t k = tid; k < vec; k += kSeg) before += vecs[k];
     }
-    const bool in_lds = EMIT && fast && given_ok && seg_total <= kOutLds;
-    if (in_lds) {  // the LDS image starts zeroed: pass 2 ORs bytes into it
-        for (uint32_t k = tid; k <= (uint32_t)seg_total / 8; k += kSeg) obuf[k] = 0ull;
+    sym[tid] = table->packed[tid], len[tid] = table->len[tid];
+    end[tid] = str_end[seg * kSeg + tid];  // read back where it is needed: one register less through the emission
+    if (MODE != FS_BYTES && !bases) {
+        for (unsigned d = 32; d >= 1; d >>= 1) before += __shfl_xor((unsigned long long)before, d, 64);
+        if (tid % 64 == 0) wsum64[tid / 64] = before;
         __syncthreads();
+        for (unsigned w = 0; w < kWaves; ++w) seg_base += wsum64[w];
+        seg_base = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(seg_base >> 32)) << 32) |
+                   (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)seg_base);
     }
-
-    if (fast) {
-        // pass 2: string-start positions (and, in LDS, the decoded bytes)
-        const uint32_t dummy = kSeg + 1 + lane;
-        if (q0 < q1) {  // the first granule from registers, with its lengths from pass 1
-            const uint64_t sb  = sbits[q0 >> 5] | ((uint64_t)sbits[(q0 >> 5) + 1] << 32);
-            const uint32_t lim = q1 - q0 < kShare ? q1 - q0 : kShare;
-            const uint32_t run0 = st.run;
-            if (in_lds) {
-                if (__all(codes0)) emit_codes(wd0, kp0, sym, obuf, st);
-                else emit_first(wd0, nb0, sb, kp0, sym, obuf, st);
+    if (MODE != FS_BYTES && seg == 0 && tid == 0) oseg[0] = 0;
+    const bool fits = seg_base <= cap && seg_total <= cap - seg_base;
+    if (!(st.before & kMalformed) && given_ok) {
+        const bool emit = EMIT && fits;
+        if (EMIT && !fits && tid == 0) atomicOr(err, kErrCap);
+        uint32_t done = 0;     // decoded bytes of the chunks before
+        uint32_t end_rel = 0;  // this string's end
+        for (uint32_t c0 = 0; c0 < g.n; c0 += kChunk) {
+            if (c0) r = open_granule(g, c0, tid), sz = r.lim ? size_at[r.q0 / kShare] : 0u;
+            const uint32_t size = sz & ~kSpecial;
+            uint32_t       total;
+            const uint32_t at = block_exclusive_scan(size, wsum, &total);
+            total             = __builtin_amdgcn_readfirstlane(total);  // the same in every lane: scalar from here on
+            if constexpr (MODE != FS_BYTES) sbase[tid] = at;
+            Escapes es {0, 0};
+            if (sz & kSpecial) es = find_escapes(g, r);
+            else if (r.lim < kShare) es.none = ~0u << r.lim;
+            const bool drops = es.none != 0;
+            if (drops) static_for<8>([&](auto d) { r.wd[d] |= spread4(es.none >> (4 * decltype(d)::value)); });
+            // the image starts at the output's place within 16 bytes; windows of it while the chunk has more (offsets
+            // alone: the words are dropped)
+            uint8_t* const dst = out + seg_base + done;
+            const uint32_t sh  = EMIT ? (uint32_t)((uintptr_t)dst & 15u) : 0u;
+            bool           ends_done = MODE == FS_BYTES;
+            for (uint32_t w0 = 0; w0 < total || !ends_done;) {  // bytes [w0, w1) of the chunk, whole granules
+                uint32_t w1 = total;
+                if (total - w0 > kOutLds) {  // uniform
+                    if (tid == 0) window = total;
+                    __syncthreads();
+                    if (at >= w0 && at + size - w0 > kOutLds) atomicMin(&window, at);
+                    __syncthreads();
+                    w1 = __builtin_amdgcn_readfirstlane(window);
+                }
+                const bool mine = at >= w0 && at + size <= w1 && r.lim;
+                // the last word may have no byte that completes it
+                if (tid == 0) *reinterpret_cast<uint64_t*>(image + ((sh + w1 - w0) & ~7u)) = 0ull;
+                Emit o {image, 0ull, 8 * (sh + at - w0)};
+                if (mine) {
+                    uint32_t lk[8];
+                    if constexpr (!EMIT) {  // lengths alone
+                        if (__any(drops)) emit_granule<2, true>(r.wd, es.none, sym, len, o, lk);
+                        else emit_granule<2, false>(r.wd, 0u, sym, len, o, lk);
+                    } else if (__any(drops)) {
+                        if (kind == 0) emit_granule<0, true>(r.wd, es.none, sym, len, o, lk);
+                        else if (kind == 1) emit_granule<1, true>(r.wd, es.none, sym, len, o, lk);
+                        else emit_granule<2, true>(r.wd, es.none, sym, len, o, lk);
+                    } else {
+                        if (kind == 0) emit_granule<0, false>(r.wd, 0u, sym, len, o, lk);
+                        else if (kind == 1) emit_granule<1, false>(r.wd, 0u, sym, len, o, lk);
+                        else emit_granule<2, false>(r.wd, 0u, sym, len, o, lk);
+                    }
+                    granule_prefix(lk, pre + kShare * tid);
+                }
+                __syncthreads();
+                if (mine && EMIT) {
+                    if (o.at & 63u)
+                        atomicOr(reinterpret_cast<unsigned long long*>(image + ((o.at >> 3) & ~7u)), (unsigned long long)o.acc);
+                    for (uint32_t m = es.esc; m; m &= m - 1) {  // the escapes' bytes, 0 so far
+                        const uint32_t j = (uint32_t)__builtin_ctz(m), b = sh + at - w0 + pre[kShare * tid + j];
+                        atomicOr(reinterpret_cast<uint32_t*>(image + (b & ~3u)),
+                                 (uint32_t)g.seg[r.q0 + j + 1] << (8 * (b & 3u)));
+                    }
+                }
+                if (!ends_done && w1 == total) {  // every granule's prefix is there
+                    const uint32_t e = end[tid];
+                    if (e >= c0 && e - c0 < kChunk && e < g.n) end_rel = done + sbase[(e - c0) / kShare] + pre[e - c0];
+                    ends_done = true;
+                }
+                __syncthreads();
+                if (emit) {
+                    // copy-out: whole 16-byte words of the output, then the bytes before the first and after the last
+                    uint8_t*       base0 = dst - sh + w0;  // image byte 0
+                    const uint32_t lo = sh, hi = sh + w1 - w0, lo16 = (lo + 15) & ~15u, hi16 = hi & ~15u;
+                    for (uint32_t k = lo16 + 16 * tid; k < hi16; k += 16 * kSeg)
+                        *reinterpret_cast<v4u_ua*>(base0 + k) = *reinterpret_cast<const v4u*>(image + k);
+                    const uint32_t head = lo16 < hi ? lo16 : hi, tail = hi16 > head ? hi16 : head;
+                    if (lo + tid < head) base0[lo + tid] = image[lo + tid];
+                    if (tail + tid < hi) base0[tail + tid] = image[tail + tid];
+                }
+                w0 = w1;
+                if (w0 >= total) break;
+                __syncthreads();  // the image is free again
             }
-            record_starts((uint32_t)sb & (lim == kShare ? ~0u : (1u << lim) - 1), kp0, run0, ostart, st);
-            st.lit = lit1;  // the literal chain continues into the next granule
+            done += total;
+            if (g.n - c0 > kChunk) __syncthreads();  // pre, sbase and the scan's sums are free again
         }
-        for (uint32_t b = q0 + kShare; b < q1; b += kShare) {
-            const uint64_t sb  = sbits[b >> 5] | ((uint64_t)sbits[(b >> 5) + 1] << 32);
-            const uint32_t lim = q1 - b < kShare ? q1 - b : kShare;
-            uint32_t       wd[8];
-            load_granule(seg + b, n - b, wd);
-            const uint32_t nb = b + kShare < n ? seg[b + kShare] : 0u;
-            if (in_lds) walk_granule<true, false>(wd, nb, sb, lim, kp0, sym, len, ostart, dummy, obuf, st);
-            else walk_granule<false, false>(wd, nb, sb, lim, kp0, sym, len, ostart, dummy, obuf, st);
-        }
-        if (in_lds && q0 < q1)
-            atomicOr(reinterpret_cast<unsigned long long*>(obuf + st.w), (unsigned long long)st.acc);
+        if (end[tid] == g.n) end_rel = done;
+        if constexpr (MODE != FS_BYTES) oseg[tid + 1] = seg_base + end_rel;
+    } else {
+        // per string: malformed offsets (clamped, so that every read stays inside the vector), or the caller's offsets
+        // do not fit the segment
         __syncthreads();
-        // this thread's string: output positions of its start and end from their start ranks
-        auto rank_of = [&](uint32_t p) -> uint32_t {
-            if (p >= n) return n_starts;
-            const uint32_t T = C == kShare ? p / kShare : p / C;  // one granule per share: a shift
-            uint32_t       r = rank0[T];
-            for (uint32_t w = T * C / 32; w < p / 32; ++w) r += __popc(sbits[w]);
-            return r + __popc(sbits[p >> 5] & ((1u << (p & 31)) - 1));
-        };
-        start_rel = ostart[rank_of(s - s0)];
-        end_rel   = ostart[rank_of(e - s0)];
-    }
-
-    // the segment's output base: wave 0 looks back after pass 2 (an earlier look-back finds more predecessors that
-    // have not published yet and polls longer) and publishes the inclusive prefix
-    if constexpr (LOOKBACK) {
-        if (tid < 64) {
-            const uint64_t excl = g == 0 ? 0ull : look_back(sc, epoch, g, err);
-            if (tid == 0) {
-                if (g != 0)
-                    __hip_atomic_store(sc.status + g, status_word(epoch, kFlagPrefix, excl + seg_total),
-                                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                bcast = excl;
-            }
-        }
-        __syncthreads();
-        seg_base = bcast;
-        oseg[tid + 1] = seg_base + end_rel;
-        if (g == 0 && tid == 0) oseg[0] = 0;
-    }
-
-    if constexpr (EMIT) {
-        if (in_lds) {
-            if (seg_base + seg_total > cap) {
-                if (tid == 0) atomicOr(err, kErrCap);
-                return;
-            }
-            // copy-out: 16 bytes per thread per step (unaligned global stores), then the tail byte by byte
-            const uint32_t nb = (uint32_t)seg_total, n16 = nb & ~15u;
-            const uint8_t* src = reinterpret_cast<const uint8_t*>(obuf);
-            uint8_t*       dst = out + seg_base;
-            for (uint32_t k = 16 * tid; k < n16; k += 16 * kSeg)
-                *reinterpret_cast<v4u_ua*>(dst + k) = *reinterpret_cast<const v4u*>(src + k);
-            for (uint32_t k = n16 + tid; k < nb; k += kSeg) dst[k] = src[k];
+        const uint32_t stop_c = end[tid] + st.s0, s_in = tid ? end[tid - 1] + st.s0 : st.s0, s = s_in < stop_c ? s_in : stop_c;
+        uint64_t       w0, stop;
+        if (MODE != FS_BYTES || given_ok) {
+            const uint64_t tot = string_length(cb, s, stop_c, len);
+            uint64_t       all;
+            w0   = seg_base + block_exclusive_scan(tot, wsum64, &all);
+            stop = w0 + tot;
+            if constexpr (MODE != FS_BYTES) oseg[tid + 1] = stop;
         } else {
-            uint64_t w0, stop;
-            if (LOOKBACK || given_ok) w0 = seg_base + start_rel, stop = seg_base + end_rel;
-            else w0 = oseg[tid], stop = oseg[tid + 1];  // the caller's offsets, string by string
-            if (s > e) s = e;
+            w0 = oseg[tid], stop = oseg[tid + 1];  // the caller's offsets, string by string
+        }
+        if constexpr (EMIT) {
             if (stop > cap || stop < w0) atomicOr(err, kErrCap);
-            else decode_string_global(cb, s, e, sym, len, out, w0, stop);
+            else decode_string_global(cb, s, stop_c, table, out, w0, stop);
         }
     }
 }
 
 __global__ void k_zero_first(uint64_t* offsets) { offsets[0] = 0; }
 
-// Start of a look-back call: the ticket counter's current value becomes the call's base, and the epoch advances.
-__global__ void k_begin_call(uint64_t* ticket) {
-    ticket[kCallBase]     = __hip_atomic_load(ticket, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    ticket[kCallBase + 1] = ticket[kCallBase + 1] % 0xffffu + 1;
-}
-
 template <int MODE>
 int launch_pages(const Column& col, StringPlan& sp, const uint8_t* dev_enc, uint64_t* dev_offsets, uint8_t* dev_bytes,
                  uint64_t cap, hipStream_t s) {
-    if (MODE != FS_BYTES) hipLaunchKernelGGL(k_begin_call, dim3(1), dim3(1), 0, s, sp.d_ticket);
-    uint64_t ticket_off = 0;
+    auto* const     segs  = static_cast<FsstSeg*>(sp.d_segs);
+    uint64_t* const vecs  = sp.d_vecs;
+    uint64_t* const bases = sp.n_vec > kDirect ? vecs + sp.n_vec : nullptr;
     for (size_t i = 0; i < col.pages.size(); ++i) {
         const PageEntry& pe = col.pages[i];
         if (!pe.vec_c) continue;
-        const unsigned grid = pe.vec_c * kSegPerV;
-        SegCtl         sc {sp.d_status, sp.d_ticket, ticket_off, (pe.out_index / 1024) * kSegPerV, 1u << 20};
-        hipLaunchKernelGGL(k_fsst<MODE>, dim3(grid), dim3(kSeg), 0, s, dev_enc + pe.page_off, sp.d_tables + i,
-                           pe.out_index, dev_offsets, dev_bytes, cap, sp.d_err, sc);
-        ticket_off += grid;
+        const bool wide = pe.vec_c <= kWideCount;
+        hipLaunchKernelGGL(wide ? k_fsst_count<4> : k_fsst_count<1>, dim3(pe.vec_c), dim3(wide ? 4 * kSeg : kSeg), 0, s,
+                           dev_enc + pe.page_off, pe.page_off, sp.d_tables + i, pe.out_index / kSeg, segs, vecs, sp.d_ends,
+                           sp.d_sizes);
+    }
+    if (bases && MODE != FS_BYTES) hipLaunchKernelGGL(k_fsst_scan, dim3(1), dim3(1024), 0, s, vecs, bases, (uint32_t)sp.n_vec);
+    for (size_t i = 0; i < col.pages.size(); ++i) {
+        const PageEntry& pe = col.pages[i];
+        if (!pe.vec_c) continue;
+        hipLaunchKernelGGL(k_fsst<MODE>, dim3(pe.vec_c * kSegPerV), dim3(kSeg), 0, s, dev_enc + pe.page_off, pe.page_off,
+                           sp.d_tables + i, pe.out_index, dev_offsets, dev_bytes, cap, sp.d_err, segs, vecs, bases,
+                           sp.d_ends, sp.d_sizes, pe.out_index / kSeg);
     }
     if (MODE != FS_BYTES && col.n_values == 0) {
         // offsets[0] of an empty column, by a kernel: a memset node recorded into a caller's captured graph is not
@@ -670,14 +618,22 @@ int strings_prepare(const Column& col, const uint8_t* host, StringPlan& sp) {
     std::vector<FsstTableDev> tabs(col.pages.size());
     for (size_t i = 0; i < col.pages.size(); ++i) {
         std::memset(&tabs[i], 0, sizeof(FsstTableDev));
+        unsigned max_len = 0;
         for (int c = 0; c < 255; ++c) {
             // bytes beyond a symbol's length must be zero: the decoder ORs whole symbols into its output words
             const unsigned l = col.pages[i].fsst.len[c];
             uint64_t       x = col.pages[i].fsst.symbol[c];
             if (l < 8) x &= (1ull << (8 * l)) - 1;
             tabs[i].symbol[c] = x, tabs[i].len[c] = (uint8_t)l;
+            max_len = std::max(max_len, l);
         }
-        tabs[i].len[255] = 1;
+        FsstTableDev& t = tabs[i];
+        t.len[255]      = 1;  // an escape emits one byte
+        t.kind          = max_len <= 3 ? 0 : max_len <= 7 ? 1 : 2;
+        for (int c = 0; c < 256; ++c)
+            t.packed[c] = t.kind == 0   ? t.symbol[c] | (uint64_t)(8 * t.len[c]) << 32
+                          : t.kind == 1 ? t.symbol[c] | (uint64_t)t.len[c] << 56
+                                        : t.symbol[c];
     }
     sp.n_vec           = col.n_values / 1024;
     const uint64_t nsg = sp.n_vec * kSegPerV;
@@ -685,10 +641,10 @@ int strings_prepare(const Column& col, const uint8_t* host, StringPlan& sp) {
     if ((e = hipMalloc(&sp.d_tables, tabs.size() * sizeof(FsstTableDev) + 1)) != hipSuccess) return hip_fail(e, "hipMalloc");
     if ((e = hipMemcpy(sp.d_tables, tabs.data(), tabs.size() * sizeof(FsstTableDev), hipMemcpyHostToDevice)) != hipSuccess)
         return hip_fail(e, "hipMemcpy");
-    if ((e = hipMalloc(&sp.d_status, (nsg + 1) * sizeof(uint64_t))) != hipSuccess) return hip_fail(e, "hipMalloc");
-    if ((e = hipMemset(sp.d_status, 0, (nsg + 1) * sizeof(uint64_t))) != hipSuccess) return hip_fail(e, "hipMemset");
-    if ((e = hipMalloc(&sp.d_ticket, (kCallBase + 2) * sizeof(uint64_t))) != hipSuccess) return hip_fail(e, "hipMalloc");
-    if ((e = hipMemset(sp.d_ticket, 0, (kCallBase + 2) * sizeof(uint64_t))) != hipSuccess) return hip_fail(e, "hipMemset");
+    if ((e = hipMalloc(&sp.d_segs, nsg * sizeof(FsstSeg) + 1)) != hipSuccess) return hip_fail(e, "hipMalloc");
+    if ((e = hipMalloc(&sp.d_vecs, 2 * sp.n_vec * sizeof(uint64_t) + 1)) != hipSuccess) return hip_fail(e, "hipMalloc");
+    if ((e = hipMalloc(&sp.d_ends, nsg * kSeg * sizeof(uint32_t) + 1)) != hipSuccess) return hip_fail(e, "hipMalloc");
+    if ((e = hipMalloc(&sp.d_sizes, (col.size / kShare + nsg + 1) * sizeof(uint16_t))) != hipSuccess) return hip_fail(e, "hipMalloc");
     if ((e = hipMalloc(&sp.d_err, 4)) != hipSuccess) return hip_fail(e, "hipMalloc");
     if ((e = hipMemset(sp.d_err, 0, 4)) != hipSuccess) return hip_fail(e, "hipMemset");
     return FLS_OK;
@@ -696,8 +652,10 @@ int strings_prepare(const Column& col, const uint8_t* host, StringPlan& sp) {
 
 void strings_release(StringPlan& sp) {
     if (sp.d_tables) (void)hipFree(sp.d_tables);
-    if (sp.d_status) (void)hipFree(sp.d_status);
-    if (sp.d_ticket) (void)hipFree(sp.d_ticket);
+    if (sp.d_segs) (void)hipFree(sp.d_segs);
+    if (sp.d_ends) (void)hipFree(sp.d_ends);
+    if (sp.d_vecs) (void)hipFree(sp.d_vecs);
+    if (sp.d_sizes) (void)hipFree(sp.d_sizes);
     if (sp.d_err) (void)hipFree(sp.d_err);
     sp = StringPlan {};
 }
@@ -721,7 +679,6 @@ int strings_check(StringPlan& sp, hipStream_t s) {
     hipError_t e = hipMemcpyAsync(&h, sp.d_err, 4, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return hip_fail(e, "check");
-    if (h & (kErrSpin | kErrTicket)) return fail(FLS_E_DATA, "string offsets: segment look-back did not complete");
     return h ? fail(FLS_E_DATA, "string offsets exceed the output capacity") : FLS_OK;
 }
 

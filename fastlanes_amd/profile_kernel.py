@@ -25,7 +25,7 @@ def main():
     ap.add_argument("--fsst-log2-strings", type=int, default=0,
                     help="instead: decode an FSST string column of 2^k vocabulary strings (offsets + bytes)")
     ap.add_argument("--fsst-two-step", action="store_true",
-                    help="with --fsst-log2-strings: offsets, then bytes (two launches per page) instead of one pass")
+                    help="with --fsst-log2-strings: offsets, then bytes, instead of one call")
     ap.add_argument("--dict-rle", action="store_true",
                     help="instead: decode a DICT_RLE column (pool id 27) of 2^log2n values of --width bits, runs of "
                          "mean length 16 over 4096 keys")

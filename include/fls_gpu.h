@@ -59,11 +59,10 @@ int fls_gpu_plan_string_offsets(fls_gpu_plan* plan, const uint8_t* dev_encoded, 
                                 void* stream);
 int fls_gpu_plan_decode_strings(fls_gpu_plan* plan, const uint8_t* dev_encoded, const uint64_t* dev_offsets,
                                 uint8_t* dev_bytes, uint64_t bytes_capacity, void* stream);
-/* Steps 1 and 2 in one pass over the compressed bytes: writes the n+1 offsets and the bytes (bytes_capacity bounds
- * the bytes; a column that needs more reports FLS_E_DATA at fls_gpu_plan_check). No reference counterpart: the
- * reference decodes string by string on the CPU. Calls on one plan must not overlap (they share its segment status
- * words). Kernel launches only: the call may be captured into a HIP graph; each replay takes its ticket base and
- * epoch on the device. */
+/* Steps 1 and 2 in one call: writes the n+1 offsets and the bytes (bytes_capacity bounds the bytes; a column that needs
+ * more reports FLS_E_DATA at fls_gpu_plan_check). No reference counterpart: the reference decodes string by string on the
+ * CPU. Kernel launches only: the call, like steps 1 and 2, may be captured into a HIP graph. Every call on a plan counts
+ * decoded sizes into the plan's arrays first, which hold the same values after each. */
 int fls_gpu_plan_decode_strings_fused(fls_gpu_plan* plan, const uint8_t* dev_encoded, uint64_t* dev_offsets,
                                       uint8_t* dev_bytes, uint64_t bytes_capacity, void* stream);
 

@@ -165,3 +165,59 @@ def test_fused_decode_in_a_graph(torch_cuda, oracle):
         plan.decode_strings_fused(d_in.data_ptr(), e_off.data_ptr(), e_bytes.data_ptr(), data.size)
         plan.check()
         np.testing.assert_array_equal(e_bytes.cpu().numpy()[: data.size], data)
+
+
+@pytest.mark.parametrize("length", ["short", "long"])
+@pytest.mark.parametrize("symbols", ["pairs", "quads", "words"])
+def test_fused_symbol_tables(torch_cuda, symbols, length):
+    """Tables whose longest symbol has at most 3, at most 7 and 8 bytes (each has its own emission), with escapes in
+    three strings of a hundred (runs of rare bytes, 0xFF among them, so that they fall on 32-byte and 8 KiB edges and across
+    them), for strings short enough that a segment is one chunk and long enough that it is several, whose output takes
+    several windows of the LDS image. Both call forms."""
+    torch = torch_cuda
+    g = np.random.default_rng(len(symbols) * 10 + len(length))
+    words = wl.vocabulary(40, seed=3)
+    rows = []
+    for i in range(3 * 1024):
+        n = int(g.integers(0, 21)) if length == "short" else int(g.integers(60, 500))
+        if symbols == "pairs":
+            b = bytearray(g.integers(97, 123, n, dtype=np.uint8).tobytes())
+        elif symbols == "quads":
+            b = bytearray(g.integers(97, 103, n, dtype=np.uint8).tobytes())
+        else:
+            b = bytearray(b" ".join(words[int(k)] for k in g.integers(0, 40, n // 6 + 1))[:n])
+        if i % 100 < 3:
+            p = int(g.integers(0, len(b) + 1))
+            b[p:p] = (g.integers(160, 256, int(g.integers(1, 30)), dtype=np.uint8) | np.uint8(g.random() < 0.5)).tobytes()
+        rows.append(bytes(b))
+    offs, data = _strs_from(rows)
+    enc = fa.encode_strings(offs.astype(np.uint32), data)
+    longest = int(np.nonzero(enc[17:25])[0][-1]) + 1  # lenHisto of the serialized table: symbols of 1 .. 8 bytes
+    print(f"fsst symbols={symbols} length={length} longest={longest}", flush=True)
+    assert {"pairs": longest <= 3, "quads": 4 <= longest <= 7, "words": longest == 8}[symbols], longest
+    plan, d_in = fa.Plan(enc, "str"), dev(torch, enc)
+    got_off, got = _fused(torch, plan, d_in, offs.size - 1, data.size)
+    np.testing.assert_array_equal(got_off, offs)
+    np.testing.assert_array_equal(got[: data.size], data)
+    d_off = torch.zeros(offs.size, dtype=torch.int64, device="cuda")
+    plan.string_offsets(d_in.data_ptr(), d_off.data_ptr())
+    np.testing.assert_array_equal(d_off.cpu().numpy(), offs)
+    d_bytes = empty(torch, data.size + 3)
+    plan.decode_strings(d_in.data_ptr(), d_off.data_ptr(), d_bytes.data_ptr() + 3, data.size)  # unaligned output
+    plan.check()
+    np.testing.assert_array_equal(d_bytes.cpu().numpy()[3: 3 + data.size], data)
+
+
+@pytest.mark.parametrize("vectors", [1, 1024, 1025])
+def test_fused_segment_bases(torch_cuda, vectors):
+    """Columns whose blocks sum the vectors' sizes themselves (up to 1024) and one that the scan kernel serves."""
+    torch = torch_cuda
+    print(f"fsst bases vectors={vectors}", flush=True)
+    g = np.random.default_rng(vectors)
+    lens = g.integers(0, 9, vectors * 1024)
+    offs = np.concatenate([[0], np.cumsum(lens)])
+    data = g.integers(97, 107, int(offs[-1]), dtype=np.uint8)
+    enc = fa.encode_strings(offs.astype(np.uint32), data)
+    got_off, got = _fused(torch, fa.Plan(enc, "str"), dev(torch, enc), offs.size - 1, data.size)
+    np.testing.assert_array_equal(got_off, offs)
+    np.testing.assert_array_equal(got[: data.size], data)
