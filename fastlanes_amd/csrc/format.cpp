@@ -268,6 +268,7 @@ std::string parse_page(const Reader& r, uint64_t off, uint8_t dtype, PageEntry& 
             if (ok) {
                 const unsigned bw = bwc(v, q);
                 ok = bw <= CW && need(v, q + 2, 128ull * bw);
+                if (bw > pe.bw_max) pe.bw_max = (uint8_t)bw;
             }
             if (ok && patch) {  // [exception values][positions | bitmap | count + first position]
                 const uint8_t* b1  = pg + boff[o + 1] + ep(v, o + 1);

@@ -127,6 +127,7 @@ struct PageEntry {
     // RLE / DICT_RLE with DELTA positions: the largest position bit width over the page's vectors (0 or 1 for
     // every page the encoders write)
     uint8_t pos_bw_max = 0;
+    uint8_t bw_max     = 0;  // FFOR-shaped pages: the largest bit width over the page's vectors
     // FSST (string columns)
     FsstTableH fsst;
 };

@@ -141,7 +141,7 @@ hipError_t page_launch(fls_gpu_plan* plan, size_t i, const uint8_t* dev_encoded,
     DevDict&         d    = plan->dicts[i];
     PageMeta         pm {};
     for (unsigned b = 0; b < pe.arr_c && b < 6; ++b) pm.off[b] = pe.boff[b];
-    pm.arr_c = pe.arr_c, pm.fixed = pe.fixed_meta;
+    pm.arr_c = pe.arr_c, pm.fixed = pe.fixed_meta, pm.bw_max = pe.bw_max;
     if (!pe.vec_c) return hipSuccess;
     Expr e;
     expr_from_page(pe.exp_t, pe.var, e);

@@ -74,7 +74,7 @@ hipError_t launch_page_int(unsigned W, int mode, const uint8_t* page, const Page
     case 8: return page_int_w<8>(mode, page, pm, vec_c, out, sel, s);
     case 16: return page_int_w<16>(mode, page, pm, vec_c, out, sel, s);
     case 32: return page_int_w<32>(mode, page, pm, vec_c, out, sel, s);
-    case 64: return page_int_w<64>(mode, page, pm, vec_c, out, sel, s);
+    case 64: return page_int64_wave(mode, page, pm, vec_c, out, sel, s);
     default: return hipErrorInvalidValue;
     }
 }

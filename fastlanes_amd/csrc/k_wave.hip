@@ -1,0 +1,212 @@
+// k_wave.hip -- integer pages of 64-bit values: one wave per vector, output order straight from the packed rows.
+//
+// The wave stages its vector's packed rows in LDS (16-byte chunks, loaded one vector ahead) and then every lane takes
+// the output positions that it will store: iteration k, lane l holds values 128 k + 2 l and the next, which are positions
+// p = 2 (l % 32) and p + 1 of FastLanes lane 2 k + l / 32, so a store instruction writes 1 KiB of consecutive output and
+// nothing is staged on the way out. p does not depend on k: a lane's two bit offsets, LDS addresses and shifts are set
+// once per vector, and an iteration reads them at a constant 16 bytes further (the rows of FastLanes lanes i and i + 2
+// are 16 bytes apart). DELTA scans the differences over the 32 lanes of a half wave.
+//
+// The form that this replaces gave a thread a whole FastLanes lane (64 values by a compile-time bit width, through 34 KB
+// of LDS per wave, so four waves per compute unit): 113.9 us for 65536 vectors of int64 timestamps (DELTA, bit width 7;
+// 537 MB out, 69 MB in), 103.0 us here, 5.9 TB/s against 6.9 of a fill. A predicate on 32768 FFOR vectors of bit width
+// 17, where the old form staged every value in LDS to compare it: 68.9 us, 30.1 us here. Blocks of two waves measured
+// best from 32768 vectors on (DELTA: 103.5 us, four waves 106.5, eight 111.7).
+//
+// Bit widths are run-time values (uniform over the wave). Rows sit 144 bytes apart in LDS, so that the eight rows that
+// the lanes of an instruction read at small bit widths are on different banks; a value is cut from two dwords (bit
+// widths up to 32) or three.
+// Page layout and expressions: page_kernels.hpp (int_meta).
+#include "launch.hpp"
+#include "page_kernels.hpp"
+
+namespace fls {
+namespace {
+
+constexpr unsigned kRow    = 144;  // LDS bytes per packed row of 128
+constexpr unsigned kAhead  = 4;    // 16-byte chunks per lane loaded ahead: bit widths up to 32
+constexpr unsigned kLbRows = 128;  // LDS bytes of a DELTA vector's lane bases
+
+// Inclusive sum over the first 32 lanes or the last 32 (WAVE: over all 64).
+template <bool WAVE>
+__device__ __forceinline__ uint32_t lane_scan(uint32_t x) {
+    x += __builtin_amdgcn_update_dpp(0u, x, 0x111, 0xf, 0xf, false);  // row_shr:1
+    x += __builtin_amdgcn_update_dpp(0u, x, 0x112, 0xf, 0xf, false);  // row_shr:2
+    x += __builtin_amdgcn_update_dpp(0u, x, 0x114, 0xf, 0xf, false);  // row_shr:4
+    x += __builtin_amdgcn_update_dpp(0u, x, 0x118, 0xf, 0xf, false);  // row_shr:8
+    x += __builtin_amdgcn_update_dpp(0u, x, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+    if constexpr (WAVE) x += __builtin_amdgcn_update_dpp(0u, x, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2, 3
+    return x;
+}
+template <bool WAVE>
+__device__ __forceinline__ uint64_t lane_scan(uint64_t x) {
+    const unsigned lane = threadIdx.x % 64;
+    for (unsigned d = 1; d < (WAVE ? 64 : 32); d <<= 1) {
+        const uint64_t y = __shfl_up((unsigned long long)x, d, WAVE ? 64 : 32);
+        if ((WAVE ? lane : lane % 32) >= d) x += y;
+    }
+    return x;
+}
+
+template <typename T>
+__device__ __forceinline__ T uniform(T x) {
+    if constexpr (sizeof(T) == 8)
+        return (T)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)((uint64_t)x >> 32)) << 32) |
+                   (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)x));
+    else return (T)__builtin_amdgcn_readfirstlane((uint32_t)x);
+}
+
+// Packed rows of a vector: the first kAhead chunks of every lane, in flight while the vector before is decoded.
+struct Ahead {
+    v4u c[kAhead];
+};
+__device__ __forceinline__ void load_ahead(const uint8_t* pk, uint32_t chunks, unsigned lane, Ahead& a) {
+    static_for<kAhead>([&](auto k) {
+        const uint32_t c = lane + 64u * decltype(k)::value;
+        if (c < chunks) a.c[k] = ld16(pk + 16 * c);
+    });
+}
+__device__ __forceinline__ uint32_t row_place(uint32_t c) { return (c >> 3) * kRow + (c & 7) * 16; }
+__device__ __forceinline__ void stage_rows(const uint8_t* pk, uint32_t chunks, unsigned lane, const Ahead& a, uint8_t* rows) {
+    static_for<kAhead>([&](auto k) {
+        const uint32_t c = lane + 64u * decltype(k)::value;
+        if (c < chunks) *reinterpret_cast<v4u*>(rows + row_place(c)) = a.c[k];
+    });
+    for (uint32_t c = lane + 64u * kAhead; c < chunks; c += 64u) *reinterpret_cast<v4u*>(rows + row_place(c)) = ld16(pk + 16 * c);
+}
+
+// MODE 0 UNCOMPRESSED, 1 FFOR, 2 DELTA, as k_page_int. SEL: a predicate's bitmap instead of values; iteration k, lane l
+// then holds value 64 k + l alone, so that a ballot is the bitmap's word k.
+template <int MODE, bool NT, bool SEL>
+__global__ __launch_bounds__(kMaxBlock) void k_wave_int64(const uint8_t* __restrict__ page, PageMeta pm, uint32_t vec_c,
+                                                          uint8_t* __restrict__ out, SelArgs sa, uint32_t wave_lds) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t fls_lds[];
+    constexpr unsigned P  = MODE == 0 ? 0 : (MODE == 2 ? 3 : 2);
+    constexpr unsigned NV = SEL ? 1 : 2, IT = 16 / NV;  // values per lane and iteration, iterations
+    const unsigned     lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    uint8_t* const     lb   = fls_lds + wave * wave_lds;  // DELTA lane bases, then the rows
+    uint8_t* const     rows = lb + (MODE == 2 ? kLbRows : 0);
+    const unsigned     p    = SEL ? lane : 2 * (lane % 32), half = SEL ? 0 : lane / 32;
+    const unsigned     j    = 8 * (p % 8) + order8(p / 8);
+    const uint64_t     N = vec_c, stride = (uint64_t)gridDim.x * (blockDim.x / 64);
+    uint64_t           v = (uint64_t)blockIdx.x * (blockDim.x / 64) + wave;
+    auto meta   = [&](uint64_t u) { return int_meta<64, MODE>(page, pm, u, lane % 16); };
+    // (never more rows than the launch's LDS was sized for, whatever the page holds)
+    auto width  = [&](const IntMeta& m) -> uint32_t { return MODE == 0 ? 64u : min(uniform(m.bw), pm.bw_max); };
+    auto packed = [&](const IntMeta& m) { return page + pm.off[P] + uniform(m.ep); };
+    IntMeta m0 {}, m1 {};
+    Ahead   a;
+    if (v < N) {
+        m0 = meta(v);
+        load_ahead(packed(m0), 8 * width(m0), lane, a);
+    }
+    if (v + stride < N) m1 = meta(v + stride);
+    for (; v < N; v += stride) {
+        const uint32_t bw   = width(m0);
+        const uint64_t base = MODE == 0 ? 0ull : uniform(m0.base);
+        stage_rows(packed(m0), 8 * bw, lane, a, rows);
+        if constexpr (MODE == 2)
+            if (lane < 16) reinterpret_cast<uint64_t*>(lb)[lane] = m0.lb;
+        m0 = m1;
+        if (v + stride < N) load_ahead(packed(m0), 8 * width(m0), lane, a);
+        if (v + 2 * stride < N) m1 = meta(v + 2 * stride);
+        wave_sync();
+        // a lane's values start at bit j * bw (and (j + 8) * bw) of their FastLanes lane: dword d of it sits in row
+        // d / 2, and dword d + 2 one row further
+        const uint8_t* at[NV];
+        int32_t        next[NV];
+        uint32_t       sh[NV];
+        static_for<NV>([&](auto e) {
+            const uint32_t bit = (j + 8 * decltype(e)::value) * bw, d = bit >> 5;
+            at[e]              = rows + (d >> 1) * kRow + 4 * (d & 1) + 8 * half;
+            next[e]            = d & 1 ? (int32_t)kRow - 4 : 4;
+            sh[e]              = bit & 31;
+        });
+        const uint64_t mask = bw >= 64 ? ~0ull : ((1ull << bw) - 1);
+        uint64_t       word = 0;
+        uint32_t       cnt  = 0;
+        auto           done = [&](auto k, const uint64_t (&x)[NV]) {
+            if constexpr (SEL) {
+                const uint64_t b = __ballot(sa.dbl ? sel_pred<uint64_t, true>(x[0], sa) : sel_pred<uint64_t, false>(x[0], sa));
+                if (lane == decltype(k)::value) word = b;
+                cnt += (uint32_t)__popcll(b);
+            } else {
+                st16<NT>(out + v * 8192 + 1024 * k + 16 * lane, v4u {(uint32_t)x[0], (uint32_t)(x[0] >> 32), (uint32_t)x[NV - 1],
+                                                                    (uint32_t)(x[NV - 1] >> 32)});
+            }
+        };
+        constexpr unsigned SB = SEL ? 8 : 16;  // LDS bytes between the rows of an iteration and the next
+        auto dword = [&](const uint8_t* q) { return *reinterpret_cast<const uint32_t*>(q); };
+        if (MODE == 2 && bw <= 26) {
+            // 64 differences sum to less than 2^32 without their base, which is added p + 1 times
+            uint64_t pb[NV];
+            static_for<NV>([&](auto e) { pb[e] = base * (p + 1 + decltype(e)::value); });
+            static_for<IT>([&](auto k) {
+                uint32_t u[NV];
+                static_for<NV>([&](auto e) {
+                    u[e] = __builtin_amdgcn_alignbit(dword(at[e] + SB * k + next[e]), dword(at[e] + SB * k), sh[e]) & (uint32_t)mask;
+                });
+                const uint32_t s = lane_scan<SEL>(NV == 2 ? u[0] + u[NV - 1] : u[0]);
+                const uint64_t b = *reinterpret_cast<const uint64_t*>(lb + SB * k + 8 * half);
+                uint64_t       x[NV];
+                if constexpr (NV == 2) x[0] = b + pb[0] + (s - u[1]);
+                x[NV - 1] = b + pb[NV - 1] + s;
+                done(k, x);
+            });
+        } else {
+            static_for<IT>([&](auto k) {
+                uint64_t x[NV];
+                static_for<NV>([&](auto e) {
+                    const uint32_t lo = dword(at[e] + SB * k), mid = dword(at[e] + SB * k + next[e]);
+                    const uint32_t a0 = __builtin_amdgcn_alignbit(mid, lo, sh[e]);
+                    uint32_t       a1 = 0;
+                    if (bw > 32) a1 = __builtin_amdgcn_alignbit(dword(at[e] + SB * k + kRow), mid, sh[e]);
+                    x[e] = (((uint64_t)a1 << 32 | a0) & mask) + base;
+                });
+                if constexpr (MODE == 2) {
+                    const uint64_t s = lane_scan<SEL>(NV == 2 ? x[0] + x[NV - 1] : x[0]);
+                    const uint64_t b = *reinterpret_cast<const uint64_t*>(lb + SB * k + 8 * half);
+                    if constexpr (NV == 2) x[0] = b + s - x[1];
+                    x[NV - 1] = b + s;
+                }
+                done(k, x);
+            });
+        }
+        if constexpr (SEL) {
+            if (lane < 16) sa.bitmap[v * 16 + lane] = word;
+            if (lane == 0) sa.counts[v] = cnt;
+        }
+        wave_sync();
+    }
+}
+
+}  // namespace
+
+hipError_t page_int64_wave(int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
+                           const SelArgs* sel, hipStream_t s) {
+    Tune           t  = tune_for(mode == 0 ? FAM_PAGE_UNC : mode == 1 ? FAM_PAGE_FFOR : FAM_PAGE_DELTA, 64, 255);
+    const unsigned bw = mode == 0 ? 64u : pm.bw_max ? pm.bw_max : 1u;
+    const unsigned wl = (bw + 1) * kRow + (mode == 2 ? kLbRows : 0);  // a value's last dword may lie in the row after
+    unsigned       waves = t.block / 64;
+    while (waves > 1 && waves * wl > 65536) --waves;
+    t.block            = (uint16_t)(64 * waves);
+    const dim3     g(grid_for(vec_c, t, 64)), b(t.block);
+    const SelArgs  sa = sel ? *sel : SelArgs {};
+#define L(M, NT, SL) hipLaunchKernelGGL((k_wave_int64<M, NT, SL>), g, b, waves * wl, s, page, pm, vec_c, out, sa, wl)
+#define LM(M)                      \
+    if (sel) L(M, false, true);    \
+    else if (t.nt & 1) L(M, true, false); \
+    else L(M, false, false);
+    if (mode == 0) {
+        LM(0)
+    } else if (mode == 1) {
+        LM(1)
+    } else {
+        LM(2)
+    }
+#undef LM
+#undef L
+    return hipGetLastError();
+}
+
+}  // namespace fls

@@ -78,6 +78,9 @@ hipError_t launch_hzl(unsigned DW, const uint8_t* enc, const HzlChunk* chunks, u
 template <int W>
 hipError_t page_int_w(int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
                       const SelArgs* sel, hipStream_t s);
+// integer pages of 64-bit values (k_wave.hip)
+hipError_t page_int64_wave(int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
+                           const SelArgs* sel, hipStream_t s);
 template <int W>
 hipError_t page_patch_w(int var, bool rsum, const void* dict, uint32_t dict_n, const uint8_t* page, const PageMeta& pm,
                         uint32_t vec_c, uint8_t* out, uint32_t* err, const SelArgs* sel, const uint8_t* exc,

@@ -254,6 +254,7 @@ struct PageMeta {
     uint32_t off[6];
     uint32_t arr_c;
     uint32_t fixed;
+    uint32_t bw_max;  // largest FFOR bit width of the page's vectors
 };
 
 // Per-vector metadata of an integer page: bit width, FFOR base, the thread's lane base (DELTA) and the entry point of
@@ -291,8 +292,8 @@ __device__ __forceinline__ IntMeta int_meta(const uint8_t* page, const PageMeta&
 // Staged loop as staged_vector_loop, software-pipelined one step deep: the metadata of the vector a thread decodes
 // next is loaded right after the current vector's values are decoded, so it arrives while the wave writes its
 // output, and each step waits on one round of loads (the packed values) instead of three dependent ones.
-// DIRECT (32/64-bit values): no LDS staging; each thread writes its lane's contiguous segment (128 or 512 bytes,
-// whole lines) straight to HBM, so occupancy is bounded by registers instead of the staging buffers.
+// DIRECT (32-bit values): no LDS staging; each thread writes its lane's contiguous segment (128 bytes, whole lines)
+// straight to HBM, so occupancy is bounded by registers instead of the staging buffers. 64-bit pages: k_wave.hip.
 template <int W, int MODE, bool NT, bool DIRECT = false, bool SEL = false>
 __global__ __launch_bounds__(kMaxBlock) void k_page_int(const uint8_t* __restrict__ page, PageMeta pm, uint32_t vec_c,
                                                         uint8_t* __restrict__ out, SelArgs sa) {
@@ -309,9 +310,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_page_int(const uint8_t* __restric
     uint64_t       v0     = ((uint64_t)blockIdx.x * waves + wave) * WS::VPW;
     IntMeta        m {};
     if (v0 + slot < N) m = int_meta<W, MODE>(page, pm, v0 + slot, t);
-    if constexpr (SEL && W <= 32) {
-        // predicate pushdown: values become bits in registers; LDS holds only the wave's bitmaps (128 B per vector).
-        // (64-bit values take the staged path below: their register form compiled to slower code.)
+    if constexpr (SEL) {
+        // predicate pushdown: values become bits in registers; LDS holds only the wave's bitmaps (128 B per vector)
         using T         = typename uint_of<W>::type;
         uint32_t* wbits = reinterpret_cast<uint32_t*>(fls_lds) + wave * (WS::VPW * 32);
         for (; v0 < N; v0 += stride) {
@@ -362,8 +362,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_page_int(const uint8_t* __restric
         if constexpr (!DIRECT) {
             wave_sync();
             const uint64_t left = N - v0;
-            wave_out<typename uint_of<W>::type, TPV, VB, NT, SEL>(wl, out, v0, left < WS::VPW ? (uint32_t)left : WS::VPW,
-                                                                  lane, sa);
+            wave_out<typename uint_of<W>::type, TPV, VB, NT, false>(wl, out, v0, left < WS::VPW ? (uint32_t)left : WS::VPW,
+                                                                    lane, sa);
             wave_sync();
         }
     }

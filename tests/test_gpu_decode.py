@@ -630,6 +630,48 @@ def test_predicate_pushdown_matches_numpy(torch_cuda, oracle, dtype, eid):
     np.testing.assert_array_equal(d_cnt.cpu().numpy(), both.reshape(-1, 1024).sum(axis=1))
 
 
+@pytest.mark.parametrize("eid", [0, 1, 11])
+@pytest.mark.parametrize("shape", [(64, 1), (256, 2), (512, 0)])
+def test_wave_per_vector_pages_every_bit_width(torch_cuda, oracle, eid, shape):
+    """64-bit integer pages with one vector of every bit width 0 .. 64 in one page (a value cut from two dwords or
+    three, sums in 32 or 64 bits), a wave striding over many vectors or each taking one; decode and select."""
+    import ctypes as C
+
+    torch, (block, maxb) = torch_cuda, shape
+    g = np.random.default_rng(eid)
+    rows = []
+    for w in list(range(65)) + [64, 0, 33, 26, 1]:
+        top = (1 << w) - 1
+        r = g.integers(0, top, 1024, dtype=np.uint64, endpoint=True)
+        r[g.permutation(1024)[:2]] = (0, top)  # exactly w bits
+        rows.append(np.cumsum(r, dtype=np.uint64) if eid == 11 else r + np.uint64((1 << 64) - 1 - top) // np.uint64(2))
+    x = np.concatenate(rows)
+    enc = oracle.encode_column(x, eid)
+    want = oracle.decode_column(enc, np.uint64, x.size)
+    n_vec = x.size // 1024
+    lib = fa.lib()
+    try:
+        fa.check(lib.fls_gpu_tune_set({0: 1, 1: 2, 11: 3}[eid], 64, 255, block, 1, maxb), "tune_set")
+        plan = fa.Plan(enc, np.uint64)
+        d_in = dev(torch, enc)
+        d_out = torch.full((x.nbytes + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+        plan.decode(d_in.data_ptr(), d_out.data_ptr(), x.nbytes)
+        plan.check()
+        np.testing.assert_array_equal(to_np(d_out, np.uint64, x.size), want)
+        assert bool((d_out[x.nbytes:] == 0x5A).all())
+        c = x[517]
+        d_bm = torch.zeros(16 * n_vec, dtype=torch.int64, device="cuda")
+        d_cnt = torch.zeros(n_vec, dtype=torch.int32, device="cuda")
+        plan.select(d_in.data_ptr(), "<", c, d_bm.data_ptr(), d_cnt.data_ptr())
+        plan.check()
+        np.testing.assert_array_equal(d_bm.cpu().numpy().view(np.uint64), _bitmap_words(want < c))
+        np.testing.assert_array_equal(d_cnt.cpu().numpy(), (want < c).reshape(-1, 1024).sum(axis=1))
+    finally:
+        path = os.path.join(os.path.dirname(os.path.abspath(fa.__file__)), "tuning.txt")
+        lib.fls_gpu_tune_load.argtypes = [C.c_char_p]
+        assert lib.fls_gpu_tune_load(path.encode()) > 0
+
+
 def test_predicate_on_doubles(torch_cuda):
     """DOUBLE columns (UNCOMPRESSED) compare as IEEE values: NaN selects nothing but !=, -0.0 equals 0.0."""
     torch = torch_cuda
