@@ -95,6 +95,7 @@ hipError_t launch_page_patch(unsigned W, int var, bool rsum, const void* dict, u
 hipError_t launch_page_rle(unsigned W, int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
                            uint32_t* err, hipStream_t s, const SelArgs* sel, const RunSrc* runs, bool pos_bw1) {
     if (!vec_c) return hipSuccess;
+    if (W >= 32 && var == 2 && pos_bw1) return page_rle_wave(W, page, pm, vec_c, out, err, sel, runs, s);
     switch (W) {
     case 8: return page_rle_w<8>(var, page, pm, vec_c, out, err, sel, runs, pos_bw1, s);
     case 16: return page_rle_w<16>(var, page, pm, vec_c, out, err, sel, runs, pos_bw1, s);

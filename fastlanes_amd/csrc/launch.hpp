@@ -81,6 +81,8 @@ hipError_t page_int_w(int mode, const uint8_t* page, const PageMeta& pm, uint32_
 // integer pages of 64-bit values (k_wave.hip)
 hipError_t page_int64_wave(int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
                            const SelArgs* sel, hipStream_t s);
+hipError_t page_rle_wave(unsigned W, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out, uint32_t* err,
+                         const SelArgs* sel, const RunSrc* runs, hipStream_t s);  // W 32/64, positions of bit width <= 1
 template <int W>
 hipError_t page_patch_w(int var, bool rsum, const void* dict, uint32_t dict_n, const uint8_t* page, const PageMeta& pm,
                         uint32_t vec_c, uint8_t* out, uint32_t* err, const SelArgs* sel, const uint8_t* exc,

@@ -235,6 +235,92 @@ def test_rle_positions_past_the_runs_are_clamped_and_reported(torch_cuda, oracle
     np.testing.assert_array_equal(got[keep], x.reshape(8, 1024)[keep])
 
 
+def _rle_model(enc, dt):
+    """Values (clamped like the decoder) and the count of positions past the runs of a one-page RLE column (run values, u16 position lanes of bit width 0 or 1),
+    straight from the layout."""
+    vec_c = int(enc[4]) | int(enc[5]) << 8
+    off = enc[8:28].view(np.uint32).astype(np.int64)
+    ep = np.zeros((vec_c, 5), dtype=np.int64)
+    ep[1:] = enc[28: 28 + 20 * (vec_c - 1)].copy().view(np.uint32).reshape(-1, 5)
+    sz = np.dtype(dt).itemsize
+    i, p = np.arange(64)[:, None], np.arange(16)[None, :]
+    place = 64 * (i % 16) + 16 * np.array([0, 2, 1, 3])[i // 16] + p
+    out, bad = np.empty((vec_c, 1024), dt), 0
+    for v in range(vec_c):
+        r1 = ep[v + 1, 0] if v + 1 < vec_c else off[1] - off[0]
+        runs = enc[off[0] + ep[v, 0]: off[0] + r1].copy().view(dt)
+        lb = enc[off[1] + ep[v, 1]:][:128].copy().view(np.uint16).astype(np.int64)
+        bw, base = int(enc[off[2] + ep[v, 2]]), int(enc[off[3] + ep[v, 3]:][:2].copy().view(np.uint16)[0])
+        w = enc[off[4] + ep[v, 4]:][:128].copy().view(np.uint16).astype(np.int64) if bw else np.zeros(64, np.int64)
+        diff = (w[:, None] >> (2 * (p % 8) + p // 8)) & 1  # in value order
+        pos = (lb[:, None] + np.cumsum(diff, axis=1) + (p + 1) * base) & 0xFFFF
+        bad += int((pos >= runs.size).sum())
+        out[v, place.ravel()] = runs[np.minimum(pos, runs.size - 1)].ravel()
+    return out, bad
+
+
+@pytest.mark.parametrize("W", [32, 64])
+@pytest.mark.parametrize("form", ["runs", "lane_base", "base", "many_runs"])
+def test_wave_rle_pages(torch_cuda, oracle, W, form):
+    """One-wave-per-vector RLE pages: 1 .. 1024 runs a vector; lane bases that leave the runs or wrap; a FFOR base;
+    a vector that owns more runs than it has values. Decode and select, waves with one vector and with many."""
+    import ctypes as C
+
+    torch, lib, dt = torch_cuda, fa.lib(), W2DT[W]
+    g = np.random.default_rng(W)
+    rows = []
+    for n in [1, 2, 63, 64, 65, 255, 256, 257, 512, 1023, 1024, 1, 300, 40] * 2:
+        idx = np.zeros(1024, np.int64)
+        idx[np.sort(g.permutation(1023)[: n - 1]) + 1] = 1
+        rows.append(g.integers(0, np.iinfo(dt).max, n, dtype=dt)[np.cumsum(idx)])
+    x = np.concatenate(rows)
+    enc = oracle.encode_column(x, 6).copy()
+    n_vec = len(rows)
+    want, bad = _rle_model(enc, dt)
+    np.testing.assert_array_equal(want.ravel(), x)
+    assert bad == 0
+    off = enc[8:28].copy().view(np.uint32)
+    put = lambda at, val: enc.__setitem__(slice(int(at), int(at) + 2), np.array([val], np.uint16).view(np.uint8))
+    if form == "lane_base":  # vectors 3 and 12 (fixed 128-byte lane bases), lanes 5 and 40
+        put(off[1] + 3 * 128 + 2 * 5, 2000)
+        put(off[1] + 12 * 128 + 2 * 40, 65535)
+    elif form == "base":
+        for v, val in ((7, 1), (10, 3), (13, 65530)):
+            put(off[3] + 2 * v, val)
+    elif form == "many_runs":  # vector 9 takes nearly all runs of vector 10, whose positions then clamp
+        eps = enc[28: 28 + 20 * (n_vec - 1)].view(np.uint32).reshape(-1, 5)
+        eps[9, 0] += 1000 * (W // 8)
+        for lane in range(0, 64, 3):
+            put(off[1] + 9 * 128 + 2 * lane, 990 + 10 * lane)
+    want, bad = _rle_model(enc, dt)
+    assert (bad > 0) == (form != "runs")
+    d_in = dev(torch, enc)
+    c = x[700]
+    try:
+        for block, maxb in ((256, 0), (64, 1)):
+            print(f"wave rle W={W} {form} block={block} max_blocks={maxb}", flush=True)
+            fa.check(lib.fls_gpu_tune_set(4, W, 255, block, 1, maxb), "tune_set")
+            plan = fa.Plan(enc, dt)
+            d_out = torch.full((x.nbytes + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+            d_bm = torch.zeros(16 * n_vec, dtype=torch.int64, device="cuda")
+            d_cnt = torch.zeros(n_vec, dtype=torch.int32, device="cuda")
+            plan.decode(d_in.data_ptr(), d_out.data_ptr(), x.nbytes)
+            plan.select(d_in.data_ptr(), "<", c, d_bm.data_ptr(), d_cnt.data_ptr())
+            if bad:
+                with pytest.raises(fa.FlsError):
+                    plan.check()
+            else:
+                plan.check()
+            np.testing.assert_array_equal(to_np(d_out, dt, x.size).reshape(-1, 1024), want)
+            assert bool((d_out[x.nbytes:] == 0x5A).all())
+            np.testing.assert_array_equal(d_bm.cpu().numpy().view(np.uint64), _bitmap_words(want.ravel() < c))
+            np.testing.assert_array_equal(d_cnt.cpu().numpy(), (want < c).sum(axis=1))
+    finally:
+        path = os.path.join(os.path.dirname(os.path.abspath(fa.__file__)), "tuning.txt")
+        lib.fls_gpu_tune_load.argtypes = [C.c_char_p]
+        assert lib.fls_gpu_tune_load(path.encode()) > 0
+
+
 @pytest.mark.parametrize("W", [8, 16])
 def test_rle_two_lane_kernel(torch_cuda, oracle, W):
     """Tuning bit 2 of the RLE family switches narrow pages back to the two-lanes-per-thread kernel (the one that
