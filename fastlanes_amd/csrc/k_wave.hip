@@ -1,5 +1,5 @@
 // k_wave.hip -- one wave per vector, output order straight from the packed rows: integer pages of 64-bit values, RLE
-// pages of 32/64-bit values (k_wave_rle, below).
+// and dictionary pages of 32/64-bit values (k_wave_rle and k_wave_dict, below).
 //
 // Integer pages. The wave stages its vector's packed rows in LDS (16-byte chunks, loaded one vector ahead) and then every lane takes
 // the output positions that it will store: iteration k, lane l holds values 128 k + 2 l and the next, which are positions
@@ -292,6 +292,152 @@ __global__ __launch_bounds__(kMaxBlock) void k_wave_rle(const uint8_t* __restric
     }
 }
 
+// Dictionary pages of 32/64-bit values: u32 codes (VAR 1 raw, 2 FFOR, 7 DELTA; dict_vector has the layout), out[i] = dict[code[i]]. As
+// k_wave_int64, with the codes' rows of 32 lanes: value o is position p = o % 32 of code lane o / 64 + 16 (o / 32 % 2).
+// A lane holds the 16 bytes that it stores, NV values from one code lane, and gathers them from the dictionary: IN_LDS,
+// every block first copies it there or (hz.chunks) decodes its HZL chunks into it; else from L2. DELTA sums over the
+// 32 / NV lanes that share a code lane. The form before decoded a code lane a thread by a compile-time bit width and
+// staged every value in LDS on its way out: 97.2 us for 65536 vectors of int32 with 4096 keys (two pages; 268 MB out,
+// 101 MB in), 76.6 us here; 60000 keys (from L2) 186 and 121 us; DELTA codes 158 and 117 us; 32768 vectors of int64 with
+// 2000 keys 99.8 and 61.0 us, with 40000 101.7 and 75 us; 2000 vectors of int32 10.7 and 7.0 us. What is left over a copy's
+// rate is the start of each page (metadata, rows and dictionary are loads that wait for each other).
+template <unsigned G>
+__device__ __forceinline__ uint32_t group_scan(uint32_t x, unsigned lane) {  // inclusive, over groups of G lanes
+    if constexpr (G == 32) return lane_scan<false>(x);
+    static_for<4>([&](auto d) {
+        constexpr unsigned n = 1u << decltype(d)::value;
+        if constexpr (n < G) {
+            const uint32_t y = __builtin_amdgcn_update_dpp(0u, x, 0x110 + n, 0xf, 0xf, false);  // row_shr
+            x += lane % G >= n ? y : 0u;
+        }
+    });
+    return x;
+}
+
+// A block decodes a dictionary's HZL chunks (no exceptions) into LDS, four values a thread at once: chunk headers, then
+// packed words, are two rounds of loads for 2048 values. Full chunks hold 1024 values and the raw tail follows them.
+template <typename D>
+__device__ __forceinline__ void fill_dict(const HzlSrc& hz, uint32_t dict_n, D* ldict) {
+    constexpr unsigned DW = 8 * sizeof(D), L = 1024 / DW;
+    for (uint32_t b0 = 0; b0 < dict_n; b0 += 4 * blockDim.x) {
+        D        lo[4], hi[4], base[4];
+        uint32_t bw[4], sh[4];
+        static_for<4>([&](auto u) {
+            const uint32_t b = b0 + decltype(u)::value * blockDim.x;
+            if (b >= dict_n) return;
+            uint32_t g = b + threadIdx.x;
+            g          = g < dict_n ? g : dict_n - 1;
+            const uint32_t  c  = __builtin_amdgcn_readfirstlane(min(g >> 10, hz.n_chunks - 1)), k = g - (c << 10);
+            const HzlChunk& ch = hz.chunks[c];
+            const uint8_t*  in = hz.enc + ch.src;
+            bw[u] = ch.bw, base[u] = (D)ch.base;
+            const uint32_t bit = k / L * bw[u], w = bit / DW, lane = k % L;
+            sh[u] = bit % DW;
+            // the tail: value k as it stands; bit width 0: any bytes (the chunk's header) and an empty mask
+            const uint32_t o0 = bw[u] == 255 ? k : w * L + lane, o1 = bw[u] == 255 ? k : (w + 1 < bw[u] ? w + 1 : w) * L + lane;
+            const uint8_t* at = bw[u] ? in : in - 12;
+            lo[u] = load_t<D>(at + (bw[u] ? (uint64_t)o0 * sizeof(D) : 0ull));
+            hi[u] = load_t<D>(at + (bw[u] ? (uint64_t)o1 * sizeof(D) : 0ull));
+        });
+        static_for<4>([&](auto u) {
+            const uint32_t b = b0 + decltype(u)::value * blockDim.x;
+            if (b >= dict_n) return;
+            D v = bw[u] == 255 ? lo[u] : (D)((lo[u] >> sh[u]) | (sh[u] ? hi[u] << (DW - sh[u]) : (D)0));
+            if (bw[u] < DW) v &= ((D)1 << bw[u]) - 1;
+            if (bw[u] != 255) v += base[u];
+            if (b + threadIdx.x < dict_n) ldict[b + threadIdx.x] = v;
+        });
+    }
+}
+
+template <typename T, int VAR, bool NT, bool IN_LDS, bool SEL>
+__global__ __launch_bounds__(kMaxBlock) void k_wave_dict(const uint8_t* __restrict__ page, PageMeta pm, uint32_t vec_c,
+                                                         const T* __restrict__ dict, uint32_t dict_n,
+                                                         uint8_t* __restrict__ out, uint32_t* err, SelArgs sa, HzlSrc hz,
+                                                         uint32_t dict_lds, uint32_t wave_lds) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t fls_lds[];
+    if (dict_n == 0) return;  // the host rejects such pages
+    constexpr unsigned P  = VAR == 1 ? 0 : (VAR == 7 ? 3 : 2);
+    constexpr unsigned NV = SEL ? 1 : 16 / sizeof(T), IT = 16 / NV;  // values per lane and iteration, iterations
+    T* const ldict = reinterpret_cast<T*>(fls_lds);
+    const unsigned lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    uint8_t* const lb   = fls_lds + dict_lds + wave * wave_lds;  // DELTA lane bases, then the rows
+    uint8_t* const rows = lb + (VAR == 7 ? kLbRows : 0);
+    const unsigned q = NV * lane, p = q % 32, col = q / 64 + 16 * (q / 32 % 2);  // an iteration on: NV code lanes further
+    const uint32_t last = dict_n - 1;
+    const uint64_t N = vec_c, stride = (uint64_t)gridDim.x * (blockDim.x / 64);
+    uint64_t       v = (uint64_t)blockIdx.x * (blockDim.x / 64) + wave;
+    auto meta   = [&](uint64_t u) { return code_meta<VAR>(page, pm, u, lane % 32); };
+    auto width  = [&](const CodeMeta& m) -> uint32_t { return VAR == 1 ? 32u : min(uniform(m.bw), pm.bw_max); };
+    auto packed = [&](const CodeMeta& m) { return page + pm.off[P] + uniform(m.ep); };
+    CodeMeta m0 {}, m1 {};
+    Ahead    a;
+    bool     bad = false;
+    if (v < N) {
+        m0 = meta(v);
+        load_ahead(packed(m0), 8 * width(m0), lane, a);
+    }
+    if (v + stride < N) m1 = meta(v + stride);
+    if constexpr (IN_LDS) {
+        if (hz.chunks) fill_dict(hz, dict_n, ldict);
+        else
+            for (uint32_t i = threadIdx.x; i < dict_n; i += blockDim.x) ldict[i] = dict[i];
+        __syncthreads();
+    }
+    for (; v < N; v += stride) {
+        const uint32_t bw   = width(m0);
+        const uint32_t base = VAR == 1 ? 0u : uniform(m0.base);
+        stage_rows(packed(m0), 8 * bw, lane, a, rows);
+        if constexpr (VAR == 7)
+            if (lane < 32) reinterpret_cast<uint32_t*>(lb)[lane] = m0.lb;
+        m0 = m1;
+        if (v + stride < N) load_ahead(packed(m0), 8 * width(m0), lane, a);
+        if (v + 2 * stride < N) m1 = meta(v + 2 * stride);
+        wave_sync();
+        const uint32_t mask = bw >= 32 ? ~0u : (1u << bw) - 1;
+        uint64_t       word = 0;
+        uint32_t       cnt  = 0;
+        const uint8_t* at[NV];  // the dword that the lane's first code e starts in; the next is a row further
+        uint32_t       sh[NV];
+        static_for<NV>([&](auto e) {
+            const uint32_t bit = j_of_p<32>(p + decltype(e)::value) * bw;
+            at[e]              = rows + (bit >> 5) * kRow + 4 * col;
+            sh[e]              = bit & 31;
+        });
+        static_for<IT>([&](auto k) {
+            constexpr unsigned S = 4 * NV * decltype(k)::value;
+            auto     dword = [&](const uint8_t* r) { return *reinterpret_cast<const uint32_t*>(r + S); };
+            uint32_t c[NV];
+            T        vals[NV];
+            static_for<NV>([&](auto e) { c[e] = (__builtin_amdgcn_alignbit(dword(at[e] + kRow), dword(at[e]), sh[e]) & mask) + base; });
+            if constexpr (VAR == 7) {
+                static_for<NV - 1>([&](auto e) { c[e + 1] += c[e]; });
+                const uint32_t before = group_scan<32 / NV>(c[NV - 1], lane) - c[NV - 1] +
+                                        *reinterpret_cast<const uint32_t*>(lb + S + 4 * col);
+                static_for<NV>([&](auto e) { c[e] += before; });
+            }
+            static_for<NV>([&](auto e) {
+                bad |= c[e] > last;
+                c[e]    = min(c[e], last);
+                vals[e] = IN_LDS ? ldict[c[e]] : dict[c[e]];
+            });
+            if constexpr (SEL) {
+                const uint64_t b = __ballot(sizeof(T) == 8 && sa.dbl ? sel_pred<T, true>(vals[0], sa) : sel_pred<T, false>(vals[0], sa));
+                if (lane == decltype(k)::value) word = b;
+                cnt += (uint32_t)__popcll(b);
+            } else {
+                st16<NT>(out + v * (1024 * sizeof(T)) + 1024 * decltype(k)::value + 16 * lane, *reinterpret_cast<const v4u*>(vals));
+            }
+        });
+        if constexpr (SEL) {
+            if (lane < 16) sa.bitmap[v * 16 + lane] = word;
+            if (lane == 0) sa.counts[v] = cnt;
+        }
+        wave_sync();
+    }
+    if (bad) atomicOr(err, 2u);
+}
+
 }  // namespace
 
 hipError_t page_int64_wave(int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
@@ -342,6 +488,68 @@ hipError_t page_rle_wave(unsigned W, const uint8_t* page, const PageMeta& pm, ui
                          const SelArgs* sel, const RunSrc* runs, hipStream_t s) {
     const RunSrc rs = runs ? *runs : RunSrc {page + pm.off[0], pm.off[1] - pm.off[0], W == 64 ? 3u : 2u};
     return W == 64 ? rle_wave<uint64_t>(page, pm, vec_c, out, err, sel, rs, s) : rle_wave<uint32_t>(page, pm, vec_c, out, err, sel, rs, s);
+}
+
+template <typename T>
+static hipError_t dict_wave(int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, const void* dict, uint32_t dict_n,
+                            uint8_t* out, uint32_t* err, const SelArgs* sel, const HzlSrc* hz, hipStream_t s) {
+    const T*       d  = static_cast<const T*>(dict);
+    Tune           t  = tune_for(FAM_PAGE_DICT, 8 * sizeof(T), 255);
+    const unsigned bw = var == 1 ? 32u : pm.bw_max ? pm.bw_max : 1u;
+    const unsigned wl = (bw + 1) * kRow + (var == 7 ? kLbRows : 0);
+    // a dictionary of up to 32 KiB goes to LDS: a block's waves fit beside it
+    const bool     in_lds = (uint64_t)dict_n * sizeof(T) <= 32768;
+    const unsigned dl     = in_lds ? (dict_n * (unsigned)sizeof(T) + 15) & ~15u : 0u;
+    unsigned       waves  = t.block / 64;
+    while (waves > 1 && dl + waves * wl > 65536) --waves;
+    t.block = (uint16_t)(64 * waves);
+    // every block fills its own copy, so few blocks that stride over many vectors, the same number each (65536 vectors of
+    // int32, 4096 keys: 256 blocks of 8 waves 76 us, 1024 80 us, a block per 8 vectors 84); without a copy no cap
+    // (60000 keys: 121 us, 1536 blocks 150)
+    if (!in_lds) t.max_blocks = 0;
+    unsigned blocks = grid_for(vec_c, t, 64);
+    if (t.max_blocks) {
+        const uint64_t steps = (vec_c + (uint64_t)blocks * waves - 1) / ((uint64_t)blocks * waves);
+        blocks               = (unsigned)((vec_c + steps * waves - 1) / (steps * waves));
+    }
+    const dim3    g(blocks), b(t.block);
+    const SelArgs sa = sel ? *sel : SelArgs {};
+    // without HZL exceptions every block decodes the chunks itself; otherwise the HZL kernels fill the global copy first
+    const bool   fused = in_lds && hz && !hz->exc;
+    const HzlSrc hs    = fused ? *hz : HzlSrc {};
+    if (hz && !fused) {
+        const hipError_t e = launch_hzl(8 * sizeof(T), hz->enc, hz->chunks, hz->n_chunks,
+                                        reinterpret_cast<uint8_t*>(const_cast<T*>(d)), hz->exc != 0, s);
+        if (e != hipSuccess) return e;
+    }
+#define L(V, NT, K, SL) \
+    hipLaunchKernelGGL((k_wave_dict<T, V, NT, K, SL>), g, b, dl + waves * wl, s, page, pm, vec_c, d, dict_n, out, err, sa, hs, dl, wl)
+#define LK(V, K)                    \
+    if (sel) L(V, false, K, true);  \
+    else if (t.nt & 1) L(V, true, K, false); \
+    else L(V, false, K, false);
+#define LV(V)        \
+    if (in_lds) {    \
+        LK(V, true)  \
+    } else {         \
+        LK(V, false) \
+    }
+    if (var == 1) {
+        LV(1)
+    } else if (var == 2) {
+        LV(2)
+    } else {
+        LV(7)
+    }
+#undef LV
+#undef LK
+#undef L
+    return hipGetLastError();
+}
+hipError_t page_dict_wave(unsigned W, int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, const void* dict,
+                          uint32_t dict_n, uint8_t* out, uint32_t* err, const SelArgs* sel, const HzlSrc* hz, hipStream_t s) {
+    return W == 64 ? dict_wave<uint64_t>(var, page, pm, vec_c, dict, dict_n, out, err, sel, hz, s)
+                   : dict_wave<uint32_t>(var, page, pm, vec_c, dict, dict_n, out, err, sel, hz, s);
 }
 
 }  // namespace fls

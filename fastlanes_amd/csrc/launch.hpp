@@ -83,6 +83,8 @@ hipError_t page_int64_wave(int mode, const uint8_t* page, const PageMeta& pm, ui
                            const SelArgs* sel, hipStream_t s);
 hipError_t page_rle_wave(unsigned W, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out, uint32_t* err,
                          const SelArgs* sel, const RunSrc* runs, hipStream_t s);  // W 32/64, positions of bit width <= 1
+hipError_t page_dict_wave(unsigned W, int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, const void* dict,
+                          uint32_t dict_n, uint8_t* out, uint32_t* err, const SelArgs* sel, const HzlSrc* hz, hipStream_t s);
 template <int W>
 hipError_t page_patch_w(int var, bool rsum, const void* dict, uint32_t dict_n, const uint8_t* page, const PageMeta& pm,
                         uint32_t vec_c, uint8_t* out, uint32_t* err, const SelArgs* sel, const uint8_t* exc,

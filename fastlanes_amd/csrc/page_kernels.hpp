@@ -1035,14 +1035,11 @@ __global__ __launch_bounds__(256) void k_drle_fused(const uint8_t* __restrict__ 
     if (bad) atomicOr(err, 2u);
 }
 
-// Dictionary pages, pipelined like k_page_int. IN_LDS: the decoded dictionary is first copied into LDS (after the
-// waves' staging areas) and the code gathers read LDS instead of L2; the host picks it when the dictionary fits.
-// DIRECT (64-bit values): no output staging, segments stored straight to HBM (as k_page_rle); LDS holds only the
-// dictionary.
-// FROM_HZL (with IN_LDS): every block decodes the dictionary's HZL chunks straight into LDS, so no separate
-// dictionary pass runs before the page (chunks without exceptions only).
-template <typename T, typename D, int VAR, bool NT, bool IN_LDS, bool SEL = false, bool DIRECT = false,
-          bool FROM_HZL = false>
+// Dictionary pages of 8/16-bit values (wider ones: k_wave.hip, which a lane of 8 or 16 codes made slower here: 18.5 us
+// against 15.5 for 20011 vectors of uint16, 43 against 36 for 65536 of uint8), pipelined like k_page_int. IN_LDS: every
+// block first copies the decoded dictionary into LDS (after the waves' staging areas), or (hz.chunks) decodes its HZL
+// chunks into it, and the code gathers read LDS instead of L2; the host picks it when the dictionary fits.
+template <typename T, typename D, int VAR, bool NT, bool IN_LDS, bool SEL = false>
 __global__ __launch_bounds__(kMaxBlock) void k_page_dict(const uint8_t* __restrict__ page, PageMeta pm, uint32_t vec_c,
                                                          const D* __restrict__ dict, uint32_t dict_n,
                                                          uint8_t* __restrict__ out, uint32_t* err, SelArgs sa,
@@ -1052,11 +1049,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_page_dict(const uint8_t* __restri
     constexpr unsigned VB = 1024 * sizeof(T);
     constexpr unsigned P  = VAR == 1 ? 0 : (VAR == 7 ? 3 : 2);
     using WS              = WaveStage<32, VB>;
-    constexpr unsigned SB = DIRECT ? 0u : WS::BYTES;  // staging bytes per wave
-    const D* dp           = dict;
+    const D* dp = dict;
     if constexpr (IN_LDS) {
-        D* ldict = reinterpret_cast<D*>(fls_lds + (blockDim.x / 64) * SB);
-        if constexpr (FROM_HZL) {
+        D* ldict = reinterpret_cast<D*>(fls_lds + (blockDim.x / 64) * WS::BYTES);
+        if (hz.chunks) {
             for (uint32_t c = 0; c < hz.n_chunks; ++c) {
                 const HzlChunk ch  = hz.chunks[c];
                 const uint8_t* in  = hz.enc + ch.src;
@@ -1072,8 +1068,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_page_dict(const uint8_t* __restri
     }
     const unsigned lane = threadIdx.x % 64, wave = threadIdx.x / 64, waves = blockDim.x / 64;
     const unsigned t = lane % 32, slot = lane / 32;
-    uint8_t*       wl = fls_lds + wave * SB;
-    const LdsSink  lsink {wl + slot * WS::PVB};
+    uint8_t*       wl = fls_lds + wave * WS::BYTES;
+    const LdsSink  sink {wl + slot * WS::PVB};
     const uint64_t N      = vec_c;
     const uint64_t stride = (uint64_t)gridDim.x * waves * WS::VPW;
     uint64_t       v0     = ((uint64_t)blockIdx.x * waves + wave) * WS::VPW;
@@ -1082,26 +1078,20 @@ __global__ __launch_bounds__(kMaxBlock) void k_page_dict(const uint8_t* __restri
     for (; v0 < N; v0 += stride) {
         const uint64_t v = v0 + slot;
         if (v < N) {
-            const uint8_t* pk   = page + pm.off[P] + m.ep;
-            auto           body = [&](const auto& sink) {
-                if constexpr (VAR == 1) {
-                    dict_vector<T, D, 32, false>(pk, 0, 0, t, dp, dict_n, sink, err);
-                } else {
-                    dispatch_bw<32>(m.bw, [&](auto BW) {
-                        dict_vector<T, D, BW, VAR == 7>(pk, m.base, m.lb, t, dp, dict_n, sink, err);
-                    });
-                }
-            };
-            if constexpr (DIRECT) body(GlobalSink<NT> {out + v * VB});
-            else body(lsink);
+            const uint8_t* pk = page + pm.off[P] + m.ep;
+            if constexpr (VAR == 1) {
+                dict_vector<T, D, 32, false>(pk, 0, 0, t, dp, dict_n, sink, err);
+            } else {
+                dispatch_bw<32>(m.bw, [&](auto BW) {
+                    dict_vector<T, D, BW, VAR == 7>(pk, m.base, m.lb, t, dp, dict_n, sink, err);
+                });
+            }
         }
         if (v + stride < N) m = code_meta<VAR>(page, pm, v + stride, t);
-        if constexpr (!DIRECT) {
-            wave_sync();
-            const uint64_t left = N - v0;
-            wave_out<T, 32, VB, NT, SEL>(wl, out, v0, left < WS::VPW ? (uint32_t)left : WS::VPW, lane, sa);
-            wave_sync();
-        }
+        wave_sync();
+        const uint64_t left = N - v0;
+        wave_out<T, 32, VB, NT, SEL>(wl, out, v0, left < WS::VPW ? (uint32_t)left : WS::VPW, lane, sa);
+        wave_sync();
     }
 }
 

@@ -661,6 +661,42 @@ def test_zipf_int32_dictionary(torch_cuda, oracle, eid):
     np.testing.assert_array_equal(fa.encode_from_memory(x, eid), enc)
 
 
+@pytest.mark.parametrize("n_keys", [1, 2, 33, 1023, 1024, 1025, 2049, 4096, 4097, 8192, 8193, 20000])
+@pytest.mark.parametrize("dtype", [np.uint16, np.uint32, np.int64])
+def test_dictionary_sizes(torch_cuda, oracle, dtype, n_keys):
+    """Dictionaries around the HZL chunk size (1024 and the raw tail) and the LDS limit (32 KiB of values), codes of
+    every bit width up to theirs, plain, FFOR and DELTA codes, blocks with one vector and with many; decode and select."""
+    torch = torch_cuda
+    W = np.dtype(dtype).itemsize * 8
+    g = np.random.default_rng(n_keys + W)
+    info = np.iinfo(dtype)
+    keys = np.unique(g.integers(info.min, info.max, 2 * n_keys, dtype=dtype, endpoint=True))
+    keys = g.permutation(keys)[:n_keys]
+    bits = max(1, int(keys.size - 1).bit_length())
+    rows = [g.integers(0, min(keys.size, 1 << b), 1024) for b in range(bits + 1)] + [np.arange(keys.size)]
+    code = np.concatenate(rows)
+    code = np.concatenate([code, np.full(-code.size % 1024, keys.size - 1), g.integers(0, keys.size, 5 * 1024)])
+    x = keys[code]
+    n_vec = x.size // 1024
+    c = x[x.size // 2]
+    for eid in (16, 17, 22):
+        enc = oracle.encode_column(x, eid)
+        want = oracle.decode_column(enc, dtype, x.size)
+        plan = fa.Plan(enc, dtype)
+        d_in = dev(torch, enc)
+        d_out = torch.full((x.nbytes + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+        d_bm = torch.zeros(16 * n_vec, dtype=torch.int64, device="cuda")
+        d_cnt = torch.zeros(n_vec, dtype=torch.int32, device="cuda")
+        print(f"dictionary {np.dtype(dtype).name} keys={keys.size} expr={eid}", flush=True)
+        plan.decode(d_in.data_ptr(), d_out.data_ptr(), x.nbytes)
+        plan.select(d_in.data_ptr(), ">", c, d_bm.data_ptr(), d_cnt.data_ptr())
+        plan.check()
+        np.testing.assert_array_equal(to_np(d_out, dtype, x.size), want, err_msg=f"expr {eid}")
+        assert bool((d_out[x.nbytes:] == 0x5A).all())
+        np.testing.assert_array_equal(d_bm.cpu().numpy().view(np.uint64), _bitmap_words(want > c), err_msg=f"expr {eid}")
+        np.testing.assert_array_equal(d_cnt.cpu().numpy(), (want > c).reshape(-1, 1024).sum(axis=1))
+
+
 def _bitmap_words(mask: np.ndarray) -> np.ndarray:
     """SelectionDS bitmap words of a boolean mask: per 1024 values, 16 uint64 words, bit i of word j = value 64j+i."""
     bits = np.packbits(mask.reshape(-1, 64), axis=1, bitorder="little")
