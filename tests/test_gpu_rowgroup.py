@@ -258,3 +258,22 @@ def test_rowgroup_dictionary_chunks(torch_cuda, oracle, dtype):
         d_out = torch.full((rg.total_bytes,), 0xA5, dtype=torch.uint8, device="cuda")
         rg.decode(d_enc.data_ptr(), d_out.data_ptr(), 0, fa.stream_ptr())
         verify(torch, rg, d_out, [w for _, w in cols], "dictionary chunks")
+
+
+@pytest.mark.parametrize("n_columns,n_vec", [(1, 1), (1, 5), (2, 63), (7, 30), (16, 130)])
+def test_rowgroup_few_tiles(torch_cuda, oracle, n_columns, n_vec):
+    """Row-groups too small for every wave to have a tile: tiles go down to 2 KiB and no block is launched without one."""
+    torch = torch_cuda
+    cols = []
+    for c in range(n_columns):
+        kind, eid = list(wl.ROWGROUP_EXPRS.items())[c % len(wl.ROWGROUP_EXPRS)]
+        cols.append((wl.rowgroup_column(kind, (8, 16, 32, 64)[(c // 2) % 4], max(1, n_vec - c) * 1024, 50 + c), eid))
+    rg, d_enc, want = build(torch, oracle, cols)
+    tiles, blocks, _, runs = rg.work_list()
+    waves = (runs.size - 1) // blocks
+    print(f"rowgroup few tiles: {n_columns} columns, {tiles.size} tiles, {blocks} blocks", flush=True)
+    assert runs[-1] == tiles.size and blocks == -(-tiles.size // waves)
+    d_out = torch.full((rg.total_bytes + 256,), 0x69, dtype=torch.uint8, device="cuda")
+    rg.decode(d_enc.data_ptr(), d_out.data_ptr(), 0, fa.stream_ptr())
+    verify(torch, rg, d_out, want, "few tiles")
+    assert bool((d_out[rg.total_bytes:] == 0x69).all())
