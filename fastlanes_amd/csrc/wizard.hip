@@ -59,6 +59,20 @@ __device__ __forceinline__ T wave_max(T v) {
     }
     return v;
 }
+// Smallest / largest u32 of a wave, in scalar registers, without the LDS crossbar (a shuffle reduction is six of its
+// accesses, and the sizer's waves share one).
+template <bool MAX>
+__device__ __forceinline__ uint32_t wave_extreme(uint32_t v) {
+    constexpr uint32_t none = MAX ? 0u : ~0u;
+    auto take = [&](uint32_t o) { v = MAX ? max(v, o) : min(v, o); };
+    take(__builtin_amdgcn_update_dpp(none, v, 0x111, 0xf, 0xf, false));  // row_shr:1
+    take(__builtin_amdgcn_update_dpp(none, v, 0x112, 0xf, 0xf, false));  // row_shr:2
+    take(__builtin_amdgcn_update_dpp(none, v, 0x114, 0xf, 0xf, false));  // row_shr:4
+    take(__builtin_amdgcn_update_dpp(none, v, 0x118, 0xf, 0xf, false));  // row_shr:8
+    take(__builtin_amdgcn_update_dpp(none, v, 0x142, 0xa, 0xf, false));  // row_bcast:15 into rows 1 and 3
+    take(__builtin_amdgcn_update_dpp(none, v, 0x143, 0xc, 0xf, false));  // row_bcast:31 into rows 2 and 3
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
     for (int s = 32; s >= 1; s >>= 1) v += __shfl_xor(v, s, 64);
     return v;
@@ -68,6 +82,14 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The lane number, opaque to the optimiser: what a step derives from it (addresses, exchange directions) is computed
+// there again instead of being kept in registers from one step to the next, through spills.
+__device__ __forceinline__ unsigned fresh_lane() {
+    unsigned lane = threadIdx.x % 64;
+    asm volatile("" : "+v"(lane));
+    return lane;
 }
 
 // Sorts the 1024 values of buf (the wave's LDS buffer) ascending with a bitonic network held in registers: lane l
@@ -80,7 +102,7 @@ __device__ __forceinline__ void ce_regs(uint64_t& a, uint64_t& b, bool desc) {
     a = x, b = y;
 }
 __device__ void wave_sort1024(uint64_t* buf) {
-    const unsigned lane = threadIdx.x % 64;
+    const unsigned lane = fresh_lane();
     uint64_t       v[16];
     wave_lds_sync();
 #pragma unroll
@@ -133,7 +155,7 @@ struct PatchPlan {
     uint64_t base;
 };
 __device__ PatchPlan patch_plan(const uint64_t* s, uint32_t bwu) {
-    const unsigned lane = threadIdx.x % 64, bw_hi = bwu < 1 ? 1 : bwu < 63 ? bwu : 63;
+    const unsigned lane = fresh_lane(), bw_hi = bwu < 1 ? 1 : bwu < 63 ? bwu : 63;
     uint64_t       key  = ~0ull;  // (size << 32) | (i << 8) | (63 - bw): the smallest key is the plan
     for (unsigned h = 0; h < 2; ++h) {
         const unsigned i = lane + 64 * h;
@@ -192,7 +214,7 @@ struct VecStats {
 };
 
 __device__ VecStats vector_stats(const uint64_t* __restrict__ x) {
-    const unsigned lane = threadIdx.x % 64;
+    const unsigned lane = fresh_lane();
     uint64_t       v[16];
     const v4u*     p = reinterpret_cast<const v4u*>(x + 16 * lane);
 #pragma unroll
@@ -316,16 +338,21 @@ __device__ uint32_t block_popcount_scan(const uint32_t* bitmap, uint32_t* base, 
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Exhaustive sizing: one 1024-thread block per row-group (grid-stride); per block a global hash table region.
-// Only the block's own threads touch its table, slots and first positions, so the barriers' workgroup-scope
-// ordering is all the phases need (a device-scope fence would write back and invalidate the XCD's whole L2).
+// Exhaustive sizing: one 1024-thread block per row-group (grid-stride). 256 row-groups of 65536 values (mixed families),
+// one per compute unit: 1678 us when every value went through a hash table in global memory and every extreme through
+// LDS shuffles, 1182 us now; of a row-group of mostly distinct values (the slowest) 260 us are the per-vector sorts and
+// patch plans (VALU and the LDS crossbar alike), 480 the four partition passes of lds_firsts (VALU: the probes; the old
+// table took 700, bound by its random 128-byte lines), 100 the codes' widths (180), 115 the run codes (145).
+// Where an LDS table cannot serve, each block has a global one. Only the block's own threads touch its table, slots and
+// first positions, so the barriers' workgroup-scope ordering is all the phases need (a device-scope fence would write back
+// and invalidate the XCD's whole L2).
 // ---------------------------------------------------------------------------------------------------------------
 // DELTA patches (delta_exp.hpp:56-131: RSUM, then PA_ANALYZE over the lane differences): the patch plan of one
 // vector's differences (the value minus its predecessor inside each 64-value lane, 0 at a lane start), sorted in the
 // wave's buffer sb, and its exceptions in transposed order with the LL chain's hop links, as for the values.
 __device__ PatchPlan delta_patch(const uint64_t* __restrict__ xv, uint64_t* sb, uint32_t bwdu, uint32_t& n,
                                  uint32_t& extra) {
-    const unsigned lane = threadIdx.x % 64;
+    const unsigned lane = fresh_lane();
     auto diff = [&](unsigned o) { return (o % 64) ? xv[o] - xv[o - 1] : 0ull; };
     wave_lds_sync();  // the previous plan has read the sort buffer
 #pragma unroll
@@ -355,6 +382,174 @@ __device__ PatchPlan delta_patch(const uint64_t* __restrict__ xv, uint64_t* sb, 
     return pd;
 }
 
+// The sizer's LDS table (over the sort buffers, which are idle by then). A slot holds 15 hash bits and the smallest
+// position of its value, so a value is compared through the row-group's own values only where 15 more bits of its hash
+// agree. The four positions that a thread takes at a time probe in step, so that their LDS
+// reads, exchanges and value loads are in flight together. All values at once or those of one of 4 hash partitions after
+// another; every position's partition and slot go to slot[]. Returns false when the table takes no more (the values of a
+// partition are too many); the block is at a barrier then.
+// (a table filled to 28000 of its 32768 slots made some probes hundreds of slots long: 2570 us for the slowest row-groups)
+constexpr unsigned kLt = 32768, kLtTake = 20000;
+constexpr unsigned kBatch = 4;
+static_assert(kLtTake + 1024 * kBatch < kLt / 4 * 3, "claims in flight when the count passes the limit: still short probes");
+__device__ __forceinline__ bool lds_firsts(const uint64_t* __restrict__ x, uint32_t* tab, uint32_t* claims, uint32_t* bitmap,
+                                           uint32_t* __restrict__ slot, uint32_t* __restrict__ fpos, unsigned parts) {
+    const unsigned t = threadIdx.x, lane = t % 64, stride = blockDim.x;
+    for (unsigned part = 0; part < parts; ++part) {
+        __syncthreads();
+        for (unsigned i = t; i < kLt / 4; i += stride) reinterpret_cast<v4u*>(tab)[i] = v4u {kNoPos, kNoPos, kNoPos, kNoPos};
+        if (t == 0) *claims = 0;
+        __syncthreads();
+        for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
+            if (*const_cast<volatile uint32_t*>(claims) > kLtTake) break;
+            uint64_t v[kBatch];
+            uint32_t h[kBatch], me[kBatch], todo = 0;  // slot and partition; what goes into the slot; positions to insert
+            bool     lead[kBatch];
+            uint32_t won = 0;
+#pragma unroll
+            for (unsigned k = 0; k < kBatch; ++k) v[k] = x[o0 + k * stride];
+            // a run of equal values at consecutive positions of the wave: only its first lane inserts (the others'
+            // positions are no first occurrences) and the others take its slot
+#pragma unroll
+            for (unsigned k = 0; k < kBatch; ++k) {
+                const uint64_t pv = __shfl_up(v[k], 1, 64);
+                const uint32_t m = mix64(v[k]), p = m >> 15 & 3;
+                lead[k]          = lane == 0 || pv != v[k];
+                h[k]             = (m & (kLt - 1)) | p << 16;
+                me[k]            = (m >> 17) << 16 | (o0 + k * stride);
+                todo |= (lead[k] && (parts == 1 || p == part)) ? 1u << k : 0u;
+            }
+            while (__any(todo != 0)) {
+                uint32_t cur[kBatch], same = 0;
+#pragma unroll
+                for (unsigned k = 0; k < kBatch; ++k) cur[k] = tab[h[k] & (kLt - 1)];
+#pragma unroll
+                for (unsigned k = 0; k < kBatch; ++k)
+                    if ((todo >> k & 1) && cur[k] == kNoPos) cur[k] = atomicCAS(&tab[h[k] & (kLt - 1)], kNoPos, me[k]);
+#pragma unroll
+                for (unsigned k = 0; k < kBatch; ++k) {
+                    const bool here = todo >> k & 1, claimed = here && cur[k] == kNoPos;
+                    won += claimed;
+                    todo &= claimed ? ~(1u << k) : ~0u;
+                    same |= here && (cur[k] ^ me[k]) < 65536 ? 1u << k : 0u;  // (an empty slot's top bit is set, me's is not)
+                }
+                if (__any(same != 0)) {
+                    uint64_t xv[kBatch];
+#pragma unroll
+                    for (unsigned k = 0; k < kBatch; ++k) xv[k] = x[same >> k & 1 ? cur[k] & 0xffff : o0 + k * stride];
+#pragma unroll
+                    for (unsigned k = 0; k < kBatch; ++k)
+                        if ((same >> k & 1) && xv[k] == v[k]) {
+                            if (me[k] < cur[k]) atomicMin(&tab[h[k] & (kLt - 1)], me[k]);
+                            todo &= ~(1u << k);
+                        }
+                }
+#pragma unroll
+                for (unsigned k = 0; k < kBatch; ++k)
+                    if (todo >> k & 1) h[k] = (h[k] & ~(kLt - 1)) | ((h[k] + 1) & (kLt - 1));
+            }
+            won = wave_sum(won);
+            if (lane == 0 && won) atomicAdd(claims, won);
+#pragma unroll
+            for (unsigned k = 0; k < kBatch; ++k) {
+                const uint64_t lm  = __ballot(lead[k]);  // lane 0 always leads
+                const unsigned src = 63u - (unsigned)__clzll((long long)(lm & ((2ull << lane) - 1)));
+                slot[o0 + k * stride] = (uint32_t)__shfl((int)h[k], (int)src, 64);  // (other partitions': not yet final)
+            }
+        }
+        __syncthreads();
+        if (*claims > kLtTake) return false;
+        for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
+            uint32_t sl[kBatch];
+#pragma unroll
+            for (unsigned k = 0; k < kBatch; ++k) sl[k] = slot[o0 + k * stride];
+#pragma unroll
+            for (unsigned k = 0; k < kBatch; ++k) {
+                const unsigned o = o0 + k * stride;
+                if (parts > 1 && sl[k] >> 16 != part) continue;
+                const uint32_t f = tab[sl[k] & (kLt - 1)] & 0xffff;
+                fpos[o]          = f;
+                if (f == o) atomicOr(&bitmap[o >> 5], 1u << (o & 31));
+            }
+        }
+    }
+    __syncthreads();
+    return true;
+}
+
+// The same over the block's global table.
+__device__ __forceinline__ void global_firsts(const uint64_t* __restrict__ x, uint32_t* first, uint32_t* bitmap, uint32_t* __restrict__ slot,
+                              uint32_t* __restrict__ fpos) {
+    const unsigned t = threadIdx.x, lane = t % 64, stride = blockDim.x;
+    // dictionary: insert every value, remember its slot. A thread takes kBatch positions at a time: their loads
+    // and first probes are issued together, so kBatch atomics are in flight per thread instead of one.
+    for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
+        uint64_t v[kBatch];
+        uint32_t h[kBatch], cur[kBatch], hs[kBatch];
+        bool     lead[kBatch], done[kBatch];
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) v[k] = x[o0 + k * stride];
+        // a run of equal values at consecutive positions of the wave: only its first lane inserts (the others'
+        // positions are no first occurrences) and the others take its slot -- many lanes exchanging or
+        // min-ing one slot would serialize on that address
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) {
+            const uint64_t pv = __shfl_up(v[k], 1, 64);
+            lead[k]           = lane == 0 || pv != v[k];
+            h[k]              = mix64(v[k]) & (kHt - 1);
+            hs[k]             = h[k];
+        }
+        // the home slots' contents, then the exchanges into the empty ones, then the value comparisons: the
+        // batch's loads and atomics of each step are in flight together
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) cur[k] = lead[k] ? l2_load(&first[h[k]]) : 0u;
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) {
+            done[k] = !lead[k];
+            if (!done[k] && cur[k] == kNoPos) {
+                cur[k]  = wg_cas(&first[h[k]], kNoPos, o0 + k * stride);
+                done[k] = cur[k] == kNoPos;
+            }
+        }
+        uint64_t xv[kBatch];
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) xv[k] = done[k] ? 0ull : x[cur[k]];
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) {
+            const unsigned o = o0 + k * stride;
+            if (done[k]) continue;
+            if (xv[k] == v[k]) {
+                if (o < cur[k]) wg_min(&first[h[k]], o);
+            } else {  // the home slot holds another value: probe on
+                hs[k] = ht_insert(first, x, kHt - 1, v[k], o, (h[k] + 1) & (kHt - 1),
+                                  l2_load(&first[(h[k] + 1) & (kHt - 1)]));
+            }
+        }
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) {
+            const uint64_t lm  = __ballot(lead[k]);  // lane 0 always leads
+            const unsigned src = 63u - (unsigned)__clzll((long long)(lm & ((2ull << lane) - 1)));
+            slot[o0 + k * stride] = (uint32_t)__shfl((int)hs[k], (int)src, 64);
+        }
+    }
+    __syncthreads();
+    for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
+        uint32_t sl[kBatch], f[kBatch];
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) sl[k] = slot[o0 + k * stride];
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k)
+            f[k] = l2_load(&first[sl[k]]);
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) {
+            const unsigned o = o0 + k * stride;
+            fpos[o]          = f[k];
+            if (f[k] == o) atomicOr(&bitmap[o >> 5], 1u << (o & 31));
+        }
+    }
+    __syncthreads();
+}
+
 struct SizerLds {
     uint32_t bitmap[kRG / 32];
     uint32_t base[kRG / 32];
@@ -370,7 +565,8 @@ struct SizerLds {
     unsigned long long pbase[kVPR], excmin[8], excmax[8];
     // DICT_RLE: the page's run codes in chunks of 1024 (its HZL chain)
     uint32_t rcmin[kVPR], rcmax[kVPR], runpref[kVPR + 1];
-    uint64_t sortbuf[16][1024];  // one vector per wave, sorted for the patch plan
+    uint32_t claims, rich;  // rich: distinct values of the first 16 vectors, each vector's counted by itself
+    alignas(16) uint64_t sortbuf[16][1024];  // one vector per wave, sorted for the patch plan; then lds_firsts' table
 };
 
 __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restrict__ values, uint64_t n_rg,
@@ -392,14 +588,27 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
             L.rcmin[t] = ~0u, L.rcmax[t] = 0;
         }
         if (t < 8) L.excmin[t] = kEmpty, L.excmax[t] = 0;
+        if (t == 0) L.rich = 0;
+        __syncthreads();
         // per-vector statistics and patch plans (wave w takes vectors w, w + 16, ...)
+#pragma unroll 1
         for (unsigned v = wave; v < kVPR; v += blockDim.x / 64) {
+            const unsigned lane = fresh_lane();
             const VecStats s = vector_stats(x + v * 1024);
+            __builtin_amdgcn_sched_barrier(0);
             uint64_t*      sb = L.sortbuf[wave];
 #pragma unroll
             for (unsigned i = 0; i < 16; ++i) sb[64 * i + lane] = x[v * 1024 + 64 * i + lane];
             wave_sort1024(sb);
+            __builtin_amdgcn_sched_barrier(0);
+            if (v < 16) {
+                uint32_t d = 0;
+                for (unsigned q = 0; q < 16; ++q) d += (64 * q + lane) == 0 || sb[64 * q + lane] != sb[64 * q + lane - 1];
+                d = wave_sum(d);
+                if (lane == 0) atomicAdd(&L.rich, d);
+            }
             const PatchPlan pp = patch_plan(sb, s.bwu);
+            __builtin_amdgcn_sched_barrier(0);
             // exceptions in transposed order (the order the encoder stores them) and the LL chain's hop entries:
             // a gap g between consecutive exceptions adds floor((g - 1) / hop) links, hop = 2^min(bw, 11)
             const unsigned hop = 1u << (pp.bw < 11 ? pp.bw : 11);
@@ -430,75 +639,20 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
             const PatchPlan pd = delta_patch(x + v * 1024, sb, s.bwdu, dn, dextra);
             if (lane == 0) L.dbw[v] = pd.bw, L.dexc[v] = dn, L.dchain[v] = dn + dextra;
         }
-        // dictionary: insert every value, remember its slot. A thread takes kBatch positions at a time: their loads
-        // and first probes are issued together, so kBatch atomics are in flight per thread instead of one.
-        constexpr unsigned kBatch = 4;
-        const unsigned     stride = blockDim.x;
-        for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
-            uint64_t v[kBatch];
-            uint32_t h[kBatch], cur[kBatch], hs[kBatch];
-            bool     lead[kBatch], done[kBatch];
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) v[k] = x[o0 + k * stride];
-            // a run of equal values at consecutive positions of the wave: only its first lane inserts (the others'
-            // positions are no first occurrences) and the others take its slot -- many lanes exchanging or
-            // min-ing one slot would serialize on that address
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) {
-                const uint64_t pv = __shfl_up(v[k], 1, 64);
-                lead[k]           = lane == 0 || pv != v[k];
-                h[k]              = mix64(v[k]) & (kHt - 1);
-                hs[k]             = h[k];
-            }
-            // the home slots' contents, then the exchanges into the empty ones, then the value comparisons: the
-            // batch's loads and atomics of each step are in flight together
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) cur[k] = lead[k] ? l2_load(&first[h[k]]) : 0u;
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) {
-                done[k] = !lead[k];
-                if (!done[k] && cur[k] == kNoPos) {
-                    cur[k]  = wg_cas(&first[h[k]], kNoPos, o0 + k * stride);
-                    done[k] = cur[k] == kNoPos;
-                }
-            }
-            uint64_t xv[kBatch];
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) xv[k] = done[k] ? 0ull : x[cur[k]];
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) {
-                const unsigned o = o0 + k * stride;
-                if (done[k]) continue;
-                if (xv[k] == v[k]) {
-                    if (o < cur[k]) wg_min(&first[h[k]], o);
-                } else {  // the home slot holds another value: probe on
-                    hs[k] = ht_insert(first, x, kHt - 1, v[k], o, (h[k] + 1) & (kHt - 1),
-                                      l2_load(&first[(h[k] + 1) & (kHt - 1)]));
-                }
-            }
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) {
-                const uint64_t lm  = __ballot(lead[k]);  // lane 0 always leads
-                const unsigned src = 63u - (unsigned)__clzll((long long)(lm & ((2ull << lane) - 1)));
-                slot[o0 + k * stride] = (uint32_t)__shfl((int)hs[k], (int)src, 64);
-            }
-        }
+        // dictionary: every position's first occurrence, over the LDS table (all values at once, or by hash partition when
+        // they are too many), or over the global one where a partition is too large for it (hashes that agree)
+        const unsigned stride = blockDim.x;
+        uint32_t*      tab    = reinterpret_cast<uint32_t*>(L.sortbuf);
         __syncthreads();
-        for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
-            uint32_t sl[kBatch], f[kBatch];
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) sl[k] = slot[o0 + k * stride];
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k)
-                f[k] = l2_load(&first[sl[k]]);
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) {
-                const unsigned o = o0 + k * stride;
-                fpos[o]          = f[k];
-                if (f[k] == o) atomicOr(&L.bitmap[o >> 5], 1u << (o & 31));
-            }
+        // (drawn evenly from 20000 values, the most that one table takes, a vector has 998 different ones)
+        bool           in_lds = L.rich < 16 * 998 && lds_firsts(x, tab, &L.claims, L.bitmap, slot, fpos, 1);
+        if (!in_lds) in_lds = lds_firsts(x, tab, &L.claims, L.bitmap, slot, fpos, 4);
+        if (!in_lds) {
+            __syncthreads();
+            for (unsigned i = t; i < kRG / 32; i += stride) L.bitmap[i] = 0;  // partitions before may have set some
+            __syncthreads();
+            global_firsts(x, first, L.bitmap, slot, fpos);
         }
-        __syncthreads();
         const uint32_t D = block_popcount_scan(L.bitmap, L.base, kRG / 32, L.tmp);
         // codes: per vector min/max and 32-segment delta min/max; dictionary chunk min/max
         for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
@@ -516,7 +670,8 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
             const uint32_t c  = rank_of(L.bitmap, L.base, f);
             const uint32_t cp = (o % 32) ? rank_of(L.bitmap, L.base, fpb[k]) : c;
             const uint32_t d  = c - cp;  // 0 at a segment start
-            const uint32_t cmn = wave_min(c), cmx = wave_max(c), dmn = wave_min(d), dmx = wave_max(d);
+            const uint32_t cmn = wave_extreme<false>(c), cmx = wave_extreme<true>(c);
+            const uint32_t dmn = wave_extreme<false>(d), dmx = wave_extreme<true>(d);
             if (lane == 0) {
                 const unsigned v = o >> 10;  // the whole wave lies in one vector
                 atomicMin(&L.cmin[v], cmn), atomicMax(&L.cmax[v], cmx);
@@ -545,10 +700,12 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
                 const uint64_t val = xv[o];
                 const bool     chg = o == 0 || val != xv[o - 1];
                 const uint64_t mr  = __ballot(chg);
-                if (chg) {
-                    const uint32_t c     = rank_of(L.bitmap, L.base, fpos[v * 1024 + o]);
-                    const uint32_t chunk = (nr + (uint32_t)__popcll(mr & ((1ull << lane) - 1))) >> 10;
-                    atomicMin(&L.rcmin[chunk], c), atomicMax(&L.rcmax[chunk], c);
+                const uint32_t c  = rank_of(L.bitmap, L.base, fpos[v * 1024 + o]);
+                const uint32_t ck = (nr + (uint32_t)__popcll(mr & ((1ull << lane) - 1))) >> 10;
+                // (a wave's run starts lie in one chunk or two)
+                for (uint32_t k = nr >> 10; mr && k <= (nr + (uint32_t)__popcll(mr) - 1) >> 10; ++k) {
+                    const uint32_t cmn = wave_extreme<false>(chg && ck == k ? c : ~0u), cmx = wave_extreme<true>(chg && ck == k ? c : 0u);
+                    if (lane == 0) atomicMin(&L.rcmin[k], cmn), atomicMax(&L.rcmax[k], cmx);
                 }
                 nr += (uint32_t)__popcll(mr);
                 const uint64_t ev = xv[orig_of(o)];
@@ -624,8 +781,8 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
                 sizes[r * kK + k] = s[k];
             }
         }
-        // reset the slots this row-group used (the next row-group of this block reuses the table)
-        for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
+        // reset the slots of the global table that this row-group used (the next row-group of this block reuses it)
+        for (unsigned o0 = t; !in_lds && o0 < kRG; o0 += kBatch * stride) {
             uint32_t sl[kBatch];
 #pragma unroll
             for (unsigned k = 0; k < kBatch; ++k) sl[k] = slot[o0 + k * stride];
@@ -750,7 +907,8 @@ __global__ __launch_bounds__(256) void k_wizard_features(const uint64_t* __restr
             const uint32_t c  = rank_of(L.bitmap, L.base, fp[j]);
             const uint32_t cp = (p % 32) ? rank_of(L.bitmap, L.base, L.tab[L.slot[p - 1]]) : c;
             const uint32_t d  = c - cp;
-            const uint32_t cmn = wave_min(c), cmx = wave_max(c), dmn = wave_min(d), dmx = wave_max(d);
+            const uint32_t cmn = wave_extreme<false>(c), cmx = wave_extreme<true>(c);
+            const uint32_t dmn = wave_extreme<false>(d), dmx = wave_extreme<true>(d);
             if (lane == 0) {
                 const unsigned v = p >> 10;
                 atomicMin(&L.cmin[v], cmn), atomicMax(&L.cmax[v], cmx);

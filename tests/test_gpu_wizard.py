@@ -176,3 +176,42 @@ def test_exhaustive_sizes_many_rowgroups_per_block(torch_cuda, wiz):
     sizes = d_s.cpu().numpy()
     for r, j in enumerate(order):
         np.testing.assert_array_equal(sizes[r], want[j], err_msg=f"row-group {r} ({rgs[j][0]})")
+
+
+def _mix64(z):
+    """The sizer's value hash (splitmix64's finalizer), low 32 bits."""
+    z = z.astype(np.uint64)
+    z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+    z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+    return (z ^ (z >> np.uint64(31))).astype(np.uint32)
+
+
+@pytest.mark.parametrize("order", ["shuffled", "sorted"])
+def test_sizes_over_dictionary_tables(torch_cuda, wiz, order):
+    """Row-groups that the sizer counts in one LDS table (up to 20000 distinct values), in four hash partitions, and in
+    the global table (most values in one partition); the second call uses every table again."""
+    torch = torch_cuda
+    g = np.random.default_rng(5)
+    n = 65536
+    pool = g.integers(-(1 << 62), 1 << 62, 8 * n, dtype=np.int64)
+    one = pool[(_mix64(pool.view(np.uint64)) >> 15 & 3) == 2]
+    assert one.size > n
+    rgs = []
+    for d in (1, 1000, 19000, 20000, 21000, 25000, 40000, n):
+        rgs.append(np.concatenate([pool[:d], pool[g.integers(0, d, n - d)]]))
+    rgs.append(one[:n])  # all distinct, one partition
+    rgs.append(np.concatenate([one[:30000], pool[:20000], one[:n - 50000]]))
+    rgs.append(np.repeat(pool[: n // 4], 4))
+    rgs = [np.sort(x) if order == "sorted" else g.permutation(x) for x in rgs]
+    rgs = rgs[::-1] + rgs
+    d_x = torch.from_numpy(np.concatenate(rgs)).cuda()
+    d_s = torch.zeros((len(rgs), len(wo.CANDIDATES)), dtype=torch.int64, device="cuda")
+    want = [wo.candidate_sizes(x).astype(np.int64) for x in rgs]
+    for rep in range(2):
+        print(f"wizard sizes over the tables, {order}, call {rep}", flush=True)
+        d_s.zero_()
+        wiz.exhaustive_sizes(d_x.data_ptr(), len(rgs), d_s.data_ptr())
+        torch.cuda.synchronize()
+        sizes = d_s.cpu().numpy()
+        for r in range(len(rgs)):
+            np.testing.assert_array_equal(sizes[r], want[r], err_msg=f"row-group {r}")
