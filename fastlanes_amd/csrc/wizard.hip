@@ -78,19 +78,26 @@ __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
     return v;
 }
 
+// A value that all lanes of the wave hold, in a scalar register.
+__device__ __forceinline__ uint32_t wave_uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ uint64_t wave_uniform(uint64_t v) {
+    return (uint64_t)wave_uniform((uint32_t)(v >> 32)) << 32 | wave_uniform((uint32_t)v);
+}
+
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The lane number, opaque to the optimiser: what a step derives from it (addresses, exchange directions) is computed
+// The thread and lane number, opaque to the optimiser: what a step derives from it (addresses, exchange directions) is computed
 // there again instead of being kept in registers from one step to the next, through spills.
-__device__ __forceinline__ unsigned fresh_lane() {
-    unsigned lane = threadIdx.x % 64;
-    asm volatile("" : "+v"(lane));
-    return lane;
+__device__ __forceinline__ unsigned fresh_thread() {
+    unsigned t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
 }
+__device__ __forceinline__ unsigned fresh_lane() { return fresh_thread() % 64; }
 
 // Sorts the 1024 values of buf (the wave's LDS buffer) ascending with a bitonic network held in registers: lane l
 // keeps elements 16l .. 16l+15, so the stages over distances 1-8 (34 of 55) are compare-exchanges inside a lane and
@@ -186,12 +193,12 @@ __device__ PatchPlan patch_plan(const uint64_t* s, uint32_t bwu) {
             key = kk < key ? kk : key;
         }
     }
-    key = wave_min(key);
+    key = wave_uniform(wave_min(key));
     PatchPlan pp {64, 0, 0};
     if ((key >> 32) < 128ull * 64) {
         const unsigned i = (unsigned)(key >> 8) & 0xffffff;
         pp.bw   = 63 - (uint32_t)(key & 0xff);
-        pp.base = s[i];
+        pp.base = wave_uniform(s[i]);
         pp.exc  = (uint32_t)(((key >> 32) - 128ull * pp.bw) / 8);
     }
     return pp;
@@ -251,11 +258,11 @@ __device__ VecStats vector_stats(const uint64_t* __restrict__ x) {
     VecStats s;
     s.umin = wave_min(mn), s.umax = wave_max(mx);
     s.smin = wave_min(smn), s.smax = wave_max(smx);
-    s.bwf  = bitlen64((uint64_t)s.smax - (uint64_t)s.smin);
-    s.bwu  = bitlen64(s.umax - s.umin);
-    s.bwd  = bitlen64((uint64_t)wave_max(dmx) - (uint64_t)wave_min(dmn));
-    s.bwdu = bitlen64(wave_max(dux) - wave_min(dun));
-    s.runs = wave_sum(runs), s.bwp = wave_sum(inner) != 0;
+    s.bwf  = wave_uniform(bitlen64((uint64_t)s.smax - (uint64_t)s.smin));
+    s.bwu  = wave_uniform(bitlen64(s.umax - s.umin));
+    s.bwd  = wave_uniform(bitlen64((uint64_t)wave_max(dmx) - (uint64_t)wave_min(dmn)));
+    s.bwdu = wave_uniform(bitlen64(wave_max(dux) - wave_min(dun)));
+    s.runs = wave_uniform(wave_sum(runs)), s.bwp = wave_uniform((uint32_t)(wave_sum(inner) != 0));
     s.eq = wave_sum(eq), s.nondec = wave_sum(nondec), s.inc = wave_sum(inc);
     return s;
 }
@@ -339,10 +346,11 @@ __device__ uint32_t block_popcount_scan(const uint32_t* bitmap, uint32_t* base, 
 
 // ---------------------------------------------------------------------------------------------------------------
 // Exhaustive sizing: one 1024-thread block per row-group (grid-stride). 256 row-groups of 65536 values (mixed families),
-// one per compute unit: 1678 us when every value went through a hash table in global memory and every extreme through
-// LDS shuffles, 1182 us now; of a row-group of mostly distinct values (the slowest) 260 us are the per-vector sorts and
-// patch plans (VALU and the LDS crossbar alike), 480 the four partition passes of lds_firsts (VALU: the probes; the old
-// table took 700, bound by its random 128-byte lines), 100 the codes' widths (180), 115 the run codes (145).
+// one per compute unit: 1663 us when every value went through a hash table in global memory and every extreme through
+// LDS shuffles, 1139 us now; of a row-group of mostly distinct values (the slowest) 230 us are the per-vector sorts and
+// patch plans (VALU and the LDS crossbar alike; 280 with 80 registers spilled), 490 the four partition passes of
+// lds_firsts (VALU: the probes; the old table took 700, bound by its random 128-byte lines), 100 the codes' widths (155),
+// 115 the run codes (145). 8192 row-groups: 42.4 and 28.9 ms (before the spills were out).
 // Where an LDS table cannot serve, each block has a global one. Only the block's own threads touch its table, slots and
 // first positions, so the barriers' workgroup-scope ordering is all the phases need (a device-scope fence would write back
 // and invalidate the XCD's whole L2).
@@ -394,10 +402,12 @@ constexpr unsigned kBatch = 4;
 static_assert(kLtTake + 1024 * kBatch < kLt / 4 * 3, "claims in flight when the count passes the limit: still short probes");
 __device__ __forceinline__ bool lds_firsts(const uint64_t* __restrict__ x, uint32_t* tab, uint32_t* claims, uint32_t* bitmap,
                                            uint32_t* __restrict__ slot, uint32_t* __restrict__ fpos, unsigned parts) {
-    const unsigned t = threadIdx.x, lane = t % 64, stride = blockDim.x;
+    const unsigned t = fresh_thread(), lane = t % 64, stride = blockDim.x;
     for (unsigned part = 0; part < parts; ++part) {
         __syncthreads();
-        for (unsigned i = t; i < kLt / 4; i += stride) reinterpret_cast<v4u*>(tab)[i] = v4u {kNoPos, kNoPos, kNoPos, kNoPos};
+        uint32_t none = kNoPos;
+        asm volatile("" : "+v"(none));  // (four registers kept for it through the kernel otherwise)
+        for (unsigned i = t; i < kLt / 4; i += stride) reinterpret_cast<v4u*>(tab)[i] = v4u {none, none, none, none};
         if (t == 0) *claims = 0;
         __syncthreads();
         for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
@@ -480,7 +490,7 @@ __device__ __forceinline__ bool lds_firsts(const uint64_t* __restrict__ x, uint3
 // The same over the block's global table.
 __device__ __forceinline__ void global_firsts(const uint64_t* __restrict__ x, uint32_t* first, uint32_t* bitmap, uint32_t* __restrict__ slot,
                               uint32_t* __restrict__ fpos) {
-    const unsigned t = threadIdx.x, lane = t % 64, stride = blockDim.x;
+    const unsigned t = fresh_thread(), lane = t % 64, stride = blockDim.x;
     // dictionary: insert every value, remember its slot. A thread takes kBatch positions at a time: their loads
     // and first probes are issued together, so kBatch atomics are in flight per thread instead of one.
     for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
@@ -575,12 +585,12 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
     // dynamic LDS (the launch passes sizeof(SizerLds), about 150 KB)
     extern __shared__ __attribute__((aligned(16))) uint8_t wiz_lds[];
     SizerLds&      L = *reinterpret_cast<SizerLds*>(wiz_lds);
-    const unsigned t = threadIdx.x, lane = t % 64, wave = t / 64;
     uint32_t* first  = firsts_all + (uint64_t)blockIdx.x * (2 * kHt + 64);  // the table: first position per slot
     uint32_t* fpos   = first + kHt + 32;                                   // first occurrence per position (kRG)
     uint32_t* slot   = slots_all + (uint64_t)blockIdx.x * kRG;
     for (uint64_t r = blockIdx.x; r < n_rg; r += gridDim.x) {
         const uint64_t* x = values + r * kRG;
+        const unsigned  t = fresh_thread(), wave = wave_uniform(t / 64);
         for (unsigned i = t; i < kRG / 32; i += blockDim.x) L.bitmap[i] = 0;
         if (t < kVPR) {
             L.cmin[t] = ~0u, L.cmax[t] = 0, L.cdmin[t] = ~0u, L.cdmax[t] = 0;
@@ -595,6 +605,7 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
         for (unsigned v = wave; v < kVPR; v += blockDim.x / 64) {
             const unsigned lane = fresh_lane();
             const VecStats s = vector_stats(x + v * 1024);
+            if (lane == 0) L.bwf[v] = s.bwf, L.bwd[v] = s.bwd, L.runs[v] = s.runs, L.bwp[v] = s.bwp;
             __builtin_amdgcn_sched_barrier(0);
             uint64_t*      sb = L.sortbuf[wave];
 #pragma unroll
@@ -632,7 +643,6 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
             }
             extra = wave_sum(extra);
             if (lane == 0) {
-                L.bwf[v] = s.bwf, L.bwd[v] = s.bwd, L.runs[v] = s.runs, L.bwp[v] = s.bwp;
                 L.pbw[v] = pp.bw, L.pbase[v] = pp.base, L.pexc[v] = n, L.pchain[v] = n + extra;
             }
             uint32_t dn = 0, dextra = 0;
@@ -655,7 +665,8 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
         }
         const uint32_t D = block_popcount_scan(L.bitmap, L.base, kRG / 32, L.tmp);
         // codes: per vector min/max and 32-segment delta min/max; dictionary chunk min/max
-        for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
+        for (unsigned o0 = fresh_thread(); o0 < kRG; o0 += kBatch * stride) {
+          const unsigned lane = o0 % 64;
           uint32_t fb[kBatch], fpb[kBatch];
 #pragma unroll
           for (unsigned k = 0; k < kBatch; ++k) {
@@ -692,6 +703,7 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
         __syncthreads();
         // DICT_RLE run codes and S_PATCH_REC exception values, each as the page's chain in chunks of 1024
         for (unsigned v = wave; v < kVPR; v += blockDim.x / 64) {
+            const unsigned  lane = fresh_lane();
             const uint64_t* xv = x + v * 1024;
             PatchPlan       pp {L.pbw[v], 0, L.pbase[v]};
             uint32_t        nr = L.runpref[v], ne = L.excpref[v];
@@ -782,7 +794,7 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
             }
         }
         // reset the slots of the global table that this row-group used (the next row-group of this block reuses it)
-        for (unsigned o0 = t; !in_lds && o0 < kRG; o0 += kBatch * stride) {
+        for (unsigned o0 = fresh_thread(); !in_lds && o0 < kRG; o0 += kBatch * stride) {
             uint32_t sl[kBatch];
 #pragma unroll
             for (unsigned k = 0; k < kBatch; ++k) sl[k] = slot[o0 + k * stride];
