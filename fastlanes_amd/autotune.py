@@ -2,7 +2,7 @@
 
 For every kernel family (raw streams per element width and bit width; UNCOMPRESSED / FFOR / DELTA / RLE /
 dictionary pages per element width) it times candidate launch shapes -- threads per block, non-temporal stores,
-a cap on the grid (persistent blocks), direct stores for wide values, and for narrow RLE pages the vectors per
+a cap on the grid (persistent blocks), direct stores for 32-bit values, and for narrow RLE pages the vectors per
 wavefront (one vector with one position lane per thread, or two with two) -- on the GPU and writes the fastest into a
 tuning table (`fastlanes_amd/tuning.txt` by default) that the library loads on first use. The row-group launch (family 6) is
 tuned on the mixed 64-column row-group: KiB of decoded values per tile and blocks per compute unit. Entries of
@@ -56,8 +56,7 @@ def _candidates(n_cu, nts=NTS):
 def tune_family(lib, family, W, bw, fn, stream, n_cu, bytes_moved):
     best = None
     # integer pages of 32/64-bit values may also write without LDS staging (bit 1 of the store flags)
-    nts = NTS + (2, 3) if (family in (FAM_UNC, FAM_FFOR, FAM_DELTA) and W >= 32) or \
-        (family in (FAM_RLE, FAM_DICT) and W == 64) else NTS
+    nts = NTS + (2, 3) if family in (FAM_UNC, FAM_FFOR, FAM_DELTA) and W == 32 else NTS
     # RLE pages of 8/16-bit values: one vector per wave with one position lane per thread, or (bit 2) two vectors per
     # wave with two lanes per thread and LDS staging -- the vectors-per-wavefront choice of this family
     if family == FAM_RLE and W <= 16:

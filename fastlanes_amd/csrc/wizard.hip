@@ -350,7 +350,7 @@ __device__ uint32_t block_popcount_scan(const uint32_t* bitmap, uint32_t* base, 
 // LDS shuffles, 1139 us now; of a row-group of mostly distinct values (the slowest) 230 us are the per-vector sorts and
 // patch plans (VALU and the LDS crossbar alike; 280 with 80 registers spilled), 490 the four partition passes of
 // lds_firsts (VALU: the probes; the old table took 700, bound by its random 128-byte lines), 100 the codes' widths (155),
-// 115 the run codes (145). 8192 row-groups: 42.4 and 28.9 ms (before the spills were out).
+// 115 the run codes (145). 8192 row-groups: 42.4 and 27.8 ms.
 // Where an LDS table cannot serve, each block has a global one. Only the block's own threads touch its table, slots and
 // first positions, so the barriers' workgroup-scope ordering is all the phases need (a device-scope fence would write back
 // and invalidate the XCD's whole L2).
