@@ -55,7 +55,7 @@ def _candidates(n_cu, nts=NTS):
 
 def tune_family(lib, family, W, bw, fn, stream, n_cu, bytes_moved):
     best = None
-    # integer pages of 32/64-bit values may also write without LDS staging (bit 1 of the store flags)
+    # integer pages of 32-bit values may also write without LDS staging (bit 1 of the store flags)
     nts = NTS + (2, 3) if family in (FAM_UNC, FAM_FFOR, FAM_DELTA) and W == 32 else NTS
     # RLE pages of 8/16-bit values: one vector per wave with one position lane per thread, or (bit 2) two vectors per
     # wave with two lanes per thread and LDS staging -- the vectors-per-wavefront choice of this family

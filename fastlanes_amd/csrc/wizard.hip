@@ -99,6 +99,10 @@ __device__ __forceinline__ unsigned fresh_thread() {
 }
 __device__ __forceinline__ unsigned fresh_lane() { return fresh_thread() % 64; }
 
+// A sorted buffer's place of element i: the elements that the lanes hold of one register are 128 bytes apart, which as it
+// stands is one pair of LDS banks for all of them.
+__device__ __forceinline__ unsigned sorted_at(unsigned i) { return i ^ ((i >> 4) & 15); }
+
 // Sorts the 1024 values of buf (the wave's LDS buffer) ascending with a bitonic network held in registers: lane l
 // keeps elements 16l .. 16l+15, so the stages over distances 1-8 (34 of 55) are compare-exchanges inside a lane and
 // the stages over distances 16-512 exchange with lane l ^ (distance / 16) through shuffles; LDS is read once and
@@ -139,7 +143,66 @@ __device__ void wave_sort1024(uint64_t* buf) {
         }
     }
 #pragma unroll
-    for (unsigned r = 0; r < 16; ++r) buf[16 * lane + r] = v[r];
+    for (unsigned r = 0; r < 16; ++r) buf[sorted_at(16 * lane + r)] = v[r];
+    wave_lds_sync();
+}
+
+// The same where the values' signed range is below 2^32 (1024 values: 22 us with 16 waves a compute unit, 8 here): their
+// 32-bit distances from the smallest are sorted (a
+// compare-exchange is two instructions, not six, and an exchange across lanes one cross-lane move; descending blocks are
+// sorted complemented), and written back in unsigned order: the negative values, which come first, last.
+__device__ __forceinline__ uint32_t xor_lane(uint32_t x, unsigned d) {
+    switch (d) {
+    case 1: return __builtin_amdgcn_update_dpp(0u, x, 0xb1, 0xf, 0xf, false);  // quad_perm 1 0 3 2
+    case 2: return __builtin_amdgcn_update_dpp(0u, x, 0x4e, 0xf, 0xf, false);  // quad_perm 2 3 0 1
+    case 4:                                                                    // half mirror (^ 7), quad_perm 3 2 1 0 (^ 3)
+        return __builtin_amdgcn_update_dpp(0u, __builtin_amdgcn_update_dpp(0u, x, 0x141, 0xf, 0xf, false), 0x1b, 0xf, 0xf, false);
+    case 8: return __builtin_amdgcn_update_dpp(0u, x, 0x128, 0xf, 0xf, false);  // row_ror:8
+    default: return (uint32_t)__shfl_xor((int)x, (int)d, 64);
+    }
+}
+__device__ void wave_sort1024_narrow(uint64_t* buf, uint64_t smallest) {
+    const unsigned lane = fresh_lane();
+    uint32_t       v[16], negative = 0;
+    wave_lds_sync();
+#pragma unroll
+    for (unsigned r = 0; r < 16; ++r) {
+        const uint64_t x = buf[64 * r + lane];
+        negative += (uint32_t)__popcll(__ballot((int64_t)x < 0));
+        v[r] = (uint32_t)(x - smallest);
+    }
+    wave_lds_sync();
+    uint32_t flipped = 0;
+#pragma unroll
+    for (unsigned k = 2; k <= 1024; k <<= 1) {
+        if (k >= 16) {
+            const uint32_t flip = k < 1024 && ((16 * lane) & k) ? ~0u : 0u;
+#pragma unroll
+            for (unsigned r = 0; r < 16; ++r) v[r] ^= flip ^ flipped;
+            flipped = flip;
+        }
+#pragma unroll
+        for (unsigned j = k >> 1; j > 0; j >>= 1) {
+            if (j >= 16) {
+                const bool low = (lane & (j / 16)) == 0;
+#pragma unroll
+                for (unsigned r = 0; r < 16; ++r) {
+                    const uint32_t p = xor_lane(v[r], j / 16);
+                    v[r]             = low ? min(v[r], p) : max(v[r], p);
+                }
+            } else {
+#pragma unroll
+                for (unsigned r = 0; r < 16; ++r) {
+                    if (r & j) continue;
+                    const uint32_t a = min(v[r], v[r | j]), b = max(v[r], v[r | j]);
+                    const bool     desc = k < 16 && (r & k) != 0;
+                    v[r] = desc ? b : a, v[r | j] = desc ? a : b;
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (unsigned r = 0; r < 16; ++r) buf[sorted_at((16 * lane + r - negative) & 1023)] = smallest + v[r];
     wave_lds_sync();
 }
 
@@ -154,7 +217,7 @@ __device__ __forceinline__ unsigned orig_of(unsigned k) {
 // plan_patch): over bit widths bw < 64 and window bases s[i] (first index of each distinct value among the 101
 // smallest), the window [s[i], s[i] + 2^bw - 1] (bw = 0: only base 0, window {0}) leaving at most 100 values
 // outside; the plan minimises 128 bw + 8 (values outside), ties to the smaller i, then the larger bw; it exists only
-// below 128 * 64 bytes (else bw = 64, base 0, no exceptions). s: the vector sorted ascending (LDS). A window wider
+// below 128 * 64 bytes (else bw = 64, base 0, no exceptions). s: the vector sorted ascending (LDS, element i at sorted_at(i)). A window wider
 // than the vector's unsigned FFOR width bwu is never better than bw = bwu at i = 0, so bw runs up to min(bwu, 63) --
 // and up to 1 for a constant nonzero vector, which no zero-width window holds.
 struct PatchPlan {
@@ -167,11 +230,13 @@ __device__ PatchPlan patch_plan(const uint64_t* s, uint32_t bwu) {
     for (unsigned h = 0; h < 2; ++h) {
         const unsigned i = lane + 64 * h;
         if (i > kExcLimit) continue;
-        const uint64_t si = s[i];
-        if (i && si == s[i - 1]) continue;
+        const uint64_t si = s[sorted_at(i)];
+        if (i && si == s[sorted_at(i - 1)]) continue;
         // the window must hold s[i .. 923 + i]: its width is at least bitlen(s[923 + i] - s[i])
-        const uint32_t bw_lo = bitlen64(s[1023 - kExcLimit + i] - si);
-        for (unsigned bw = bw_lo; bw <= bw_hi; ++bw) {
+        const uint32_t bw_lo = bitlen64(s[sorted_at(1023 - kExcLimit + i)] - si);
+        // from the first feasible width on (bw_lo, or 1) a wider window saves at most its 100 - i exceptions above it
+        const unsigned bw_end = min(bw_hi, bw_lo + 1 + 8 * (kExcLimit - i) / 128);
+        for (unsigned bw = bw_lo; bw <= bw_end; ++bw) {
             uint64_t upper;
             if (bw == 0) {
                 if (si != 0) continue;  // a zero-width window holds only zeros
@@ -184,7 +249,7 @@ __device__ PatchPlan patch_plan(const uint64_t* s, uint32_t bwu) {
             unsigned lo = 1023 - kExcLimit + i, hi = 1024;
             while (hi - lo > 1) {
                 const unsigned mid = (lo + hi) / 2;
-                if (s[mid] <= upper) lo = mid;
+                if (s[sorted_at(mid)] <= upper) lo = mid;
                 else hi = mid;
             }
             const uint32_t exc  = 1024 - (hi - i);
@@ -198,7 +263,7 @@ __device__ PatchPlan patch_plan(const uint64_t* s, uint32_t bwu) {
     if ((key >> 32) < 128ull * 64) {
         const unsigned i = (unsigned)(key >> 8) & 0xffffff;
         pp.bw   = 63 - (uint32_t)(key & 0xff);
-        pp.base = wave_uniform(s[i]);
+        pp.base = wave_uniform(s[sorted_at(i)]);
         pp.exc  = (uint32_t)(((key >> 32) - 128ull * pp.bw) / 8);
     }
     return pp;
@@ -217,7 +282,7 @@ __device__ __forceinline__ bool is_exception(uint64_t v, const PatchPlan& pp) {
 struct VecStats {
     uint32_t bwf, bwd, bwu, bwdu, runs, bwp, eq, nondec, inc;
     uint64_t umin, umax;
-    int64_t  smin, smax;
+    int64_t  smin, smax, dmin;
 };
 
 __device__ VecStats vector_stats(const uint64_t* __restrict__ x) {
@@ -260,7 +325,8 @@ __device__ VecStats vector_stats(const uint64_t* __restrict__ x) {
     s.smin = wave_min(smn), s.smax = wave_max(smx);
     s.bwf  = wave_uniform(bitlen64((uint64_t)s.smax - (uint64_t)s.smin));
     s.bwu  = wave_uniform(bitlen64(s.umax - s.umin));
-    s.bwd  = wave_uniform(bitlen64((uint64_t)wave_max(dmx) - (uint64_t)wave_min(dmn)));
+    s.smin = (int64_t)wave_uniform((uint64_t)s.smin), s.dmin = (int64_t)wave_uniform((uint64_t)wave_min(dmn));
+    s.bwd  = wave_uniform(bitlen64((uint64_t)wave_max(dmx) - (uint64_t)s.dmin));
     s.bwdu = wave_uniform(bitlen64(wave_max(dux) - wave_min(dun)));
     s.runs = wave_uniform(wave_sum(runs)), s.bwp = wave_uniform((uint32_t)(wave_sum(inner) != 0));
     s.eq = wave_sum(eq), s.nondec = wave_sum(nondec), s.inc = wave_sum(inc);
@@ -346,11 +412,11 @@ __device__ uint32_t block_popcount_scan(const uint32_t* bitmap, uint32_t* base, 
 
 // ---------------------------------------------------------------------------------------------------------------
 // Exhaustive sizing: one 1024-thread block per row-group (grid-stride). 256 row-groups of 65536 values (mixed families),
-// one per compute unit: 1663 us when every value went through a hash table in global memory and every extreme through
-// LDS shuffles, 1139 us now; of a row-group of mostly distinct values (the slowest) 230 us are the per-vector sorts and
-// patch plans (VALU and the LDS crossbar alike; 280 with 80 registers spilled), 490 the four partition passes of
-// lds_firsts (VALU: the probes; the old table took 700, bound by its random 128-byte lines), 100 the codes' widths (155),
-// 115 the run codes (145). 8192 row-groups: 42.4 and 27.8 ms.
+// one per compute unit: 1675 us when every value went through a hash table in global memory and every extreme through
+// LDS shuffles, 1055 us now. Of a row-group of mostly distinct values (the slowest), 115-240 us are the per-vector sorts and
+// patch plans (VALU; 280-490 before the narrow sort and the bound on a window's width), 490-580 the four partition passes
+// of lds_firsts (VALU: the probes; the old table took 700, bound by its random 128-byte lines), 100 the codes' widths (155),
+// 115 the run codes (145). 8192 row-groups: 42.4 and 23.7 ms; their sample statistics (k_wizard_features) 2.86 and 1.17 ms.
 // Where an LDS table cannot serve, each block has a global one. Only the block's own threads touch its table, slots and
 // first positions, so the barriers' workgroup-scope ordering is all the phases need (a device-scope fence would write back
 // and invalidate the XCD's whole L2).
@@ -358,15 +424,16 @@ __device__ uint32_t block_popcount_scan(const uint32_t* bitmap, uint32_t* base, 
 // DELTA patches (delta_exp.hpp:56-131: RSUM, then PA_ANALYZE over the lane differences): the patch plan of one
 // vector's differences (the value minus its predecessor inside each 64-value lane, 0 at a lane start), sorted in the
 // wave's buffer sb, and its exceptions in transposed order with the LL chain's hop links, as for the values.
-__device__ PatchPlan delta_patch(const uint64_t* __restrict__ xv, uint64_t* sb, uint32_t bwdu, uint32_t& n,
+__device__ PatchPlan delta_patch(const uint64_t* __restrict__ xv, uint64_t* sb, const VecStats& s, uint32_t& n,
                                  uint32_t& extra) {
     const unsigned lane = fresh_lane();
     auto diff = [&](unsigned o) { return (o % 64) ? xv[o] - xv[o - 1] : 0ull; };
     wave_lds_sync();  // the previous plan has read the sort buffer
 #pragma unroll
     for (unsigned i = 0; i < 16; ++i) sb[64 * i + lane] = diff(64 * i + lane);
-    wave_sort1024(sb);
-    const PatchPlan pd  = patch_plan(sb, bwdu);
+    if (s.bwd <= 32) wave_sort1024_narrow(sb, (uint64_t)s.dmin);
+    else wave_sort1024(sb);
+    const PatchPlan pd  = patch_plan(sb, s.bwdu);
     const unsigned  hop = 1u << (pd.bw < 11 ? pd.bw : 11);
     int             last = -1;
     n = 0, extra = 0;
@@ -610,11 +677,12 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
             uint64_t*      sb = L.sortbuf[wave];
 #pragma unroll
             for (unsigned i = 0; i < 16; ++i) sb[64 * i + lane] = x[v * 1024 + 64 * i + lane];
-            wave_sort1024(sb);
+            if (s.bwf <= 32) wave_sort1024_narrow(sb, (uint64_t)s.smin);
+            else wave_sort1024(sb);
             __builtin_amdgcn_sched_barrier(0);
             if (v < 16) {
                 uint32_t d = 0;
-                for (unsigned q = 0; q < 16; ++q) d += (64 * q + lane) == 0 || sb[64 * q + lane] != sb[64 * q + lane - 1];
+                for (unsigned q = 0; q < 16; ++q) d += (64 * q + lane) == 0 || sb[sorted_at(64 * q + lane)] != sb[sorted_at(64 * q + lane - 1)];
                 d = wave_sum(d);
                 if (lane == 0) atomicAdd(&L.rich, d);
             }
@@ -646,7 +714,7 @@ __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restric
                 L.pbw[v] = pp.bw, L.pbase[v] = pp.base, L.pexc[v] = n, L.pchain[v] = n + extra;
             }
             uint32_t dn = 0, dextra = 0;
-            const PatchPlan pd = delta_patch(x + v * 1024, sb, s.bwdu, dn, dextra);
+            const PatchPlan pd = delta_patch(x + v * 1024, sb, s, dn, dextra);
             if (lane == 0) L.dbw[v] = pd.bw, L.dexc[v] = dn, L.dchain[v] = dn + dextra;
         }
         // dictionary: every position's first occurrence, over the LDS table (all values at once, or by hash partition when
@@ -878,10 +946,11 @@ __global__ __launch_bounds__(256) void k_wizard_features(const uint64_t* __restr
             uint64_t*      sb = L.u.sortbuf[wave];
 #pragma unroll
             for (unsigned i = 0; i < 16; ++i) sb[64 * i + lane] = x[kSampleVec[wave] * 1024 + 64 * i + lane];
-            wave_sort1024(sb);
+            if (s.bwf <= 32) wave_sort1024_narrow(sb, (uint64_t)s.smin);
+            else wave_sort1024(sb);
             const PatchPlan pp = patch_plan(sb, s.bwu);
             uint32_t        dn = 0, dextra = 0;
-            const PatchPlan pd = delta_patch(x + kSampleVec[wave] * 1024, sb, s.bwdu, dn, dextra);
+            const PatchPlan pd = delta_patch(x + kSampleVec[wave] * 1024, sb, s, dn, dextra);
             if (lane == 0) {
                 L.pbw[wave] = pp.bw, L.pexc[wave] = pp.exc;
                 L.dpbw[wave] = pd.bw, L.dpexc[wave] = dn;
