@@ -411,13 +411,14 @@ __device__ uint32_t block_popcount_scan(const uint32_t* bitmap, uint32_t* base, 
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// Exhaustive sizing: one 1024-thread block per row-group (grid-stride). 256 row-groups of 65536 values (mixed families),
-// one per compute unit: 1675 us when every value went through a hash table in global memory and every extreme through
-// LDS shuffles, 1055 us now. Of a row-group of mostly distinct values (the slowest), 115-240 us are the per-vector sorts and
-// patch plans (VALU; 280-490 before the narrow sort and the bound on a window's width), 490-580 the four partition passes
-// of lds_firsts (VALU: the probes; the old table took 700, bound by its random 128-byte lines), 100 the codes' widths (155),
-// 115 the run codes (145). 8192 row-groups: 42.4 and 23.7 ms; their sample statistics (k_wizard_features) 2.86 and 1.17 ms.
-// Where an LDS table cannot serve, each block has a global one. Only the block's own threads touch its table, slots and
+// Exhaustive sizing: one 1024-thread block per row-group (grid-stride), or three launches for a few (below). 256 row-groups
+// of 65536 values (mixed families), one per compute unit: 1675 us when every value went through a hash table in global
+// memory and every extreme through LDS shuffles, 1055 us now. Of a row-group of mostly distinct values (the slowest),
+// 115-240 us are the per-vector sorts and patch plans (VALU; 280-490 before the narrow sort and the bound on a window's
+// width), 490-580 the four partition passes of lds_firsts (VALU: the probes; the old table took 700, bound by its random
+// 128-byte lines), 100 the codes' widths (155), 115 the run codes (145). 8192 row-groups: 42.4 and 23.7 ms; their sample
+// statistics (k_wizard_features) 2.86 and 1.17 ms.
+// Where an LDS table cannot serve, each row-group has a global one. Only the block's own threads touch its table, slots and
 // first positions, so the barriers' workgroup-scope ordering is all the phases need (a device-scope fence would write back
 // and invalidate the XCD's whole L2).
 // ---------------------------------------------------------------------------------------------------------------
@@ -460,24 +461,28 @@ __device__ PatchPlan delta_patch(const uint64_t* __restrict__ xv, uint64_t* sb, 
 // The sizer's LDS table (over the sort buffers, which are idle by then). A slot holds 15 hash bits and the smallest
 // position of its value, so a value is compared through the row-group's own values only where 15 more bits of its hash
 // agree. The four positions that a thread takes at a time probe in step, so that their LDS
-// reads, exchanges and value loads are in flight together. All values at once or those of one of 4 hash partitions after
-// another; every position's partition and slot go to slot[]. Returns false when the table takes no more (the values of a
-// partition are too many); the block is at a barrier then.
+// reads, exchanges and value loads are in flight together. All values at once (parts 1) or those of the hash partitions
+// [part, end) of 4, one after another; only their places of fpos[] are
+// written, and of slot[] (scratch; ALONE: no other block shares it, and whole lines are written). Returns false when the
+// table takes no more (the values of a partition are too many); the block is at a barrier then.
 // (a table filled to 28000 of its 32768 slots made some probes hundreds of slots long: 2570 us for the slowest row-groups)
 constexpr unsigned kLt = 32768, kLtTake = 20000;
 constexpr unsigned kBatch = 4;
 static_assert(kLtTake + 1024 * kBatch < kLt / 4 * 3, "claims in flight when the count passes the limit: still short probes");
-__device__ __forceinline__ bool lds_firsts(const uint64_t* __restrict__ x, uint32_t* tab, uint32_t* claims, uint32_t* bitmap,
-                                           uint32_t* __restrict__ slot, uint32_t* __restrict__ fpos, unsigned parts) {
+template <bool ALONE>
+__device__ __forceinline__ bool lds_firsts(const uint64_t* __restrict__ x, uint32_t* tab, uint32_t* claims,
+                                           uint32_t* __restrict__ slot, uint32_t* __restrict__ fpos, unsigned part, unsigned end,
+                                           unsigned parts) {
     const unsigned t = fresh_thread(), lane = t % 64, stride = blockDim.x;
-    for (unsigned part = 0; part < parts; ++part) {
+    for (; part < end; ++part) {
         __syncthreads();
         uint32_t none = kNoPos;
         asm volatile("" : "+v"(none));  // (four registers kept for it through the kernel otherwise)
         for (unsigned i = t; i < kLt / 4; i += stride) reinterpret_cast<v4u*>(tab)[i] = v4u {none, none, none, none};
         if (t == 0) *claims = 0;
         __syncthreads();
-        for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
+        uint64_t mine = 0;  // the thread's positions of this partition (bit o / blockDim.x)
+        for (unsigned o0 = t, n = 0; o0 < kRG; o0 += kBatch * stride, n += kBatch) {
             if (*const_cast<volatile uint32_t*>(claims) > kLtTake) break;
             uint64_t v[kBatch];
             uint32_t h[kBatch], me[kBatch], todo = 0;  // slot and partition; what goes into the slot; positions to insert
@@ -531,23 +536,21 @@ __device__ __forceinline__ bool lds_firsts(const uint64_t* __restrict__ x, uint3
             for (unsigned k = 0; k < kBatch; ++k) {
                 const uint64_t lm  = __ballot(lead[k]);  // lane 0 always leads
                 const unsigned src = 63u - (unsigned)__clzll((long long)(lm & ((2ull << lane) - 1)));
-                slot[o0 + k * stride] = (uint32_t)__shfl((int)h[k], (int)src, 64);  // (other partitions': not yet final)
+                const uint32_t hs  = (uint32_t)__shfl((int)h[k], (int)src, 64);
+                const bool own = parts == 1 || hs >> 16 == part;
+                mine |= own ? 1ull << (n + k) : 0ull;
+                if (ALONE || own) slot[o0 + k * stride] = hs & (kLt - 1);
             }
         }
         __syncthreads();
         if (*claims > kLtTake) return false;
-        for (unsigned o0 = t; o0 < kRG; o0 += kBatch * stride) {
+        for (unsigned o0 = t, n = 0; o0 < kRG; o0 += kBatch * stride, n += kBatch) {
             uint32_t sl[kBatch];
 #pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) sl[k] = slot[o0 + k * stride];
+            for (unsigned k = 0; k < kBatch; ++k) sl[k] = mine >> (n + k) & 1 ? slot[o0 + k * stride] : 0u;
 #pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) {
-                const unsigned o = o0 + k * stride;
-                if (parts > 1 && sl[k] >> 16 != part) continue;
-                const uint32_t f = tab[sl[k] & (kLt - 1)] & 0xffff;
-                fpos[o]          = f;
-                if (f == o) atomicOr(&bitmap[o >> 5], 1u << (o & 31));
-            }
+            for (unsigned k = 0; k < kBatch; ++k)
+                if (mine >> (n + k) & 1) fpos[o0 + k * stride] = tab[sl[k]] & 0xffff;
         }
     }
     __syncthreads();
@@ -555,8 +558,8 @@ __device__ __forceinline__ bool lds_firsts(const uint64_t* __restrict__ x, uint3
 }
 
 // The same over the block's global table.
-__device__ __forceinline__ void global_firsts(const uint64_t* __restrict__ x, uint32_t* first, uint32_t* bitmap, uint32_t* __restrict__ slot,
-                              uint32_t* __restrict__ fpos) {
+__device__ __forceinline__ void global_firsts(const uint64_t* __restrict__ x, uint32_t* first, uint32_t* __restrict__ slot,
+                                              uint32_t* __restrict__ fpos) {
     const unsigned t = fresh_thread(), lane = t % 64, stride = blockDim.x;
     // dictionary: insert every value, remember its slot. A thread takes kBatch positions at a time: their loads
     // and first probes are issued together, so kBatch atomics are in flight per thread instead of one.
@@ -621,260 +624,304 @@ __device__ __forceinline__ void global_firsts(const uint64_t* __restrict__ x, ui
         for (unsigned k = 0; k < kBatch; ++k) {
             const unsigned o = o0 + k * stride;
             fpos[o]          = f[k];
-            if (f[k] == o) atomicOr(&bitmap[o >> 5], 1u << (o & 31));
         }
     }
     __syncthreads();
 }
 
+// Statistics of a row-group, per vector: FFOR and DELTA widths, runs, position bit width; the patch
+// plans of the values and of their lane differences; distinct values (first 16 vectors only).
+struct RgStats {
+    uint32_t bwf[kVPR], bwd[kVPR], runs[kVPR], bwp[kVPR], pbw[kVPR], pexc[kVPR], pchain[kVPR], dbw[kVPR], dexc[kVPR], dchain[kVPR];
+    uint32_t distinct[16], crowded;  // crowded: lds_firsts gave up
+    uint64_t pbase[kVPR];
+};
+
 struct SizerLds {
-    uint32_t bitmap[kRG / 32];
+    RgStats  st;
+    uint32_t bitmap[kRG / 32];  // first occurrences
     uint32_t base[kRG / 32];
-    uint32_t bwf[kVPR], bwd[kVPR], runs[kVPR], bwp[kVPR];
     uint32_t cmin[kVPR], cmax[kVPR], cdmin[kVPR], cdmax[kVPR];
     unsigned long long dmin[kVPR], dmax[kVPR];  // dictionary chunk min / max (chunks of 1024 codes)
     uint32_t tmp[32];
-    // patched FFOR: per vector bit width, base, exceptions and LL chain length; the page's exception values in
-    // chunks of 1024 (S_PATCH_REC's HZL chain)
-    uint32_t           pbw[kVPR], pexc[kVPR], pchain[kVPR], excpref[kVPR + 1];
-    // DELTA patches: the same plan over each vector's lane differences
-    uint32_t           dbw[kVPR], dexc[kVPR], dchain[kVPR];
-    unsigned long long pbase[kVPR], excmin[8], excmax[8];
-    // DICT_RLE: the page's run codes in chunks of 1024 (its HZL chain)
-    uint32_t rcmin[kVPR], rcmax[kVPR], runpref[kVPR + 1];
-    uint32_t claims, rich;  // rich: distinct values of the first 16 vectors, each vector's counted by itself
-    alignas(16) uint64_t sortbuf[16][1024];  // one vector per wave, sorted for the patch plan; then lds_firsts' table
+    unsigned long long excmin[8], excmax[8];    // the page's exception values in chunks of 1024 (S_PATCH_REC's HZL chain)
+    uint32_t excpref[kVPR + 1];
+    uint32_t rcmin[kVPR], rcmax[kVPR], runpref[kVPR + 1];  // DICT_RLE: the page's run codes in chunks of 1024 (its HZL chain)
 };
 
+// Statistics and patch plans of vector v of row-group x, by one wave; sb: 1024 values of LDS.
+__device__ __forceinline__ void size_vector(const uint64_t* __restrict__ x, unsigned v, uint64_t* sb, RgStats& st) {
+    const unsigned lane = fresh_lane();
+    const VecStats s = vector_stats(x + v * 1024);
+    if (lane == 0) st.bwf[v] = s.bwf, st.bwd[v] = s.bwd, st.runs[v] = s.runs, st.bwp[v] = s.bwp;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (unsigned i = 0; i < 16; ++i) sb[64 * i + lane] = x[v * 1024 + 64 * i + lane];
+    if (s.bwf <= 32) wave_sort1024_narrow(sb, (uint64_t)s.smin);
+    else wave_sort1024(sb);
+    __builtin_amdgcn_sched_barrier(0);
+    if (v < 16) {
+        uint32_t d = 0;
+        for (unsigned q = 0; q < 16; ++q) d += (64 * q + lane) == 0 || sb[sorted_at(64 * q + lane)] != sb[sorted_at(64 * q + lane - 1)];
+        d = wave_sum(d);
+        if (lane == 0) st.distinct[v] = d;
+    }
+    const PatchPlan pp = patch_plan(sb, s.bwu);
+    __builtin_amdgcn_sched_barrier(0);
+    // exceptions in transposed order (the order the encoder stores them) and the LL chain's hop entries:
+    // a gap g between consecutive exceptions adds floor((g - 1) / hop) links, hop = 2^min(bw, 11)
+    const unsigned hop = 1u << (pp.bw < 11 ? pp.bw : 11);
+    uint32_t       n = 0, extra = 0;
+    int            last = -1;  // last exception index seen by the wave so far
+    uint64_t       xq[16];     // the 16 values this lane tests, loaded before the ballot chain
+#pragma unroll
+    for (unsigned q = 0; q < 16; ++q) xq[q] = x[v * 1024 + orig_of(64 * q + lane)];
+#pragma unroll
+    for (unsigned q = 0; q < 16; ++q) {
+        const unsigned k  = 64 * q + lane;
+        const bool     ex = is_exception(xq[q], pp);
+        const uint64_t m  = __ballot(ex);
+        if (ex) {
+            const uint64_t below = m & ((1ull << lane) - 1);
+            const int prev = below ? (int)(64 * q + 63 - __clzll((long long)below)) : last;
+            if (prev >= 0) extra += (k - (unsigned)prev - 1) / hop;
+        }
+        if (m) last = (int)(64 * q + 63 - __clzll((long long)m));
+        n += (uint32_t)__popcll(m);
+    }
+    extra = wave_sum(extra);
+    if (lane == 0) {
+        st.pbw[v] = pp.bw, st.pbase[v] = pp.base, st.pexc[v] = n, st.pchain[v] = n + extra;
+    }
+    uint32_t dn = 0, dextra = 0;
+    const PatchPlan pd = delta_patch(x + v * 1024, sb, s, dn, dextra);
+    if (lane == 0) st.dbw[v] = pd.bw, st.dexc[v] = dn, st.dchain[v] = dn + dextra;
+}
+
+// Whether a row-group has more distinct values than one LDS table takes, judged by its first 16 vectors: drawn evenly from
+// 20000 values, a vector has 998 different ones.
+__device__ __forceinline__ bool many_distinct(const RgStats& st) {
+    uint32_t n = 0;
+    for (unsigned v = 0; v < 16; ++v) n += st.distinct[v];
+    return wave_uniform(n) >= 16 * 998;
+}
+
+// The rest of a row-group's sizing by a block: code widths, chains, the candidates' sizes. in_lds: fpos is filled; else it is
+// filled here, through the global table `first`.
+__device__ __forceinline__ void size_rowgroup(const uint64_t* __restrict__ x, bool in_lds, uint32_t* first, uint32_t* fpos,
+                                              uint32_t* slot, SizerLds& L, uint64_t* __restrict__ sizes) {
+    const unsigned t = fresh_thread(), wave = wave_uniform(t / 64), stride = blockDim.x;
+    if (t < kVPR) {
+        L.cmin[t] = ~0u, L.cmax[t] = 0, L.cdmin[t] = ~0u, L.cdmax[t] = 0;
+        L.dmin[t] = kEmpty, L.dmax[t] = 0;
+        L.rcmin[t] = ~0u, L.rcmax[t] = 0;
+    }
+    if (t < 8) L.excmin[t] = kEmpty, L.excmax[t] = 0;
+    if (!in_lds) {
+        global_firsts(x, first, slot, fpos);
+        __syncthreads();
+    }
+    for (unsigned o0 = t; o0 < kRG; o0 += 8 * stride) {  // a bitmap word per half wave
+        uint32_t f[8];
+#pragma unroll
+        for (unsigned k = 0; k < 8; ++k) f[k] = fpos[o0 + k * stride];
+#pragma unroll
+        for (unsigned k = 0; k < 8; ++k) {
+            const unsigned o = o0 + k * stride;
+            const uint64_t m = __ballot(f[k] == o);
+            if (o % 32 == 0) L.bitmap[o / 32] = (uint32_t)(m >> (o & 32));
+        }
+    }
+    __syncthreads();
+    const uint32_t D = block_popcount_scan(L.bitmap, L.base, kRG / 32, L.tmp);
+    // codes: per vector min/max and 32-segment delta min/max; dictionary chunk min/max
+    for (unsigned o0 = fresh_thread(); o0 < kRG; o0 += kBatch * stride) {
+      const unsigned lane = o0 % 64;
+      uint32_t fb[kBatch], fpb[kBatch];
+#pragma unroll
+      for (unsigned k = 0; k < kBatch; ++k) {
+          const unsigned o = o0 + k * stride;
+          fb[k]            = fpos[o];
+          fpb[k]           = (o % 32) ? fpos[o - 1] : 0u;
+      }
+#pragma unroll
+      for (unsigned k = 0; k < kBatch; ++k) {
+        const unsigned o  = o0 + k * stride;
+        const uint32_t f  = fb[k];
+        const uint32_t c  = rank_of(L.bitmap, L.base, f);
+        const uint32_t cp = (o % 32) ? rank_of(L.bitmap, L.base, fpb[k]) : c;
+        const uint32_t d  = c - cp;  // 0 at a segment start
+        const uint32_t cmn = wave_extreme<false>(c), cmx = wave_extreme<true>(c);
+        const uint32_t dmn = wave_extreme<false>(d), dmx = wave_extreme<true>(d);
+        if (lane == 0) {
+            const unsigned v = o >> 10;  // the whole wave lies in one vector
+            atomicMin(&L.cmin[v], cmn), atomicMax(&L.cmax[v], cmx);
+            atomicMin(&L.cdmin[v], dmn), atomicMax(&L.cdmax[v], dmx);
+        }
+        if (f == o) {
+            atomicMin(&L.dmin[c >> 10], (unsigned long long)x[o]);
+            atomicMax(&L.dmax[c >> 10], (unsigned long long)x[o]);
+        }
+      }
+    }
+    __syncthreads();
+    if (t < 64) {  // exclusive prefix of the vectors' runs and exceptions
+        uint32_t a = L.st.runs[t], b = L.st.pexc[t];
+        for (unsigned d = 1; d < 64; d <<= 1) {
+            const uint32_t ya = __shfl_up(a, d, 64), yb = __shfl_up(b, d, 64);
+            if (t >= d) a += ya, b += yb;
+        }
+        if (t == 0) L.runpref[0] = 0, L.excpref[0] = 0;
+        L.runpref[t + 1] = a, L.excpref[t + 1] = b;
+    }
+    __syncthreads();
+    // DICT_RLE run codes and S_PATCH_REC exception values, each as the page's chain in chunks of 1024
+    for (unsigned v = wave; v < kVPR; v += blockDim.x / 64) {
+        const unsigned  lane = fresh_lane();
+        const uint64_t* xv = x + v * 1024;
+        PatchPlan       pp {L.st.pbw[v], 0, L.st.pbase[v]};
+        uint32_t        nr = L.runpref[v], ne = L.excpref[v];
+        for (unsigned q = 0; q < 16; ++q) {
+            const unsigned o   = 64 * q + lane;
+            const uint64_t val = xv[o];
+            const bool     chg = o == 0 || val != xv[o - 1];
+            const uint64_t mr  = __ballot(chg);
+            const uint32_t c  = rank_of(L.bitmap, L.base, fpos[v * 1024 + o]);
+            const uint32_t ck = (nr + (uint32_t)__popcll(mr & ((1ull << lane) - 1))) >> 10;
+            // (a wave's run starts lie in one chunk or two)
+            for (uint32_t k = nr >> 10; mr && k <= (nr + (uint32_t)__popcll(mr) - 1) >> 10; ++k) {
+                const uint32_t cmn = wave_extreme<false>(chg && ck == k ? c : ~0u), cmx = wave_extreme<true>(chg && ck == k ? c : 0u);
+                if (lane == 0) atomicMin(&L.rcmin[k], cmn), atomicMax(&L.rcmax[k], cmx);
+            }
+            nr += (uint32_t)__popcll(mr);
+            const uint64_t ev = xv[orig_of(o)];
+            const bool     ex = is_exception(ev, pp);
+            const uint64_t me = __ballot(ex);
+            if (ex) {
+                const uint32_t chunk = (ne + (uint32_t)__popcll(me & ((1ull << lane) - 1))) >> 10;
+                atomicMin(&L.excmin[chunk], (unsigned long long)ev), atomicMax(&L.excmax[chunk], (unsigned long long)ev);
+            }
+            ne += (uint32_t)__popcll(me);
+        }
+    }
+    __syncthreads();
+    if (t < 64) {  // a lane per vector, or per chunk of a chain
+        // an HZL chain of n values: 12 + 128 bw per full chunk of 1024 while bw is below the type's width, then 12 + the raw rest
+        auto chain = [&](uint32_t n, uint32_t bw, uint32_t width) -> uint32_t {
+            const uint64_t wide = __ballot(t < n / 1024 && bw >= width);
+            const uint32_t full = wide ? (uint32_t)__ffsll((long long)wide) - 1 : n / 1024;
+            return wave_sum(t < full ? 12 + 128 * bw : 0u) + 12 + width / 8 * (n - 1024 * full);
+        };
+        const uint32_t dict   = 8 + chain(D, bitlen64(L.dmax[t] - L.dmin[t]), 64);
+        const uint32_t rchain = chain(L.runpref[kVPR], bitlen64(L.rcmax[t] - L.rcmin[t]), 32);
+        const uint32_t echain = chain(L.excpref[kVPR], t < 8 ? bitlen64(L.excmax[t] - L.excmin[t]) : 0u, 64);
+        const RgStats& q = L.st;
+        const uint32_t pk = 9 + 128 * q.pbw[t], n = q.pexc[t], pkd = 9 + 128 * q.dbw[t], dn = q.dexc[t];
+        uint32_t s[kK];
+        s[0]  = 8192;
+        s[1]  = 9 + 128 * q.bwf[t];
+        s[2]  = 137 + 128 * q.bwd[t];
+        s[3]  = 8 * q.runs[t] + 131 + 128 * q.bwp[t];
+        s[4]  = 8 * q.runs[t] + 2048;
+        s[5]  = 4096;
+        s[6]  = 5 + 128 * bitlen64(L.cmax[t] - L.cmin[t]);
+        s[7]  = 133 + 128 * bitlen64(L.cdmax[t] - L.cdmin[t]);
+        s[8]  = 8 * n + 2 + 2 * n + pk;             // S_PATCH [exceptions][count, positions][bw][base][packed]
+        s[9]  = 2 + 2 * n + pk;                     // S_PATCH_REC: exceptions in the page's chain
+        s[10] = 8 * n + 128 + pk;                   // B_PATCH [exceptions][bitmap]...
+        s[11] = 8 * q.pchain[t] + 4 + pk;           // LL_PATCH [chain values][count, first]...
+        s[12] = 131 + 128 * q.bwp[t];               // DICT_RLE [run codes: chain][lane bases][bw][base][packed]
+        s[13] = 128 + 8 * dn + 2 + 2 * dn + pkd;    // DELTA S_PATCH [lane bases][exceptions][count, positions]...
+        s[14] = 128 + 8 * dn + 128 + pkd;           // DELTA B_PATCH [lane bases][exceptions][bitmap]...
+        s[15] = 128 + 8 * q.dchain[t] + 4 + pkd;    // DELTA LL_PATCH [lane bases][chain values][count, first]...
+        constexpr unsigned arr[kK] = {1, 3, 4, 5, 2, 1, 3, 4, 5, 5, 5, 5, 5, 6, 6, 6};
+        constexpr bool     dic[kK] = {false, false, false, false, false, true, true, true,
+                                      false, false, false, false, true, false, false, false};
+#pragma unroll
+        for (unsigned k = 0; k < kK; ++k) {
+            const uint32_t all = wave_sum(s[k]) + (k == 9 ? echain : 0u) + (k == 12 ? rchain : 0u) + 8 + 4 * arr[k] * kVPR + (dic[k] ? dict : 0u);
+            if (t == 0) sizes[k] = all;
+        }
+    }
+    // reset the slots of the global table that this row-group used (a later row-group reuses it)
+    for (unsigned o0 = fresh_thread(); !in_lds && o0 < kRG; o0 += kBatch * stride) {
+        uint32_t sl[kBatch];
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) sl[k] = slot[o0 + k * stride];
+#pragma unroll
+        for (unsigned k = 0; k < kBatch; ++k) {
+            if (fpos[o0 + k * stride] != o0 + k * stride) continue;  // each slot once: at its first occurrence
+            first[sl[k]] = kNoPos;
+        }
+    }
+}
+
+// A block per row-group.
 __global__ __launch_bounds__(1024) void k_wizard_sizes(const uint64_t* __restrict__ values, uint64_t n_rg,
                                                        uint32_t* __restrict__ firsts_all, uint32_t* __restrict__ slots_all,
                                                        uint64_t* __restrict__ sizes) {
-    // dynamic LDS (the launch passes sizeof(SizerLds), about 150 KB)
+    // the statistics, then 16 sort buffers, the table of first occurrences, or the rest of the row-group's state
     extern __shared__ __attribute__((aligned(16))) uint8_t wiz_lds[];
-    SizerLds&      L = *reinterpret_cast<SizerLds*>(wiz_lds);
-    uint32_t* first  = firsts_all + (uint64_t)blockIdx.x * (2 * kHt + 64);  // the table: first position per slot
-    uint32_t* fpos   = first + kHt + 32;                                   // first occurrence per position (kRG)
-    uint32_t* slot   = slots_all + (uint64_t)blockIdx.x * kRG;
+    SizerLds&       L   = *reinterpret_cast<SizerLds*>(wiz_lds);
+    uint8_t* const  big = wiz_lds + (sizeof(SizerLds) + 15) / 16 * 16;
+    uint32_t* const tab = reinterpret_cast<uint32_t*>(big);
+    uint32_t* first = firsts_all + (uint64_t)blockIdx.x * (2 * kHt + 64);  // the global table: first position per slot
+    uint32_t* fpos  = first + kHt + 32;                                   // first occurrence per position (kRG)
+    uint32_t* slot  = slots_all + (uint64_t)blockIdx.x * kRG;
     for (uint64_t r = blockIdx.x; r < n_rg; r += gridDim.x) {
         const uint64_t* x = values + r * kRG;
-        const unsigned  t = fresh_thread(), wave = wave_uniform(t / 64);
-        for (unsigned i = t; i < kRG / 32; i += blockDim.x) L.bitmap[i] = 0;
-        if (t < kVPR) {
-            L.cmin[t] = ~0u, L.cmax[t] = 0, L.cdmin[t] = ~0u, L.cdmax[t] = 0;
-            L.dmin[t] = kEmpty, L.dmax[t] = 0;
-            L.rcmin[t] = ~0u, L.rcmax[t] = 0;
-        }
-        if (t < 8) L.excmin[t] = kEmpty, L.excmax[t] = 0;
-        if (t == 0) L.rich = 0;
-        __syncthreads();
-        // per-vector statistics and patch plans (wave w takes vectors w, w + 16, ...)
+        const unsigned  wave = wave_uniform(fresh_thread() / 64);
 #pragma unroll 1
-        for (unsigned v = wave; v < kVPR; v += blockDim.x / 64) {
-            const unsigned lane = fresh_lane();
-            const VecStats s = vector_stats(x + v * 1024);
-            if (lane == 0) L.bwf[v] = s.bwf, L.bwd[v] = s.bwd, L.runs[v] = s.runs, L.bwp[v] = s.bwp;
-            __builtin_amdgcn_sched_barrier(0);
-            uint64_t*      sb = L.sortbuf[wave];
-#pragma unroll
-            for (unsigned i = 0; i < 16; ++i) sb[64 * i + lane] = x[v * 1024 + 64 * i + lane];
-            if (s.bwf <= 32) wave_sort1024_narrow(sb, (uint64_t)s.smin);
-            else wave_sort1024(sb);
-            __builtin_amdgcn_sched_barrier(0);
-            if (v < 16) {
-                uint32_t d = 0;
-                for (unsigned q = 0; q < 16; ++q) d += (64 * q + lane) == 0 || sb[sorted_at(64 * q + lane)] != sb[sorted_at(64 * q + lane - 1)];
-                d = wave_sum(d);
-                if (lane == 0) atomicAdd(&L.rich, d);
-            }
-            const PatchPlan pp = patch_plan(sb, s.bwu);
-            __builtin_amdgcn_sched_barrier(0);
-            // exceptions in transposed order (the order the encoder stores them) and the LL chain's hop entries:
-            // a gap g between consecutive exceptions adds floor((g - 1) / hop) links, hop = 2^min(bw, 11)
-            const unsigned hop = 1u << (pp.bw < 11 ? pp.bw : 11);
-            uint32_t       n = 0, extra = 0;
-            int            last = -1;  // last exception index seen by the wave so far
-            uint64_t       xq[16];     // the 16 values this lane tests, loaded before the ballot chain
-#pragma unroll
-            for (unsigned q = 0; q < 16; ++q) xq[q] = x[v * 1024 + orig_of(64 * q + lane)];
-#pragma unroll
-            for (unsigned q = 0; q < 16; ++q) {
-                const unsigned k  = 64 * q + lane;
-                const bool     ex = is_exception(xq[q], pp);
-                const uint64_t m  = __ballot(ex);
-                if (ex) {
-                    const uint64_t below = m & ((1ull << lane) - 1);
-                    const int prev = below ? (int)(64 * q + 63 - __clzll((long long)below)) : last;
-                    if (prev >= 0) extra += (k - (unsigned)prev - 1) / hop;
-                }
-                if (m) last = (int)(64 * q + 63 - __clzll((long long)m));
-                n += (uint32_t)__popcll(m);
-            }
-            extra = wave_sum(extra);
-            if (lane == 0) {
-                L.pbw[v] = pp.bw, L.pbase[v] = pp.base, L.pexc[v] = n, L.pchain[v] = n + extra;
-            }
-            uint32_t dn = 0, dextra = 0;
-            const PatchPlan pd = delta_patch(x + v * 1024, sb, s, dn, dextra);
-            if (lane == 0) L.dbw[v] = pd.bw, L.dexc[v] = dn, L.dchain[v] = dn + dextra;
-        }
-        // dictionary: every position's first occurrence, over the LDS table (all values at once, or by hash partition when
-        // they are too many), or over the global one where a partition is too large for it (hashes that agree)
-        const unsigned stride = blockDim.x;
-        uint32_t*      tab    = reinterpret_cast<uint32_t*>(L.sortbuf);
+        for (unsigned v = wave; v < kVPR; v += blockDim.x / 64) size_vector(x, v, reinterpret_cast<uint64_t*>(big) + 1024 * wave, L.st);
         __syncthreads();
-        // (drawn evenly from 20000 values, the most that one table takes, a vector has 998 different ones)
-        bool           in_lds = L.rich < 16 * 998 && lds_firsts(x, tab, &L.claims, L.bitmap, slot, fpos, 1);
-        if (!in_lds) in_lds = lds_firsts(x, tab, &L.claims, L.bitmap, slot, fpos, 4);
-        if (!in_lds) {
-            __syncthreads();
-            for (unsigned i = t; i < kRG / 32; i += stride) L.bitmap[i] = 0;  // partitions before may have set some
-            __syncthreads();
-            global_firsts(x, first, L.bitmap, slot, fpos);
-        }
-        const uint32_t D = block_popcount_scan(L.bitmap, L.base, kRG / 32, L.tmp);
-        // codes: per vector min/max and 32-segment delta min/max; dictionary chunk min/max
-        for (unsigned o0 = fresh_thread(); o0 < kRG; o0 += kBatch * stride) {
-          const unsigned lane = o0 % 64;
-          uint32_t fb[kBatch], fpb[kBatch];
-#pragma unroll
-          for (unsigned k = 0; k < kBatch; ++k) {
-              const unsigned o = o0 + k * stride;
-              fb[k]            = fpos[o];
-              fpb[k]           = (o % 32) ? fpos[o - 1] : 0u;
-          }
-#pragma unroll
-          for (unsigned k = 0; k < kBatch; ++k) {
-            const unsigned o  = o0 + k * stride;
-            const uint32_t f  = fb[k];
-            const uint32_t c  = rank_of(L.bitmap, L.base, f);
-            const uint32_t cp = (o % 32) ? rank_of(L.bitmap, L.base, fpb[k]) : c;
-            const uint32_t d  = c - cp;  // 0 at a segment start
-            const uint32_t cmn = wave_extreme<false>(c), cmx = wave_extreme<true>(c);
-            const uint32_t dmn = wave_extreme<false>(d), dmx = wave_extreme<true>(d);
-            if (lane == 0) {
-                const unsigned v = o >> 10;  // the whole wave lies in one vector
-                atomicMin(&L.cmin[v], cmn), atomicMax(&L.cmax[v], cmx);
-                atomicMin(&L.cdmin[v], dmn), atomicMax(&L.cdmax[v], dmx);
-            }
-            if (f == o) {
-                atomicMin(&L.dmin[c >> 10], (unsigned long long)x[o]);
-                atomicMax(&L.dmax[c >> 10], (unsigned long long)x[o]);
-            }
-          }
-        }
-        __syncthreads();
-        if (t == 0) {
-            uint32_t a = 0, b = 0;
-            for (unsigned v = 0; v < kVPR; ++v) L.runpref[v] = a, a += L.runs[v], L.excpref[v] = b, b += L.pexc[v];
-            L.runpref[kVPR] = a, L.excpref[kVPR] = b;
-        }
-        __syncthreads();
-        // DICT_RLE run codes and S_PATCH_REC exception values, each as the page's chain in chunks of 1024
-        for (unsigned v = wave; v < kVPR; v += blockDim.x / 64) {
-            const unsigned  lane = fresh_lane();
-            const uint64_t* xv = x + v * 1024;
-            PatchPlan       pp {L.pbw[v], 0, L.pbase[v]};
-            uint32_t        nr = L.runpref[v], ne = L.excpref[v];
-            for (unsigned q = 0; q < 16; ++q) {
-                const unsigned o   = 64 * q + lane;
-                const uint64_t val = xv[o];
-                const bool     chg = o == 0 || val != xv[o - 1];
-                const uint64_t mr  = __ballot(chg);
-                const uint32_t c  = rank_of(L.bitmap, L.base, fpos[v * 1024 + o]);
-                const uint32_t ck = (nr + (uint32_t)__popcll(mr & ((1ull << lane) - 1))) >> 10;
-                // (a wave's run starts lie in one chunk or two)
-                for (uint32_t k = nr >> 10; mr && k <= (nr + (uint32_t)__popcll(mr) - 1) >> 10; ++k) {
-                    const uint32_t cmn = wave_extreme<false>(chg && ck == k ? c : ~0u), cmx = wave_extreme<true>(chg && ck == k ? c : 0u);
-                    if (lane == 0) atomicMin(&L.rcmin[k], cmn), atomicMax(&L.rcmax[k], cmx);
-                }
-                nr += (uint32_t)__popcll(mr);
-                const uint64_t ev = xv[orig_of(o)];
-                const bool     ex = is_exception(ev, pp);
-                const uint64_t me = __ballot(ex);
-                if (ex) {
-                    const uint32_t chunk = (ne + (uint32_t)__popcll(me & ((1ull << lane) - 1))) >> 10;
-                    atomicMin(&L.excmin[chunk], (unsigned long long)ev), atomicMax(&L.excmax[chunk], (unsigned long long)ev);
-                }
-                ne += (uint32_t)__popcll(me);
-            }
-        }
-        __syncthreads();
-        if (t == 0) {
-            uint64_t hzl = 0, pos = 0;
-            while (D - pos >= 1024) {
-                const uint32_t bw = bitlen64(L.dmax[pos >> 10] - L.dmin[pos >> 10]);
-                if (bw >= 64) break;
-                hzl += 12 + 128ull * bw;
-                pos += 1024;
-            }
-            hzl += 12 + 8ull * (D - pos);
-            const uint64_t dict = 8 + hzl;
-            // HZL chains of the page's run codes (u32) and exception values (u64): 12 + 128 bw per full chunk of 1024
-            // while bw is below the type width, then 12 + the raw rest
-            uint64_t       rchain = 0, echain = 0;
-            {
-                const uint32_t R = L.runpref[kVPR];
-                uint32_t       p = 0;
-                for (; R - p >= 1024; p += 1024) {
-                    const uint32_t bw = bitlen64(L.rcmax[p >> 10] - L.rcmin[p >> 10]);
-                    if (bw >= 32) break;
-                    rchain += 12 + 128ull * bw;
-                }
-                rchain += 12 + 4ull * (R - p);
-                const uint32_t E = L.excpref[kVPR];
-                p = 0;
-                for (; E - p >= 1024; p += 1024) {
-                    const uint32_t bw = bitlen64(L.excmax[p >> 10] - L.excmin[p >> 10]);
-                    if (bw >= 64) break;
-                    echain += 12 + 128ull * bw;
-                }
-                echain += 12 + 8ull * (E - p);
-            }
-            uint64_t s[kK] = {};
-            for (unsigned v = 0; v < kVPR; ++v) {
-                const uint64_t pk = 9 + 128ull * L.pbw[v], n = L.pexc[v];
-                s[0] += 8192;
-                s[1] += 9 + 128ull * L.bwf[v];
-                s[2] += 137 + 128ull * L.bwd[v];
-                s[3] += 8ull * L.runs[v] + 131 + 128ull * L.bwp[v];
-                s[4] += 8ull * L.runs[v] + 2048;
-                s[5] += 4096;
-                s[6] += 5 + 128ull * bitlen64(L.cmax[v] - L.cmin[v]);
-                s[7] += 133 + 128ull * bitlen64(L.cdmax[v] - L.cdmin[v]);
-                s[8] += 8 * n + 2 + 2 * n + pk;             // S_PATCH [exceptions][count, positions][bw][base][packed]
-                s[9] += 2 + 2 * n + pk;                     // S_PATCH_REC: exceptions in the page's chain
-                s[10] += 8 * n + 128 + pk;                  // B_PATCH [exceptions][bitmap]...
-                s[11] += 8ull * L.pchain[v] + 4 + pk;       // LL_PATCH [chain values][count, first]...
-                s[12] += 131 + 128ull * L.bwp[v];           // DICT_RLE [run codes: chain][lane bases][bw][base][packed]
-                const uint64_t pkd = 9 + 128ull * L.dbw[v], dn = L.dexc[v];
-                s[13] += 128 + 8 * dn + 2 + 2 * dn + pkd;   // DELTA S_PATCH [lane bases][exceptions][count, positions]...
-                s[14] += 128 + 8 * dn + 128 + pkd;          // DELTA B_PATCH [lane bases][exceptions][bitmap]...
-                s[15] += 128 + 8ull * L.dchain[v] + 4 + pkd; // DELTA LL_PATCH [lane bases][chain values][count, first]...
-            }
-            s[9] += echain;
-            s[12] += rchain;
-            constexpr unsigned arr[kK]  = {1, 3, 4, 5, 2, 1, 3, 4, 5, 5, 5, 5, 5, 6, 6, 6};
-            constexpr bool     dic[kK]  = {false, false, false, false, false, true, true, true,
-                                           false, false, false, false, true, false, false, false};
-            for (unsigned k = 0; k < kK; ++k) {
-                s[k] += 8 + 4ull * arr[k] * kVPR + (dic[k] ? dict : 0);
-                sizes[r * kK + k] = s[k];
-            }
-        }
-        // reset the slots of the global table that this row-group used (the next row-group of this block reuses it)
-        for (unsigned o0 = fresh_thread(); !in_lds && o0 < kRG; o0 += kBatch * stride) {
-            uint32_t sl[kBatch];
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) sl[k] = slot[o0 + k * stride];
-#pragma unroll
-            for (unsigned k = 0; k < kBatch; ++k) {
-                if (fpos[o0 + k * stride] != o0 + k * stride) continue;  // each slot once: at its first occurrence
-                first[sl[k]] = kNoPos;
-            }
-        }
+        bool ok = !many_distinct(L.st) && lds_firsts<true>(x, tab, L.tmp, slot, fpos, 0, 1, 1);
+        if (!ok) ok = lds_firsts<true>(x, tab, L.tmp, slot, fpos, 0, 4, 4);
+        size_rowgroup(x, ok, first, fpos, slot, L, sizes + r * kK);
         __syncthreads();
     }
 }
+
+// The same in three launches for a few row-groups, which one block each would leave most of the chip idle: a wave per vector
+// anywhere; four blocks per row-group for the first occurrences, a hash partition each, where its values are mostly distinct
+// (else the first block alone); a block per row-group for the rest.
+constexpr unsigned kVecWaves = 4;
+__global__ __launch_bounds__(64 * kVecWaves) void k_wizard_vectors(const uint64_t* __restrict__ values, RgStats* __restrict__ stats) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t wiz_lds[];  // 8 KiB per wave
+    const unsigned wave = wave_uniform(threadIdx.x / 64), id = blockIdx.x * kVecWaves + wave;
+    RgStats&       st = stats[id / kVPR];
+    if (id % kVPR == 0 && threadIdx.x % 64 == 0) st.crowded = 0;
+    size_vector(values + (uint64_t)(id / kVPR) * kRG, id % kVPR, reinterpret_cast<uint64_t*>(wiz_lds) + 1024 * wave, st);
+}
+__global__ __launch_bounds__(1024) void k_wizard_firsts(const uint64_t* __restrict__ values, unsigned n_rg,
+                                                        RgStats* __restrict__ stats, uint32_t* __restrict__ firsts_all,
+                                                        uint32_t* __restrict__ slots_all) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t wiz_lds[];  // the table, and a count behind it
+    uint32_t* const tab = reinterpret_cast<uint32_t*>(wiz_lds);
+    // a row-group's blocks 8 apart: on one XCD, whose L2 joins the parts of lines that they write (16
+    // row-groups 393 us with neighbours on eight XCDs, 378 so)
+    const unsigned  r = blockIdx.x / 32 * 8 + blockIdx.x % 8, part = blockIdx.x / 8 % 4;
+    if (r >= n_rg) return;
+    const bool      many = many_distinct(stats[r]);
+    const uint64_t* x    = values + (uint64_t)r * kRG;
+    uint32_t*       slot = slots_all + (uint64_t)r * kRG;
+    uint32_t*       fpos = firsts_all + (uint64_t)r * (2 * kHt + 64) + kHt + 32;
+    if (!many && part) return;
+    bool ok = !many && lds_firsts<false>(x, tab, tab + kLt, slot, fpos, 0, 1, 1);
+    if (!ok) ok = lds_firsts<false>(x, tab, tab + kLt, slot, fpos, many ? part : 0, many ? part + 1 : 4, 4);
+    if (!ok && threadIdx.x == 0) stats[r].crowded = 1;
+}
+__global__ __launch_bounds__(1024) void k_wizard_finish(const uint64_t* __restrict__ values, const RgStats* __restrict__ stats,
+                                                        uint32_t* __restrict__ firsts_all, uint32_t* __restrict__ slots_all,
+                                                        uint64_t* __restrict__ sizes) {
+    __shared__ SizerLds L;
+    const uint64_t r     = blockIdx.x;
+    uint32_t*      first = firsts_all + r * (2 * kHt + 64);
+    static_assert(sizeof(RgStats) % 4 == 0 && sizeof(RgStats) <= 4096, "copied by one round of the block");
+    if (threadIdx.x < sizeof(RgStats) / 4)
+        reinterpret_cast<uint32_t*>(&L.st)[threadIdx.x] = reinterpret_cast<const uint32_t*>(stats + r)[threadIdx.x];
+    size_rowgroup(values + r * kRG, stats[r].crowded == 0, first, first + kHt + 32, slots_all + r * kRG, L, sizes + r * kK);
+}
+
 
 __global__ void k_wizard_best(const uint64_t* __restrict__ sizes, uint64_t n_rg, int32_t* __restrict__ choice) {
     const uint64_t r = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1092,7 +1139,8 @@ __global__ __launch_bounds__(256) void k_wizard_features(const uint64_t* __restr
 struct SizerWs {
     uint32_t* firsts = nullptr;
     uint32_t* slots  = nullptr;
-    unsigned  blocks = 0;
+    RgStats*  stats  = nullptr;
+    unsigned  blocks = 0;  // row-groups it holds
 };
 std::mutex           g_ws_mu;
 std::vector<SizerWs> g_ws;
@@ -1104,16 +1152,17 @@ int sizer_ws(SizerWs*& out) {
     std::lock_guard<std::mutex> lk(g_ws_mu);
     if ((int)g_ws.size() <= dev) g_ws.resize(dev + 1);
     SizerWs& w = g_ws[dev];
-    if (!w.firsts) {
+    if (!w.stats) {  // (allocated last: a call that failed half way is taken up again)
         hipDeviceProp_t prop;
         if ((e = hipGetDeviceProperties(&prop, dev)) != hipSuccess) return hip_fail(e, "device properties");
         w.blocks = (unsigned)prop.multiProcessorCount;
         const size_t fb = (size_t)w.blocks * (2 * kHt + 64) * 4, sb = (size_t)w.blocks * kRG * 4;
-        if ((e = hipMalloc(&w.firsts, fb)) != hipSuccess) return hip_fail(e, "hipMalloc");
-        if ((e = hipMalloc(&w.slots, sb)) != hipSuccess) return hip_fail(e, "hipMalloc");
+        if (!w.firsts && (e = hipMalloc(&w.firsts, fb)) != hipSuccess) return hip_fail(e, "hipMalloc");
+        if (!w.slots && (e = hipMalloc(&w.slots, sb)) != hipSuccess) return hip_fail(e, "hipMalloc");
         // empty slots; the kernel restores this state after every row-group
         if ((e = hipMemset(w.firsts, 0xFF, fb)) != hipSuccess) return hip_fail(e, "hipMemset");
         if ((e = hipDeviceSynchronize()) != hipSuccess) return hip_fail(e, "sync");
+        if ((e = hipMalloc(&w.stats, w.blocks * sizeof(RgStats))) != hipSuccess) return hip_fail(e, "hipMalloc");
     }
     out = &w;
     return FLS_OK;
@@ -1136,11 +1185,23 @@ int fls_wizard_sizes(const int64_t* dev_values, uint64_t n_rowgroups, uint64_t* 
     SizerWs* w  = nullptr;
     int      rc = sizer_ws(w);
     if (rc) return rc;
-    const unsigned blocks = (unsigned)std::min<uint64_t>(n_rowgroups, w->blocks);
-    hipLaunchKernelGGL(k_wizard_sizes, dim3(blocks), dim3(1024), sizeof(SizerLds), (hipStream_t)stream, (const uint64_t*)dev_values,
-                       n_rowgroups, w->firsts, w->slots, dev_sizes);
+    const uint64_t* x = (const uint64_t*)dev_values;
+    hipStream_t     q = (hipStream_t)stream;
+    // four blocks per row-group as long as each has a compute unit: 1 row-group 282 us (707 by one block), 16 378 (978), 64 839
+    // (998); past that their partial lines of the scratch arrays cost more (256 row-groups: 1489 us, 1060 by one block each)
+    if (n_rowgroups * 4 <= w->blocks) {
+        const unsigned n = (unsigned)n_rowgroups;
+        hipLaunchKernelGGL(k_wizard_vectors, dim3(n * (kVPR / kVecWaves)), dim3(64 * kVecWaves), 8192 * kVecWaves, q, x, w->stats);
+        hipLaunchKernelGGL(k_wizard_firsts, dim3((n + 7) / 8 * 32), dim3(1024), 4 * kLt + 16, q, x, n, w->stats, w->firsts, w->slots);
+        hipLaunchKernelGGL(k_wizard_finish, dim3(n), dim3(1024), 0, q, x, w->stats, w->firsts, w->slots, dev_sizes);
+    } else {
+        const unsigned blocks = (unsigned)std::min<uint64_t>(n_rowgroups, w->blocks);
+        hipLaunchKernelGGL(k_wizard_sizes, dim3(blocks), dim3(1024), (sizeof(SizerLds) + 15) / 16 * 16 + 4 * kLt, q, x, n_rowgroups,
+                           w->firsts, w->slots, dev_sizes);
+    }
     const hipError_t e = hipGetLastError();
-    return e == hipSuccess ? FLS_OK : hip_fail(e, "wizard sizes launch");
+    if (e != hipSuccess) return hip_fail(e, "wizard sizes launch");
+    return FLS_OK;
 }
 
 int fls_wizard_best(const uint64_t* dev_sizes, uint64_t n_rowgroups, int32_t* dev_choice, void* stream) {

@@ -215,3 +215,23 @@ def test_sizes_over_dictionary_tables(torch_cuda, wiz, order):
         sizes = d_s.cpu().numpy()
         for r in range(len(rgs)):
             np.testing.assert_array_equal(sizes[r], want[r], err_msg=f"row-group {r}")
+
+
+@pytest.mark.parametrize("n_rg", [1, 9, 64, 65])
+def test_sizes_of_few_row_groups(torch_cuda, wiz, n_rg):
+    """The three launches that size up to a quarter as many row-groups as there are compute units, a batch that does not
+    fill their grid, and one row-group more than they take, on row-groups of both kinds (mostly distinct or not)."""
+    torch = torch_cuda
+    g = np.random.default_rng(n_rg)
+    base = [x for _, x in rowgroups()[:8]] + [g.integers(-(1 << 62), 1 << 62, wo.RG, dtype=np.int64)]
+    want = [wo.candidate_sizes(x).astype(np.int64) for x in base]
+    pick = [(7 * r + 8) % len(base) for r in range(n_rg)]
+    d_x = torch.from_numpy(np.concatenate([base[p] for p in pick])).cuda()
+    d_s = torch.full((n_rg + 1, len(wo.CANDIDATES)), -1, dtype=torch.int64, device="cuda")
+    print(f"wizard sizes of {n_rg} row-groups", flush=True)
+    wiz.exhaustive_sizes(d_x.data_ptr(), n_rg, d_s.data_ptr())
+    torch.cuda.synchronize()
+    sizes = d_s.cpu().numpy()
+    for r, p in enumerate(pick):
+        np.testing.assert_array_equal(sizes[r], want[p], err_msg=f"row-group {r}")
+    assert (sizes[n_rg] == -1).all()
