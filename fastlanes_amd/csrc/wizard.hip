@@ -460,11 +460,11 @@ __device__ PatchPlan delta_patch(const uint64_t* __restrict__ xv, uint64_t* sb, 
 
 // The sizer's LDS table (over the sort buffers, which are idle by then). A slot holds 15 hash bits and the smallest
 // position of its value, so a value is compared through the row-group's own values only where 15 more bits of its hash
-// agree. The four positions that a thread takes at a time probe in step, so that their LDS
-// reads, exchanges and value loads are in flight together. All values at once (parts 1) or those of the hash partitions
-// [part, end) of 4, one after another; only their places of fpos[] are
-// written, and of slot[] (scratch; ALONE: no other block shares it, and whole lines are written). Returns false when the
-// table takes no more (the values of a partition are too many); the block is at a barrier then.
+// agree. The four positions that a thread takes at a time probe in step, so that their LDS reads, exchanges and value loads
+// are in flight together. All values at once (parts 1) or those of the hash partitions [part, end) of 4, one after another;
+// only their places of fpos[] are written, and of slot[] (scratch; ALONE: no other block shares it, and whole lines are
+// written). Returns false when the table takes no more (the values of a partition are too many); the block is at a barrier
+// then. Claims never fill the table: the count is looked at before every round of 1024 x kBatch, so every probe ends.
 // (a table filled to 28000 of its 32768 slots made some probes hundreds of slots long: 2570 us for the slowest row-groups)
 constexpr unsigned kLt = 32768, kLtTake = 20000;
 constexpr unsigned kBatch = 4;
