@@ -21,8 +21,9 @@
 // instructions per code, measured 135 us: unaligned LDS writes take about one cycle per lane.) 2^21 strings: 151 -> 71 us
 // a call, k_fsst 42, bound by its vector instructions. No variable of k_fsst may spill: a build whose registers did gave
 // wrong bytes in a hundredth of the segments.
-// Segments that are malformed (non-monotone offsets) take a per-string path that reads and writes global memory byte by
-// byte.
+// A vector with a malformed segment (non-monotone offsets) takes a per-string path that reads and writes global memory byte
+// by byte, for all four of its segments: the granules' sizes are kept by byte position, which is one segment's own only
+// while no segment of the vector reaches back over another.
 #include <algorithm>
 
 #include "../../include/fls_gpu.h"
@@ -103,7 +104,7 @@ __device__ __forceinline__ uint32_t byte_of(const uint32_t (&wd)[8]) {
 }
 
 // What k_fsst_count leaves for k_fsst per segment: decoded bytes, those of the vector's segments before it (kMalformed:
-// its offsets are not monotone), and the place of its compressed bytes in the vector's.
+// the vector's offsets are not monotone), and the place of its compressed bytes in the vector's.
 struct FsstSeg {
     uint64_t total, before;
     uint32_t s0, n;
@@ -118,7 +119,7 @@ struct Segment {
 };
 
 // Place of a segment's first granule in StringPlan::d_sizes: granules of 32 bytes from the column's start, one more per
-// segment before it for the partial ones.
+// segment before it for the partial ones (segments that follow one another in memory: no two share a place).
 __device__ __forceinline__ uint64_t sizes_at(uint64_t page_off, const uint8_t* page, const uint8_t* bytes, uint64_t seg) {
     return (page_off + (uint64_t)(bytes - page)) / kShare + seg;
 }
@@ -339,14 +340,14 @@ __global__ __launch_bounds__(kSeg* GROUPS, 8) void k_fsst_count(const uint8_t* _
         const uint32_t e = ends[end_place(i)], s = i ? ends[end_place(i - 1)] : 0u, s0 = bound(h);
         end[i]                          = e - s0;
         str_end[(seg + h) * kSeg + tid] = e - s0;
-        if (!(span(h) && s0 <= s && s <= e && e <= bound(h + 1))) atomicOr(&malformed, 1u << h);
+        if (!(span(h) && s0 <= s && s <= e && e <= bound(h + 1))) malformed = 1;
     }
     __syncthreads();
     for (unsigned h = group; h < kSegPerV; h += GROUPS) {
         const uint32_t s0 = bound(h);
         const Segment  g {cb + s0, span(h) ? bound(h + 1) - s0 : 0u, end + h * kSeg};
         uint64_t       mine = 0;
-        if (!((malformed >> h) & 1u)) {
+        if (!malformed) {
             uint16_t* const at = sizes + sizes_at(page_off, page, g.seg, seg + h);
             for (uint32_t c0 = 0; c0 < g.n; c0 += kChunk) {
                 const Granule r    = open_granule(g, c0, tid);
@@ -371,7 +372,7 @@ __global__ __launch_bounds__(kSeg* GROUPS, 8) void k_fsst_count(const uint8_t* _
         for (unsigned k = 0; k < kSegPerV; ++k) {
             uint64_t all = 0;
             for (unsigned w = 0; w < kWaves; ++w) all += wsum[k][w];
-            segs[seg + k] = {all, (malformed >> k) & 1u ? vec | kMalformed : vec, bound(k), span(k) ? bound(k + 1) - bound(k) : 0u};
+            segs[seg + k] = {all, malformed ? vec | kMalformed : vec, bound(k), span(k) ? bound(k + 1) - bound(k) : 0u};
             vec += all;
         }
         vecs[seg / kSegPerV] = vec;
@@ -481,6 +482,10 @@ __global__ __launch_bounds__(kSeg, 6) void k_fsst(const uint8_t* __restrict__ pa
             uint32_t       total;
             const uint32_t at = block_exclusive_scan(size, wsum, &total);
             total             = __builtin_amdgcn_readfirstlane(total);  // the same in every lane: scalar from here on
+            if (total > seg_total - done) {  // never more than what the capacity was tested with
+                if (tid == 0) atomicOr(err, kErrCap);
+                total = (uint32_t)(seg_total - done);
+            }
             if constexpr (MODE != FS_BYTES) sbase[tid] = at;
             Escapes es {0, 0};
             if (sz & kSpecial) es = find_escapes(g, r);

@@ -221,3 +221,81 @@ def test_fused_segment_bases(torch_cuda, vectors):
     got_off, got = _fused(torch, fa.Plan(enc, "str"), dev(torch, enc), offs.size - 1, data.size)
     np.testing.assert_array_equal(got_off, offs)
     np.testing.assert_array_equal(got[: data.size], data)
+
+
+def _string_page(enc):
+    """Symbols of a column's (single) FSST page, where its data page starts, and its two buffers' offsets in it."""
+    lh = [int(x) for x in enc[17:25]]  # lenHisto: symbols of 1 .. 8 bytes
+    zt, at, symbols = int(enc[16]) & 1, 25, [b"\0"] if int(enc[16]) & 1 else []
+    lh[0] -= zt
+    for k in (1, 2, 3, 4, 5, 6, 7, 0):
+        for _ in range(lh[k]):
+            symbols.append(enc[at: at + k + 1].tobytes())
+            at += k + 1
+    return symbols, at, enc[at + 8: at + 16].view(np.uint32).astype(np.int64)
+
+
+def _decode_vector(symbols, bytes_, ends):
+    """Strings of a vector: string i is the codes of bytes_[ends[i - 1] : ends[i]] (none where the end lies before)."""
+    out = []
+    for i, e in enumerate(ends):
+        q, row = int(ends[i - 1]) if i else 0, []
+        while q < e:
+            c = int(bytes_[q])
+            row.append(bytes([int(bytes_[q + 1]) if q + 1 < e else 0]) if c == 255 else symbols[c])
+            q += 2 if c == 255 else 1
+        out.append(b"".join(row))
+    return out
+
+
+@pytest.mark.parametrize("ends", ["lowered_at_segment_end", "lowered_inside", "lowered_to_zero", "raised", "shuffled"])
+def test_ends_out_of_order(torch_cuda, ends):
+    """End offsets that are not monotone in the middle one of three vectors: a segment that starts behind the one before it
+    (well-formed by itself, over bytes that other segments hold too), one whose strings alone are out of order, one that
+    starts past its first end. Every string is its own range of codes in all three call forms, its neighbours' vectors are
+    untouched, and nothing is written past the capacity."""
+    torch = torch_cuda
+    g = np.random.default_rng(5)
+    rows = [bytes(g.integers(97, 105, int(g.integers(0, 40)), dtype=np.uint8).tobytes()) for _ in range(3 * 1024)]
+    for i in range(0, len(rows), 7):  # escapes
+        rows[i] += bytes(g.integers(200, 256, 3, dtype=np.uint8).tobytes())
+    offs, data = _strs_from(rows)
+    enc = fa.encode_strings(offs.astype(np.uint32), data).copy()
+    symbols, page, boff = _string_page(enc)
+    eps = enc[page + 16: page + 32].view(np.uint32).astype(np.int64).reshape(2, 2)  # of vectors 1 and 2
+    at = page + int(boff[1] + eps[0, 1])
+    k = np.arange(1024)
+    order = np.array([0, 4, 2, 6, 1, 5, 3, 7])
+    place = 128 * (k % 8) + 16 * order[(k // 8) % 8] + k // 64  # string -> transposed position
+    stored = enc[at: at + 4096].view(np.uint32).copy()
+    e = stored[place].astype(np.int64)
+    if ends == "lowered_at_segment_end":
+        e[767] = 40
+    elif ends == "lowered_inside":
+        e[300] = e[290]
+    elif ends == "lowered_to_zero":
+        e[255:258] = 0
+    elif ends == "raised":
+        e[511] = e[600]
+    else:
+        e = g.permutation(e)
+    stored[place] = e.astype(np.uint32)
+    enc[at: at + 4096] = stored.view(np.uint8)
+    start = page + int(boff[0] + eps[0, 0])
+    rows[1024:2048] = _decode_vector(symbols, enc[start: page + int(boff[0] + eps[1, 0])], e)
+    want_off, want = _strs_from(rows)
+    print(f"fsst ends={ends} bytes={want.size}", flush=True)
+    plan, d_in, n = fa.Plan(enc, "str"), dev(torch, enc), offs.size - 1
+    got_off, got = _fused(torch, plan, d_in, n, want.size)
+    np.testing.assert_array_equal(got_off, want_off)
+    np.testing.assert_array_equal(got[: want.size], want)
+    d_off = torch.zeros(n + 1, dtype=torch.int64, device="cuda")
+    plan.string_offsets(d_in.data_ptr(), d_off.data_ptr())
+    np.testing.assert_array_equal(d_off.cpu().numpy(), want_off)
+    for cap, ok in ((want.size, True), (want.size - 1, False)):
+        d_bytes = torch.full((want.size + 65536,), 171, dtype=torch.uint8, device="cuda")
+        plan.decode_strings(d_in.data_ptr(), d_off.data_ptr(), d_bytes.data_ptr(), cap)
+        assert (d_bytes.cpu().numpy()[cap:] == 171).all()
+        if ok:
+            plan.check()
+            np.testing.assert_array_equal(d_bytes.cpu().numpy()[:cap], want)
