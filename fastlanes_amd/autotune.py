@@ -1,7 +1,7 @@
 """Launch-shape autotuner for the decode kernels.
 
-For every kernel family (raw streams per element width and bit width; UNCOMPRESSED / FFOR / DELTA / RLE /
-dictionary pages per element width) it times candidate launch shapes -- threads per block, non-temporal stores,
+For every kernel family (raw streams per element width and bit width; UNCOMPRESSED / FFOR / DELTA / RLE / dictionary
+pages per element width, patched pages and RLE pages with plain positions of 32/64-bit values) it times candidate launch shapes -- threads per block, non-temporal stores,
 a cap on the grid (persistent blocks), direct stores for 32-bit values, and for narrow RLE pages the vectors per
 wavefront (one vector with one position lane per thread, or two with two) -- on the GPU and writes the fastest into a
 tuning table (`fastlanes_amd/tuning.txt` by default) that the library loads on first use. The row-group launch (family 6) is
@@ -22,7 +22,7 @@ import numpy as np
 import fastlanes_amd as fa
 from fastlanes_amd import workloads as wl
 
-FAM_STREAM, FAM_UNC, FAM_FFOR, FAM_DELTA, FAM_RLE, FAM_DICT, FAM_ROWGROUP = range(7)
+FAM_STREAM, FAM_UNC, FAM_FFOR, FAM_DELTA, FAM_RLE, FAM_DICT, FAM_ROWGROUP, FAM_PATCH, FAM_RLE_POS = range(9)
 RG_TILE_KIB = (16, 32, 64, 128)
 RG_CU_BLOCKS = (0, 8, 16, 32, 64, 128)  # 0 = resident blocks only (one long run per wave)
 BLOCKS = (128, 256, 512)
@@ -123,6 +123,12 @@ def main():
                 FAM_RLE: (6, wl.geometric_runs(m, 16.0, seed=1, value_bits=min(W - 1, 20)).astype(dt)),
                 FAM_DICT: (17, rng.integers(0, 1 << min(W - 1, 12), m).astype(dt)),
             }
+            if W >= 32:  # after FFOR and RLE, whose entries these fall back on
+                x = rng.integers(0, 1 << 7, m, dtype=dt)
+                hit = rng.random(m) < 0.01
+                x[hit] = rng.integers(0, np.iinfo(dt).max, int(hit.sum()), dtype=dt)
+                cases[FAM_PATCH] = (2, x)
+                cases[FAM_RLE_POS] = (7, cases[FAM_RLE][1])
             for fam, (eid, x) in cases.items():
                 enc = fa.encode_from_memory(x, eid)
                 plan = fa.Plan(enc, dt)

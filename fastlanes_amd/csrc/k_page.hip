@@ -42,11 +42,18 @@ Tune tune_for(int family, unsigned W, unsigned bw) {
     if (it != g_tune.end()) return it->second;
     it = g_tune.find({family, W, 255u});
     if (it != g_tune.end()) return it->second;
+    const int general = family == FAM_PAGE_PATCH ? FAM_PAGE_FFOR : family == FAM_PAGE_RLE_POS ? FAM_PAGE_RLE : -1;
+    if (general >= 0) {
+        it = g_tune.find({general, W, 255u});
+        if (it != g_tune.end()) return it->second;
+    }
     return Tune {};
 }
 void tune_set(int family, unsigned W, unsigned bw, Tune t) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune[{family, W, bw}] = t;
+    if (family == FAM_PAGE_FFOR) g_tune.erase({FAM_PAGE_PATCH, W, bw});
+    if (family == FAM_PAGE_RLE) g_tune.erase({FAM_PAGE_RLE_POS, W, bw});
 }
 int tune_load(const char* path) {
     FILE* f = std::fopen(path, "r");

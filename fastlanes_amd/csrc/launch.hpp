@@ -20,6 +20,9 @@ enum Family : int {
     FAM_PAGE_RLE,     // RLE pages (both variants)
     FAM_PAGE_DICT,    // dictionary pages (all variants)
     FAM_ROWGROUP,     // row-group launch: block = KiB of decoded values per tile, max_blocks = blocks per compute unit
+    FAM_PAGE_PATCH,   // patched FFOR-shaped pages (without an entry of their own: as FAM_PAGE_FFOR)
+    FAM_PAGE_RLE_POS, // RLE pages of 32/64-bit values with plain positions or differences of more than one bit (without an
+                      // entry of their own: as FAM_PAGE_RLE)
     FAM_COUNT
 };
 
@@ -31,6 +34,8 @@ struct Tune {
     uint32_t max_blocks = 0;
 };
 Tune tune_for(int family, unsigned W, unsigned bw);
+// Setting FAM_PAGE_FFOR or FAM_PAGE_RLE drops the width's entry of the family that falls back on it: it covers those pages
+// too until theirs is set again.
 void tune_set(int family, unsigned W, unsigned bw, Tune t);  // bw 255 = every bit width
 int  tune_load(const char* path);                             // returns entries read, <0 on error
 

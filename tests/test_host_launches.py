@@ -1,0 +1,56 @@
+"""What the host side launches and allocates, with a host-only HIP runtime: no GPU, no kernel runs."""
+import shutil
+
+import pytest
+
+from tests import host_hip
+
+pytestmark = pytest.mark.skipif(not shutil.which("/opt/rocm/bin/hipcc"), reason="needs hipcc")
+
+
+@pytest.fixture(scope="module")
+def hip(tmp_path_factory):
+    return host_hip.build(tmp_path_factory.mktemp("host_hip"))
+
+
+# A decode of 5000 vectors of 64-bit values by each expression: blocks of its last launch.
+GRIDS = """
+L = fa.lib()
+x = np.cumsum(np.random.default_rng(1).integers(0, 1000, 5000 * 1024)).astype(np.int64)
+x[::300] = 1 << 50
+plans = {}
+for e in EXPRS:
+    enc = fa.encode_from_memory(x if e != 7 else x >> 14, e)
+    plans[e] = fa.Plan(enc, x.dtype)
+    assert plans[e].n_pages == 1
+def grid(e, family=None, cap=0):
+    if family is not None:
+        fa.check(L.fls_gpu_tune_set(family, 64, 255, 64, 1, cap), "tune_set")
+    launches()
+    plans[e].decode(4096, 4096, x.nbytes)
+    return launches()[-1][1:3]
+"""
+
+
+def test_patched_pages_have_their_own_launch_shape(hip):
+    """Patched pages of 64-bit values take the shape that the table or a caller names for them (no cap of their own besides),
+    and follow an FFOR setting made after theirs, as before they had an entry."""
+    got = host_hip.run(hip, GRIDS.replace("EXPRS", "(1, 2, 4, 5, 12)") + """
+result = {"shipped": [grid(e) for e in (2, 4, 5, 12)], "ffor": grid(1)}
+result["own"] = [grid(e, 7, 0) for e in (2, 4, 5, 12)]
+result["ffor after own"] = grid(1)
+result["by ffor"] = [grid(e, 2, 700) for e in (2, 4, 5, 12)]
+""")
+    assert got["shipped"] == [[1024, 64]] * 4 and got["ffor"] == [2500, 128]
+    assert got["own"] == [[1250, 64]] * 4 and got["ffor after own"] == [2500, 128]
+    assert got["by ffor"] == [[700, 64]] * 4
+
+
+def test_plain_position_pages_have_their_own_launch_shape(hip):
+    """RLE pages of 64-bit values with plain positions, likewise."""
+    got = host_hip.run(hip, GRIDS.replace("EXPRS", "(6, 7)") + """
+result = {"shipped": [grid(6), grid(7)], "own": grid(7, 8, 300), "rle after own": grid(6), "by rle": grid(7, 4, 200)}
+""")
+    rle, pos = got["shipped"]
+    assert pos[0] == 512 and rle == [2500, 128]
+    assert got["own"][0] == 300 and got["rle after own"] == rle and got["by rle"][0] == 200
