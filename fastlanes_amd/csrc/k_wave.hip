@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_wave_rle(const uint8_t* __restric
         const uint8_t* rp = runs_of(m0);
         // the largest position of the lane before a u16 wrap, were there one
         const uint32_t top = m0.lb + 16 * base + (uint32_t)__builtin_popcount(w0);
-        const bool     plain = base == 0 && n <= 1024 && !__any(top > last);
+        const bool     plain = n && base == 0 && n <= 1024 && !__any(top > last);  // (n = 0: no position is in range)
         pair[lane] = m0.lb | w0 << 16;
         static_for<kRunsAhead>([&](auto k) {
             const uint32_t i = lane + 64 * decltype(k)::value;

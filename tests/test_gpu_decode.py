@@ -321,6 +321,30 @@ def test_wave_rle_pages(torch_cuda, oracle, W, form):
         assert lib.fls_gpu_tune_load(path.encode()) > 0
 
 
+@pytest.mark.parametrize("dtype", [np.uint32, np.uint64])
+def test_rle_vector_without_runs_is_reported(torch_cuda, dtype):
+    """A device copy whose second vector starts at the first run (the parser rejects that on the host): the first vector has
+    no run to read, and the decode and the predicate say so; the others keep their values."""
+    torch = torch_cuda
+    x = np.repeat(np.arange(3 * 64, dtype=dtype), 16) * dtype(7)
+    enc = fa.encode_from_memory(x, 6)
+    plan = fa.Plan(enc, dtype)
+    bad = enc.copy()
+    assert (int(bad[4]) | int(bad[5]) << 8) == 3 and bad[28:32].view(np.uint32)[0] == 64 * x.itemsize  # run values of vector 1
+    bad[28:32] = 0
+    d_in, d_out = dev(torch, bad), empty(torch, x.nbytes)
+    print(f"rle without runs {np.dtype(dtype)}", flush=True)
+    plan.decode(d_in.data_ptr(), d_out.data_ptr(), x.nbytes)
+    with pytest.raises(RuntimeError, match="out-of-range"):
+        plan.check()
+    np.testing.assert_array_equal(to_np(d_out, dtype, x.size)[2048:], x[2048:])
+    plan = fa.Plan(enc, dtype)
+    d_bits, d_counts = empty(torch, 3 * 128), empty(torch, 16)
+    plan.select(d_in.data_ptr(), "==", x[0], d_bits.data_ptr(), d_counts.data_ptr())
+    with pytest.raises(RuntimeError, match="out-of-range"):
+        plan.check()
+
+
 @pytest.mark.parametrize("W", [8, 16])
 def test_rle_two_lane_kernel(torch_cuda, oracle, W):
     """Tuning bit 2 of the RLE family switches narrow pages back to the two-lanes-per-thread kernel (the one that
