@@ -301,6 +301,11 @@ __global__ __launch_bounds__(kMaxBlock) void k_wave_rle(const uint8_t* __restric
 // 101 MB in), 76.6 us here; 60000 keys (from L2) 186 and 121 us; DELTA codes 158 and 117 us; 32768 vectors of int64 with
 // 2000 keys 99.8 and 61.0 us, with 40000 101.7 and 75 us; 2000 vectors of int32 10.7 and 7.0 us. What is left over a copy's
 // rate is the start of each page (metadata, rows and dictionary are loads that wait for each other).
+// A predicate takes the same lanes, whose bits are joined across the 8 or 16 lanes of a bitmap dword; a dictionary in LDS is
+// tested once as it is filled and holds outcomes instead of values. With a value per lane and a ballot per 64 of them, it
+// took longer than the form before on large pages: 16384 vectors of int32, 50 sorted keys, 13.9 us then, 21.4, 12.1 now (FFOR
+// codes; DELTA codes 15.5, 26.0, 13.9); 4096 Zipf keys 24.9, 24.8, 17.1; 30000 sorted keys (from L2, DELTA codes) 18.4, 22.1,
+// 17.8.
 template <unsigned G>
 __device__ __forceinline__ uint32_t group_scan(uint32_t x, unsigned lane) {  // inclusive, over groups of G lanes
     if constexpr (G == 32) return lane_scan<false>(x);
@@ -314,10 +319,21 @@ __device__ __forceinline__ uint32_t group_scan(uint32_t x, unsigned lane) {  // 
     return x;
 }
 
+// OR over groups of 8 or 16 lanes.
+template <unsigned G>
+__device__ __forceinline__ uint32_t group_or(uint32_t x) {
+    x |= __builtin_amdgcn_update_dpp(0u, x, 0xb1, 0xf, 0xf, false);   // quad_perm 1 0 3 2
+    x |= __builtin_amdgcn_update_dpp(0u, x, 0x4e, 0xf, 0xf, false);   // quad_perm 2 3 0 1
+    x |= __builtin_amdgcn_update_dpp(0u, x, 0x141, 0xf, 0xf, false);  // half mirror
+    if constexpr (G == 16) x |= __builtin_amdgcn_update_dpp(0u, x, 0x140, 0xf, 0xf, false);  // mirror
+    return x;
+}
+
 // A block decodes a dictionary's HZL chunks (no exceptions) into LDS, four values a thread at once: chunk headers, then
 // packed words, are two rounds of loads for 2048 values. Full chunks hold 1024 values and the raw tail follows them.
-template <typename D>
-__device__ __forceinline__ void fill_dict(const HzlSrc& hz, uint32_t dict_n, D* ldict) {
+// keep(v): what LDS keeps of value v.
+template <typename D, typename F>
+__device__ __forceinline__ void fill_dict(const HzlSrc& hz, uint32_t dict_n, D* ldict, F keep) {
     constexpr unsigned DW = 8 * sizeof(D), L = 1024 / DW;
     for (uint32_t b0 = 0; b0 < dict_n; b0 += 4 * blockDim.x) {
         D        lo[4], hi[4], base[4];
@@ -345,7 +361,7 @@ __device__ __forceinline__ void fill_dict(const HzlSrc& hz, uint32_t dict_n, D* 
             D v = bw[u] == 255 ? lo[u] : (D)((lo[u] >> sh[u]) | (sh[u] ? hi[u] << (DW - sh[u]) : (D)0));
             if (bw[u] < DW) v &= ((D)1 << bw[u]) - 1;
             if (bw[u] != 255) v += base[u];
-            if (b + threadIdx.x < dict_n) ldict[b + threadIdx.x] = v;
+            if (b + threadIdx.x < dict_n) ldict[b + threadIdx.x] = keep(v);
         });
     }
 }
@@ -358,7 +374,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_wave_dict(const uint8_t* __restri
     extern __shared__ __attribute__((aligned(16))) uint8_t fls_lds[];
     if (dict_n == 0) return;  // the host rejects such pages
     constexpr unsigned P  = VAR == 1 ? 0 : (VAR == 7 ? 3 : 2);
-    constexpr unsigned NV = SEL ? 1 : 16 / sizeof(T), IT = 16 / NV;  // values per lane and iteration, iterations
+    constexpr unsigned NV = 16 / sizeof(T), IT = 16 / NV;  // values per lane and iteration, iterations
+    constexpr unsigned GL = 32 / NV;                       // SEL: lanes that share a dword of the bitmap (at least IT)
     T* const ldict = reinterpret_cast<T*>(fls_lds);
     const unsigned lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     uint8_t* const lb   = fls_lds + dict_lds + wave * wave_lds;  // DELTA lane bases, then the rows
@@ -379,9 +396,10 @@ __global__ __launch_bounds__(kMaxBlock) void k_wave_dict(const uint8_t* __restri
     }
     if (v + stride < N) m1 = meta(v + stride);
     if constexpr (IN_LDS) {
-        if (hz.chunks) fill_dict(hz, dict_n, ldict);
+        auto keep = [&](T x) { return SEL ? (T)sel_pred<T, false>(x, sa) : x; };  // a predicate's outcome for each entry
+        if (hz.chunks) fill_dict(hz, dict_n, ldict, keep);
         else
-            for (uint32_t i = threadIdx.x; i < dict_n; i += blockDim.x) ldict[i] = dict[i];
+            for (uint32_t i = threadIdx.x; i < dict_n; i += blockDim.x) ldict[i] = keep(dict[i]);
         __syncthreads();
     }
     for (; v < N; v += stride) {
@@ -395,9 +413,8 @@ __global__ __launch_bounds__(kMaxBlock) void k_wave_dict(const uint8_t* __restri
         if (v + 2 * stride < N) m1 = meta(v + 2 * stride);
         wave_sync();
         const uint32_t mask = bw >= 32 ? ~0u : (1u << bw) - 1;
-        uint64_t       word = 0;
-        uint32_t       cnt  = 0;
-        const uint8_t* at[NV];  // the dword that the lane's first code e starts in; the next is a row further
+        uint32_t       word = 0;  // SEL: the bitmap's dword 2 NV (lane % GL) + lane / GL
+        const uint8_t* at[NV];    // the dword that the lane's first code e starts in; the next is a row further
         uint32_t       sh[NV];
         static_for<NV>([&](auto e) {
             const uint32_t bit = j_of_p<32>(p + decltype(e)::value) * bw;
@@ -422,16 +439,22 @@ __global__ __launch_bounds__(kMaxBlock) void k_wave_dict(const uint8_t* __restri
                 vals[e] = IN_LDS ? ldict[c[e]] : dict[c[e]];
             });
             if constexpr (SEL) {
-                const uint64_t b = __ballot(sizeof(T) == 8 && sa.dbl ? sel_pred<T, true>(vals[0], sa) : sel_pred<T, false>(vals[0], sa));
-                if (lane == decltype(k)::value) word = b;
-                cnt += (uint32_t)__popcll(b);
+                uint32_t b = 0;  // the lane's values' bits in their dword, then all of the dword
+                static_for<NV>([&](auto e) {
+                    b |= (IN_LDS ? (uint32_t)vals[e] : (uint32_t)in_range<T>(vals[e], sa)) << decltype(e)::value;
+                });
+                b = group_or<GL>(b << (NV * (lane % GL)));
+                if (lane % GL == decltype(k)::value) word = b;
             } else {
                 st16<NT>(out + v * (1024 * sizeof(T)) + 1024 * decltype(k)::value + 16 * lane, *reinterpret_cast<const v4u*>(vals));
             }
         });
         if constexpr (SEL) {
-            if (lane < 16) sa.bitmap[v * 16 + lane] = word;
-            if (lane == 0) sa.counts[v] = cnt;
+            if (!IN_LDS) word = sa.none ? 0u - (uint32_t)(sa.none_val != 0) : word ^ (0u - (uint32_t)(sa.inv != 0));
+            if (lane % GL >= IT) word = 0;
+            else reinterpret_cast<uint32_t*>(sa.bitmap)[v * 32 + 2 * NV * (lane % GL) + lane / GL] = word;
+            const uint32_t n = lane_scan<true>((uint32_t)__builtin_popcount(word));
+            if (lane == 63) sa.counts[v] = n;
         }
         wave_sync();
     }

@@ -113,6 +113,11 @@ struct SelArgs {
     uint32_t  inv, none, none_val, nan_val, dbl;
 };
 
+// The range test alone, without SelArgs' none and inv (integers).
+template <typename T>
+__device__ __forceinline__ bool in_range(T x, const SelArgs& sa) {
+    return (T)((T)(x ^ (T)sa.flip) - (T)sa.lo) <= (T)sa.span;
+}
 template <typename T, bool DBL>
 __device__ __forceinline__ bool sel_pred(T x, const SelArgs& sa) {
     if constexpr (DBL && sizeof(T) == 8) {
@@ -123,9 +128,7 @@ __device__ __forceinline__ bool sel_pred(T x, const SelArgs& sa) {
         const bool     in  = key - sa.lo <= sa.span;
         return sa.none ? sa.none_val != 0 : (in != (sa.inv != 0));
     } else {
-        const T    key = (T)(x ^ (T)sa.flip);
-        const bool in  = (T)(key - (T)sa.lo) <= (T)sa.span;
-        return sa.none ? sa.none_val != 0 : (in != (sa.inv != 0));
+        return sa.none ? sa.none_val != 0 : (in_range<T>(x, sa) != (sa.inv != 0));
     }
 }
 

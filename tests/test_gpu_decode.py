@@ -721,6 +721,34 @@ def test_dictionary_sizes(torch_cuda, oracle, dtype, n_keys):
         np.testing.assert_array_equal(d_cnt.cpu().numpy(), (want > c).reshape(-1, 1024).sum(axis=1))
 
 
+@pytest.mark.parametrize("dtype", [np.uint32, np.int32, np.uint64, np.int64])
+@pytest.mark.parametrize("n_keys", [900, 20000])
+def test_dictionary_predicates(torch_cuda, oracle, dtype, n_keys):
+    """Every operator, with constants inside the dictionary and at the ends of the type (where the outcome is the same for all
+    values), on a dictionary in LDS and on one that is not; plain, FFOR and DELTA codes."""
+    torch = torch_cuda
+    g = np.random.default_rng(n_keys)
+    info = np.iinfo(dtype)
+    keys = g.permutation(np.unique(np.append(g.integers(info.min, info.max, n_keys, dtype=dtype, endpoint=True),
+                                             np.array([info.min, info.max], dtype))))
+    x = np.concatenate([keys, keys[g.integers(0, keys.size, 9 * 1024 + -keys.size % 1024)]])
+    n_vec = x.size // 1024
+    d_bm = torch.zeros(16 * n_vec, dtype=torch.int64, device="cuda")
+    d_cnt = torch.zeros(n_vec, dtype=torch.int32, device="cuda")
+    for eid in (16, 17, 22):
+        enc = oracle.encode_column(x, eid)
+        y = oracle.decode_column(enc, dtype, x.size)
+        plan, d_in = fa.Plan(enc, dtype), dev(torch, enc)
+        print(f"dictionary predicates {np.dtype(dtype).name} keys={keys.size} expr={eid}", flush=True)
+        for op, fn in PRED.items():
+            for c in (dtype(info.min), dtype(info.max), x[5]):
+                d_bm.fill_(-1), d_cnt.fill_(-1)
+                plan.select(d_in.data_ptr(), op, c, d_bm.data_ptr(), d_cnt.data_ptr())
+                np.testing.assert_array_equal(d_bm.cpu().numpy().view(np.uint64), _bitmap_words(fn(y, c)), err_msg=f"{eid} {op} {c}")
+                np.testing.assert_array_equal(d_cnt.cpu().numpy(), fn(y, c).reshape(-1, 1024).sum(axis=1))
+        plan.check()
+
+
 def _bitmap_words(mask: np.ndarray) -> np.ndarray:
     """SelectionDS bitmap words of a boolean mask: per 1024 values, 16 uint64 words, bit i of word j = value 64j+i."""
     bits = np.packbits(mask.reshape(-1, 64), axis=1, bitorder="little")
