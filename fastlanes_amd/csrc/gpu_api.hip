@@ -139,7 +139,7 @@ hipError_t page_launch(fls_gpu_plan* plan, size_t i, const uint8_t* dev_encoded,
     const unsigned   W    = plan->W;
     const uint8_t*   page = dev_encoded + pe.page_off;
     DevDict&         d    = plan->dicts[i];
-    PageMeta         pm {};
+    WaveMeta         pm {};
     for (unsigned b = 0; b < pe.arr_c && b < 6; ++b) pm.off[b] = pe.boff[b];
     pm.arr_c = pe.arr_c, pm.fixed = pe.fixed_meta, pm.bw_max = pe.bw_max;
     if (!pe.vec_c) return hipSuccess;

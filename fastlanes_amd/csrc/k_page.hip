@@ -74,7 +74,7 @@ int tune_load(const char* path) {
     return n;
 }
 
-hipError_t launch_page_int(unsigned W, int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
+hipError_t launch_page_int(unsigned W, int mode, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c, uint8_t* out,
                            hipStream_t s, const SelArgs* sel) {
     if (!vec_c) return hipSuccess;
     switch (W) {
@@ -138,7 +138,7 @@ hipError_t launch_drle_values(unsigned W, const uint32_t* codes, uint64_t n, con
     return hipGetLastError();
 }
 
-hipError_t launch_page_dict(unsigned W, int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c,
+hipError_t launch_page_dict(unsigned W, int var, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c,
                             const void* dict, uint32_t dict_n, uint8_t* out, uint32_t* err, hipStream_t s,
                             const SelArgs* sel, const HzlSrc* hz) {
     if (!vec_c) return hipSuccess;

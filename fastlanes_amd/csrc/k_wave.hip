@@ -82,7 +82,7 @@ __host__ __device__ constexpr unsigned rle_wave_lds(unsigned value_bytes) { retu
 // MODE 0 UNCOMPRESSED, 1 FFOR, 2 DELTA, as k_page_int. SEL: a predicate's bitmap instead of values; iteration k, lane l
 // then holds value 64 k + l alone, so that a ballot is the bitmap's word k.
 template <int MODE, bool NT, bool SEL>
-__global__ __launch_bounds__(kMaxBlock) void k_wave_int64(const uint8_t* __restrict__ page, PageMeta pm, uint32_t vec_c,
+__global__ __launch_bounds__(kMaxBlock) void k_wave_int64(const uint8_t* __restrict__ page, WaveMeta pm, uint32_t vec_c,
                                                           uint8_t* __restrict__ out, SelArgs sa, uint32_t wave_lds) {
     extern __shared__ __attribute__((aligned(16))) uint8_t fls_lds[];
     constexpr unsigned P  = MODE == 0 ? 0 : (MODE == 2 ? 3 : 2);
@@ -367,7 +367,7 @@ __device__ __forceinline__ void fill_dict(const HzlSrc& hz, uint32_t dict_n, D* 
 }
 
 template <typename T, int VAR, bool NT, bool IN_LDS, bool SEL>
-__global__ __launch_bounds__(kMaxBlock) void k_wave_dict(const uint8_t* __restrict__ page, PageMeta pm, uint32_t vec_c,
+__global__ __launch_bounds__(kMaxBlock) void k_wave_dict(const uint8_t* __restrict__ page, WaveMeta pm, uint32_t vec_c,
                                                          const T* __restrict__ dict, uint32_t dict_n,
                                                          uint8_t* __restrict__ out, uint32_t* err, SelArgs sa, HzlSrc hz,
                                                          uint32_t dict_lds, uint32_t wave_lds) {
@@ -463,7 +463,7 @@ __global__ __launch_bounds__(kMaxBlock) void k_wave_dict(const uint8_t* __restri
 
 }  // namespace
 
-hipError_t page_int64_wave(int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
+hipError_t page_int64_wave(int mode, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c, uint8_t* out,
                            const SelArgs* sel, hipStream_t s) {
     Tune           t  = tune_for(mode == 0 ? FAM_PAGE_UNC : mode == 1 ? FAM_PAGE_FFOR : FAM_PAGE_DELTA, 64, 255);
     const unsigned bw = mode == 0 ? 64u : pm.bw_max ? pm.bw_max : 1u;
@@ -514,7 +514,7 @@ hipError_t page_rle_wave(unsigned W, const uint8_t* page, const PageMeta& pm, ui
 }
 
 template <typename T>
-static hipError_t dict_wave(int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, const void* dict, uint32_t dict_n,
+static hipError_t dict_wave(int var, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c, const void* dict, uint32_t dict_n,
                             uint8_t* out, uint32_t* err, const SelArgs* sel, const HzlSrc* hz, hipStream_t s) {
     const T*       d  = static_cast<const T*>(dict);
     Tune           t  = tune_for(FAM_PAGE_DICT, 8 * sizeof(T), 255);
@@ -569,7 +569,7 @@ static hipError_t dict_wave(int var, const uint8_t* page, const PageMeta& pm, ui
 #undef L
     return hipGetLastError();
 }
-hipError_t page_dict_wave(unsigned W, int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, const void* dict,
+hipError_t page_dict_wave(unsigned W, int var, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c, const void* dict,
                           uint32_t dict_n, uint8_t* out, uint32_t* err, const SelArgs* sel, const HzlSrc* hz, hipStream_t s) {
     return W == 64 ? dict_wave<uint64_t>(var, page, pm, vec_c, dict, dict_n, out, err, sel, hz, s)
                    : dict_wave<uint32_t>(var, page, pm, vec_c, dict, dict_n, out, err, sel, hz, s);

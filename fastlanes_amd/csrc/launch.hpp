@@ -7,6 +7,7 @@ namespace fls {
 
 struct HzlChunk;
 struct PageMeta;
+struct WaveMeta;
 struct SelArgs;
 struct HzlSrc;
 struct RunSrc;
@@ -49,7 +50,7 @@ inline unsigned grid_for(uint64_t n_vec, const Tune& t, unsigned tpv) {
 
 hipError_t launch_unffor_stream(unsigned W, unsigned bw, const uint8_t* packed, const void* bases, uint8_t* out,
                                 uint64_t n_vec, hipStream_t s);
-hipError_t launch_page_int(unsigned W, int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
+hipError_t launch_page_int(unsigned W, int mode, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c, uint8_t* out,
                            hipStream_t s, const SelArgs* sel = nullptr);
 // runs: where the run values are (DICT_RLE pages, chained run values); nullptr: the page's buffer 0.
 // pos_bw1: every vector's DELTA positions have bit width 0 or 1 (8/16-bit values then take the one-lane-per-thread
@@ -66,7 +67,7 @@ hipError_t launch_drle_fused(unsigned W, const uint8_t* enc, const HzlChunk* run
                              hipStream_t s);
 // hz: the page's HZL dictionary payload; the launcher decodes it into `dict` (or, when it fits LDS, lets the page
 // kernel decode it per block). nullptr: `dict` already holds the decoded dictionary.
-hipError_t launch_page_dict(unsigned W, int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c,
+hipError_t launch_page_dict(unsigned W, int var, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c,
                             const void* dict, uint32_t dict_n, uint8_t* out, uint32_t* err, hipStream_t s,
                             const SelArgs* sel = nullptr, const HzlSrc* hz = nullptr);
 // Patched FFOR-shaped pages. var: patch kind in FFOR numbering (2 LL_PATCH, 3 S_PATCH, 4 B_PATCH); rsum: lane bases
@@ -84,11 +85,11 @@ template <int W>
 hipError_t page_int_w(int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
                       const SelArgs* sel, hipStream_t s);
 // integer pages of 64-bit values (k_wave.hip)
-hipError_t page_int64_wave(int mode, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out,
+hipError_t page_int64_wave(int mode, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c, uint8_t* out,
                            const SelArgs* sel, hipStream_t s);
 hipError_t page_rle_wave(unsigned W, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, uint8_t* out, uint32_t* err,
                          const SelArgs* sel, const RunSrc* runs, hipStream_t s);  // W 32/64, positions of bit width <= 1
-hipError_t page_dict_wave(unsigned W, int var, const uint8_t* page, const PageMeta& pm, uint32_t vec_c, const void* dict,
+hipError_t page_dict_wave(unsigned W, int var, const uint8_t* page, const WaveMeta& pm, uint32_t vec_c, const void* dict,
                           uint32_t dict_n, uint8_t* out, uint32_t* err, const SelArgs* sel, const HzlSrc* hz, hipStream_t s);
 template <int W>
 hipError_t page_patch_w(int var, bool rsum, const void* dict, uint32_t dict_n, const uint8_t* page, const PageMeta& pm,
