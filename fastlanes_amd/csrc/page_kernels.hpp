@@ -1112,8 +1112,26 @@ __global__ __launch_bounds__(kMaxBlock) void k_page_dict(const uint8_t* __restri
 // loads instead of a serial walk over its rows. Output in array order: out[j * L + lane] = value + base.
 template <typename D>
 __device__ __forceinline__ void hzl_chunk(const uint8_t* in, const HzlChunk& ch, D* out) {
-    const uint32_t n = ch.bw == 255 ? ch.n : 1024u;
-    for (uint32_t k = threadIdx.x; k < n; k += blockDim.x) out[k] = hzl_value<D>(in, ch, k);
+    constexpr unsigned DW = 8 * sizeof(D), L = 1024 / DW;
+    if (ch.bw == 255) {
+        for (uint32_t k = threadIdx.x; k < ch.n; k += blockDim.x) out[k] = load_t<D>(in + (uint64_t)k * sizeof(D));
+        return;
+    }
+    // hzl_value's steps with everything of the chunk taken out of the loop
+    const unsigned bw   = ch.bw;
+    const D        base = (D)ch.base;
+    const D        mask = bw >= DW ? (D)~(D)0 : (D)(((D)1 << bw) - 1);
+    for (uint32_t k = threadIdx.x; k < 1024; k += blockDim.x) {
+        const unsigned j = k / L, lane = k % L;
+        D              v = 0;
+        if (bw) {
+            const unsigned bit = j * bw, w = bit / DW, sh = bit % DW;
+            v                  = load_t<D>(in + ((uint64_t)w * L + lane) * sizeof(D)) >> sh;
+            if (sh + bw > DW) v |= load_t<D>(in + ((uint64_t)(w + 1) * L + lane) * sizeof(D)) << (DW - sh);
+            v &= mask;
+        }
+        out[k] = (D)(v + base);
+    }
 }
 template <int DW>
 __global__ __launch_bounds__(1024) void k_hzl_chunks(const uint8_t* __restrict__ enc, const HzlChunk* chunks,
@@ -1121,7 +1139,7 @@ __global__ __launch_bounds__(1024) void k_hzl_chunks(const uint8_t* __restrict__
     using D = typename uint_of<DW>::type;
     for (uint32_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
         const HzlChunk ch = chunks[c];
-        hzl_chunk<D>(enc + ch.src, ch, reinterpret_cast<D*>(dict) + ch.dst);
+        hzl_chunk<D>(enc + ch.src, ch, reinterpret_cast<D*>(dict + ch.dst * sizeof(D)));
     }
 }
 // Exceptions of an FFOR chunk: positions (u16), then values, behind its packed rows.
