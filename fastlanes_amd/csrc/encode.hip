@@ -667,30 +667,35 @@ static __device__ __align__(256) uint8_t scratch[fls::kEncFixedBytes];
 static __device__ __align__(256) uint8_t enc_slots[fls::kEncSlots * fls::kEncSlotBytes];
 
 namespace {
-// A device's scratch addresses, looked up once with that device current, and its slots' owners. Each slot, and the
-// allocation-free encoder, has a place in pinned host memory that the layout kernel writes the total to (a copy back
-// of 16 bytes takes 10 us longer).
+// A device's scratch addresses, looked up once with that device current, and its slots' owners. Each slot has a place in
+// pinned host memory that the layout kernel writes the total to (a copy back of 16 bytes takes 10 us longer); the
+// allocation-free encoder has none, because pinned memory is an allocation.
 struct EncDevice {
     uint8_t  *fixed = nullptr, *slots = nullptr;
-    EncTotal* totals = nullptr;  // kEncSlots + 1
+    EncTotal* totals = nullptr;  // kEncSlots
     unsigned  taken  = 0;        // bit k: slot k
 };
 std::mutex             g_enc_mu;
 std::vector<EncDevice> g_enc_dev;
 
-int enc_device(int& dev) {
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) return hip_fail(e, "hipGetDevice");
+int enc_device(int dev, bool noalloc) {
+    hipError_t                  e = hipSuccess;
     std::lock_guard<std::mutex> lock(g_enc_mu);
     if ((size_t)dev >= g_enc_dev.size()) g_enc_dev.resize(dev + 1);
     EncDevice& d = g_enc_dev[dev];
+    void*      p = nullptr;
+    if (noalloc) {
+        if (d.fixed) return FLS_OK;
+        if ((e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch))) != hipSuccess) return hip_fail(e, "hipGetSymbolAddress");
+        d.fixed = static_cast<uint8_t*>(p);
+        return FLS_OK;
+    }
     if (d.totals) return FLS_OK;
-    void *f = nullptr, *q = nullptr, *t = nullptr;
-    if ((e = hipGetSymbolAddress(&f, HIP_SYMBOL(scratch))) != hipSuccess) return hip_fail(e, "hipGetSymbolAddress");
-    if ((e = hipGetSymbolAddress(&q, HIP_SYMBOL(enc_slots))) != hipSuccess) return hip_fail(e, "hipGetSymbolAddress");
-    if ((e = hipHostMalloc(&t, sizeof(EncTotal) * (kEncSlots + 1), hipHostMallocPortable | hipHostMallocMapped)) != hipSuccess)
+    if ((e = hipGetSymbolAddress(&p, HIP_SYMBOL(enc_slots))) != hipSuccess) return hip_fail(e, "hipGetSymbolAddress");
+    d.slots = static_cast<uint8_t*>(p);
+    if ((e = hipHostMalloc(&p, sizeof(EncTotal) * kEncSlots, hipHostMallocPortable | hipHostMallocMapped)) != hipSuccess)
         return hip_fail(e, "hipHostMalloc");
-    d.fixed = static_cast<uint8_t*>(f), d.slots = static_cast<uint8_t*>(q), d.totals = static_cast<EncTotal*>(t);
+    d.totals = static_cast<EncTotal*>(p);
     return FLS_OK;
 }
 
@@ -727,7 +732,8 @@ int encode_impl(const void* dev_values, uint64_t n, enum data_t type, uint8_t ex
         return err == hipSuccess ? FLS_OK : hip_fail(err, "hipMemcpyAsync");
     }
     int dev = 0;
-    if (int rc = enc_device(dev)) return rc;
+    if ((err = hipGetDevice(&dev)) != hipSuccess) return hip_fail(err, "hipGetDevice");
+    if (int rc = enc_device(dev, noalloc)) return rc;
     uint8_t*  d     = nullptr;
     EncTotal* total = nullptr;  // pinned host memory
     unsigned  slot  = kEncSlots;
@@ -735,7 +741,7 @@ int encode_impl(const void* dev_values, uint64_t n, enum data_t type, uint8_t ex
         std::lock_guard<std::mutex> lock(g_enc_mu);
         EncDevice&                  ed = g_enc_dev[dev];
         if (noalloc) {
-            d = ed.fixed, total = ed.totals + kEncSlots;
+            d = ed.fixed;
         } else if (n_vec <= kEncSlotVec) {
             for (slot = 0; slot < kEncSlots && (ed.taken >> slot & 1u);) ++slot;
             if (slot < kEncSlots) ed.taken |= 1u << slot, d = ed.slots + slot * kEncSlotBytes, total = ed.totals + slot;
@@ -752,7 +758,7 @@ int encode_impl(const void* dev_values, uint64_t n, enum data_t type, uint8_t ex
     const uint64_t page_c = (n_vec + kMaxVecPerPage - 1) / kMaxVecPerPage;
     EncTotal       copy {};
     err = launch_enc_w(W, a, dev_values, type == INT64, (uint32_t)((n_vec + page_c - 1) / page_c), dev_out, s);
-    if (own && err == hipSuccess) err = hipMemcpyAsync(&copy, a.total, sizeof copy, hipMemcpyDeviceToHost, s);
+    if (!total && err == hipSuccess) err = hipMemcpyAsync(&copy, a.total, sizeof copy, hipMemcpyDeviceToHost, s);
     if (own) (void)hipFreeAsync(d, s);
     const hipError_t done = hipStreamSynchronize(s);
     if (err == hipSuccess) err = done;

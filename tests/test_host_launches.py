@@ -54,3 +54,25 @@ result = {"shipped": [grid(6), grid(7)], "own": grid(7, 8, 300), "rle after own"
     rle, pos = got["shipped"]
     assert pos[0] == 512 and rle == [2500, 128]
     assert got["own"][0] == 300 and got["rle after own"] == rle and got["by rle"][0] == 200
+
+
+ENCODE = """
+L = fa.lib()
+size = C.c_uint64()
+def encode(fn, n_vec, stream=0):
+    calls()
+    fa.check(getattr(L, fn)(4096, n_vec * 1024, 8, 1, 4096, 1 << 40, C.byref(size), stream), fn)
+    return calls()
+def current():
+    d = C.c_int(-1)
+    _h.hipGetDevice(C.byref(d))
+    return d.value
+"""
+
+
+def test_allocation_free_encoder_allocates_nothing(hip):
+    """fls_gpu_encode_noalloc neither allocates device memory nor pins host memory, on its first call either."""
+    got = host_hip.run(hip, ENCODE + """
+result = [sorted({c[0] for c in encode("fls_gpu_encode_noalloc", n)}) for n in (1, 16384)]
+""")
+    assert got == [["launch", "symbol_on"], ["launch"]]
