@@ -699,6 +699,23 @@ int enc_device(int dev, bool noalloc) {
     return FLS_OK;
 }
 
+// The stream's device, made current for as long as this lives: the scratch and the kernels belong to it, whichever device
+// the caller has current (the null stream is that one's).
+struct StreamDevice {
+    int        dev = 0, before = 0;
+    hipError_t err;
+    explicit StreamDevice(hipStream_t s) {
+        if ((err = hipGetDevice(&before)) != hipSuccess) return;
+        dev = before;
+        hipDevice_t d = (hipDevice_t)before;
+        if (s && hipStreamGetDevice(s, &d) != hipSuccess) (void)hipGetLastError(), d = (hipDevice_t)before;
+        if ((int)d != before && (err = hipSetDevice((int)d)) == hipSuccess) dev = (int)d;
+    }
+    ~StreamDevice() {
+        if (dev != before) (void)hipSetDevice(before);
+    }
+};
+
 // `noalloc`: the fixed scratch (at most kEncFixedVec vectors); otherwise a slot, or a stream allocation for larger
 // columns and when the slots are taken.
 int encode_impl(const void* dev_values, uint64_t n, enum data_t type, uint8_t expr_id, uint8_t* dev_out,
@@ -731,8 +748,9 @@ int encode_impl(const void* dev_values, uint64_t n, enum data_t type, uint8_t ex
         if (err == hipSuccess) err = hipStreamSynchronize(s);
         return err == hipSuccess ? FLS_OK : hip_fail(err, "hipMemcpyAsync");
     }
-    int dev = 0;
-    if ((err = hipGetDevice(&dev)) != hipSuccess) return hip_fail(err, "hipGetDevice");
+    const StreamDevice on(s);
+    if (on.err != hipSuccess) return hip_fail(on.err, "stream device");
+    const int dev = on.dev;
     if (int rc = enc_device(dev, noalloc)) return rc;
     uint8_t*  d     = nullptr;
     EncTotal* total = nullptr;  // pinned host memory

@@ -76,3 +76,16 @@ def test_allocation_free_encoder_allocates_nothing(hip):
 result = [sorted({c[0] for c in encode("fls_gpu_encode_noalloc", n)}) for n in (1, 16384)]
 """)
     assert got == [["launch", "symbol_on"], ["launch"]]
+
+
+def test_encoder_scratch_is_on_the_streams_device(hip):
+    """A stream of another device than the current one (0x201: device 2): its scratch and kernels are that device's, from the
+    fixed scratch, a slot, or the stream's allocator; the current device stays what it was."""
+    got = host_hip.run(hip, ENCODE + """
+result = []
+for fn, n in (("fls_gpu_encode_noalloc", 64), ("fls_gpu_encode", 64), ("fls_gpu_encode", 1 << 20)):
+    c = encode(fn, n, 0x201)
+    where = {int(x[1]) for x in c if x[0] in ("symbol_on", "malloc_async_on")} | {int(x[1].split()[-1]) for x in c if x[0] == "launch"}
+    result.append([sorted(where), current()])
+""")
+    assert got == [[[2], 0]] * 3
