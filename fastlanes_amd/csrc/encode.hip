@@ -654,9 +654,11 @@ constexpr EncScratch enc_scratch(uint64_t n_vec) {
     return l;
 }
 constexpr size_t kEncFixedBytes = enc_scratch(kEncFixedVec).size;
-// Scratch kept for fls_gpu_encode calls of up to kEncSlotVec vectors (2^26 values): a stream allocation and its release
-// cost a call 20 us, more than its kernels for a small column. A call holds a slot until its stream has completed.
-constexpr uint64_t kEncSlotVec   = 65536;
+// Scratch kept for fls_gpu_encode calls of up to kEncSlotVec vectors (2^28 values): a stream allocation, its release and the
+// copy of the total cost a call 25 to 45 us, more than its kernels for a small column and a tenth of them at this size (uint32
+// FFOR, 490 us, 538 one vector further; 65537 vectors 147 us while slots ended at 65536, 122 now). 2.5 MB a slot; past it
+// the share shrinks with the memory growing. A call holds a slot until its stream has completed.
+constexpr uint64_t kEncSlotVec   = 262144;
 constexpr size_t   kEncSlotBytes = enc_scratch(kEncSlotVec).size;
 constexpr unsigned kEncSlots     = 4;
 }  // namespace fls
