@@ -18,7 +18,9 @@
 // same-address atomic per segment) and waits took 48 of 135 us for 2^21 strings of 36 bytes. Every symbol was OR-ed into
 // a zeroed image by an LDS atomic; now a word is stored by the one thread that has its last byte, and threads that have
 // only earlier bytes of it OR them in after a barrier. (Writing each symbol's 8 bytes at its own unaligned place, two
-// instructions per code, measured 135 us: unaligned LDS writes take about one cycle per lane.) 2^21 strings: 151 -> 71 us
+// instructions per code, measured 135 us: unaligned LDS writes take about one cycle per lane.) Escapes are found from two
+// 32-bit masks of a granule, its bytes of 255 and the strings' ends in it; while every thread looked its ends up and walked
+// its escapes, a column with 3% of its bytes escaped took 102 us where it now takes 85. 2^21 strings: 151 -> 71 us
 // a call, k_fsst 42, bound by its vector instructions. No variable of k_fsst may spill: a build whose registers did gave
 // wrong bytes in a hundredth of the segments.
 // A vector with a malformed segment (non-monotone offsets) takes a per-string path that reads and writes global memory byte
@@ -90,13 +92,21 @@ __device__ __forceinline__ void load_granule(const uint8_t* p, uint32_t avail, u
         });
     }
 }
+// 0x80 in every byte of w that is 255.
+__device__ __forceinline__ uint32_t ff_bytes(uint32_t w) { return ((w & 0x7f7f7f7fu) + 0x01010101u) & w & 0x80808080u; }
 __device__ __forceinline__ bool has_ff(const uint32_t (&wd)[8]) {
     uint32_t z = 0;
-    static_for<8>([&](auto d) {
-        const uint32_t n = ~wd[d.value];
-        z |= (n - 0x01010101u) & ~n & 0x80808080u;  // a zero byte of ~w: an 0xFF byte of w
-    });
+    static_for<8>([&](auto d) { z |= ff_bytes(wd[d.value]); });
     return z != 0;
+}
+// Bit j: byte j of the granule is 255.
+__device__ __forceinline__ uint32_t ff_mask(const uint32_t (&wd)[8]) {
+    uint32_t ff = 0;
+    static_for<8>([&](auto D) {
+        constexpr unsigned d = decltype(D)::value;
+        ff |= (__builtin_amdgcn_udot4(ff_bytes(wd[d]), 0x08040201u, 0u, false) >> 7) << (4 * d);
+    });
+    return ff;
 }
 template <unsigned J>
 __device__ __forceinline__ uint32_t byte_of(const uint32_t (&wd)[8]) {
@@ -109,7 +119,7 @@ struct FsstSeg {
     uint64_t total, before;
     uint32_t s0, n;
 };
-constexpr uint64_t kMalformed = 1ull << 63;
+constexpr uint64_t kMalformed = 1ull << 63, kEscapes = 1ull << 62;  // in `before`; kEscapes: some granule is kSpecial
 
 // A segment's compressed bytes `seg`, n of them, and the ends of its strings (LDS, from its start).
 struct Segment {
@@ -123,7 +133,8 @@ struct Segment {
 __device__ __forceinline__ uint64_t sizes_at(uint64_t page_off, const uint8_t* page, const uint8_t* bytes, uint64_t seg) {
     return (page_off + (uint64_t)(bytes - page)) / kShare + seg;
 }
-constexpr uint32_t kSpecial = 0x8000;  // in d_sizes: the granule holds, or starts with, part of an escape
+// In d_sizes: the granule holds, or starts with, part of an escape; its first byte is an escape's literal.
+constexpr uint32_t kSpecial = 0x8000, kLiteral = 0x4000, kSize = kLiteral - 1;
 
 // A thread's granule of the chunk at c0: its bytes (0 past the segment), its place in the segment, how many bytes the
 // segment has there.
@@ -145,44 +156,72 @@ __device__ __forceinline__ Granule open_granule(const Segment& g, uint32_t c0, u
 
 // Bit k of m as byte k, 0 or 255.
 __device__ __forceinline__ uint32_t spread4(uint32_t m) { return (((m & 15u) * 0x00204081u) & 0x01010101u) * 255u; }
-// Number of strings of the segment that end at or before p (the ends are sorted).
-__device__ __forceinline__ uint32_t ends_upto(const uint32_t* end, uint32_t p) {
-    uint32_t lo = 0;
-    for (uint32_t step = kSeg / 2; step; step /= 2)
-        if (end[lo + step - 1] <= p) lo += step;
-    return lo + (end[lo] <= p ? 1u : 0u);
-}
 // Escapes of a granule, bit j for its byte j: `esc` the escapes that emit the byte after them (one whose string ends
 // right after it emits 0), `none` the bytes that emit nothing (literals, and bytes past the segment).
 struct Escapes {
     uint32_t esc, none;
 };
-__device__ __forceinline__ Escapes find_escapes(const Segment& g, const Granule& r) {
-    Escapes  x {0, r.lim >= kShare ? 0u : ~0u << r.lim};
-    uint32_t ff = 0;
-    static_for<32>([&](auto J) { ff |= ((byte_of<decltype(J)::value>(r.wd) + 1u) >> 8) << decltype(J)::value; });
-    ff &= ~x.none;
-    uint64_t lit = 0;  // literals; bit 32: the byte after the granule
-    uint32_t k   = ends_upto(g.end, r.q0);  // the first string that ends past q0
-    if (r.q0 && g.seg[r.q0 - 1] == 255 && !(k && g.end[k - 1] == r.q0)) {
-        // the granule starts on a literal when the run of 255 bytes before it has an odd length inside its string (a
-        // run begins with an escape code: after a code or a literal comes a code)
-        const uint32_t start = k ? g.end[k - 1] : 0u;
-        uint32_t       p     = r.q0 - 1;
-        while (p > start && g.seg[p - 1] == 255) --p;
-        lit = (r.q0 - p) & 1u;
+// Where strings end in a granule: bit j of `before`, right before its byte j; `after`, right after its last byte.
+struct Ends {
+    uint32_t before;
+    bool     after;
+};
+// ff: the bytes that are 255; literal: the first byte is one. Inside a string every second byte of a run of 255 is a literal
+// (a run begins with an escape code: after a code or a literal comes a code). Which bytes lie at an even distance from their
+// run's start is the parity of the last start at or before them, spread upwards in five steps.
+__device__ __forceinline__ Escapes find_escapes(uint32_t ff, const Ends& e, uint32_t lim, bool literal) {
+    const uint32_t past = lim >= kShare ? 0u : ~0u << lim, in = literal, f = ff & ~past & ~in;
+    const uint32_t starts = f & (~(f << 1) | e.before);
+    uint32_t       even = starts & 0x55555555u, open = ~starts;
+    for (unsigned d = 1; d < 32; d *= 2) {
+        even |= open & (even << d);
+        open &= open << d;
     }
-    // the escapes and the ends in the granule are both in order: one walk over them
-    uint32_t e = k < kSeg ? g.end[k] : ~0u;
-    while (ff) {
-        const uint32_t j = (uint32_t)__builtin_ctz(ff), p = r.q0 + j + 1;
-        ff &= ff - 1;
-        if ((lit >> j) & 1u) continue;
-        while (e < p) e = ++k < kSeg ? g.end[k] : ~0u;
-        if (e != p) x.esc |= 1u << j, lit |= 2ull << j;
+    const uint32_t codes = f & ~(even ^ 0x55555555u);
+    return {codes & ~(e.before >> 1 | (uint32_t)e.after << 31), ((codes << 1 | in) & ~e.before) | past};
+}
+// What a granule (a whole one) says of the byte after it: `lit`, that it is a literal (the run of 255 before it, inside its
+// string, is of odd length); `keeps`, that it is one if the granule's own first byte is: a granule of nothing but 255
+// inside one string, because 32 is even.
+struct After {
+    bool lit, keeps;
+};
+__device__ __forceinline__ After after_granule(uint32_t ff, const Ends& e) {
+    const uint32_t run = ff == ~0u ? 32u : (uint32_t)__builtin_clz(~ff);
+    const uint32_t own = e.before ? (uint32_t)__builtin_clz(e.before) + 1 : 32u;  // bytes of the granule in its last string
+    return {!e.after && ((run < own ? run : own) & 1u) != 0, run == 32 && !e.before && !e.after};
+}
+// The ends in granule i + lane, by a whole wave; bits: kEndWords words of LDS of its own.
+constexpr unsigned kEndWords = 65;
+__device__ __forceinline__ Ends window_ends(const uint32_t* end, uint32_t i, unsigned lane, uint32_t* bits) {
+    wave_sync();  // the last window's have been read
+    bits[lane] = 0u;
+    if (lane == 0) bits[64] = 0u;
+    wave_sync();
+    static_for<kSeg / 64>([&](auto k) {
+        const uint32_t at = end[lane + 64 * decltype(k)::value] - i * kShare;
+        if (at <= 64 * kShare) atomicOr(&bits[at / kShare], 1u << (at % kShare));
+    });
+    wave_sync();
+    return {bits[lane], (bits[lane + 1] & 1u) != 0};
+}
+// Whether granule `at` (not the first) starts on a literal, by a whole wave: 64 granules back at a time until one says so.
+__device__ __forceinline__ bool starts_on_literal(const Segment& g, uint32_t at, unsigned lane, uint32_t* bits) {
+    if (g.seg[at * kShare - 1] != 255) return false;
+    while (at) {
+        const uint32_t n = at < 64 ? at : 64, i = at - n;
+        const Ends     e = window_ends(g.end, i, lane, bits);
+        After          a {false, true};
+        if (lane < n) {
+            uint32_t wd[8];
+            load_granule(g.seg + (i + lane) * kShare, kShare, wd);
+            a = after_granule(ff_mask(wd), e);
+        }
+        const uint64_t says = __ballot(!a.keeps);
+        if (says) return (__ballot(a.lit) >> (63 - __builtin_clzll(says))) & 1u;
+        at = i;
     }
-    x.none |= (uint32_t)lit;
-    return x;
+    return false;  // the segment's first byte is a code
 }
 
 // Values the compiler cannot carry over from before: it would take the table addresses out of all forms of emit_granule,
@@ -316,7 +355,7 @@ __global__ __launch_bounds__(kSeg* GROUPS, 8) void k_fsst_count(const uint8_t* _
     __shared__ uint8_t  len[256];
     __shared__ uint32_t ends[8 * kEndRow], end[1024];  // transposed from the vector's start, then in order from the segment's
     __shared__ uint64_t wsum[kSegPerV][kWaves];
-    __shared__ uint32_t malformed;
+    __shared__ uint32_t malformed, escapes, bits[GROUPS * kWaves][kEndWords];
     const unsigned      t = threadIdx.x, tid = t % kSeg, lane = t % 64, v = blockIdx.x;
     const unsigned      group = __builtin_amdgcn_readfirstlane(t / kSeg);
     const uint8_t*      cb  = vbuf(page, 2, v, 0);
@@ -326,7 +365,7 @@ __global__ __launch_bounds__(kSeg* GROUPS, 8) void k_fsst_count(const uint8_t* _
         static_for<4>([&](auto k) { ends[(t >> 5) * kEndRow + ((t >> 2) & 7) * 17 + 4 * (t & 3) + k] = q[k.value]; });
         len[t] = table->len[t];
     }
-    if (t == 0) malformed = 0;
+    if (t == 0) malformed = 0, escapes = 0;
     __syncthreads();
     auto bound = [&](unsigned h) {  // of the segments
         return h ? (uint32_t)__builtin_amdgcn_readfirstlane(ends[end_place(h * kSeg - 1)]) : 0u;
@@ -346,23 +385,44 @@ __global__ __launch_bounds__(kSeg* GROUPS, 8) void k_fsst_count(const uint8_t* _
     for (unsigned h = group; h < kSegPerV; h += GROUPS) {
         const uint32_t s0 = bound(h);
         const Segment  g {cb + s0, span(h) ? bound(h + 1) - s0 : 0u, end + h * kSeg};
-        uint64_t       mine = 0;
+        uint32_t       own = 0;  // below 2^32: kMaxComp
         if (!malformed) {
             uint16_t* const at = sizes + sizes_at(page_off, page, g.seg, seg + h);
-            for (uint32_t c0 = 0; c0 < g.n; c0 += kChunk) {
-                const Granule r    = open_granule(g, c0, tid);
-                uint32_t      prev = (uint32_t)__shfl_up((int)r.wd[7], 1, 64) >> 24;  // the byte before the granule
-                if (lane == 0) prev = r.q0 && r.lim ? g.seg[r.q0 - 1] : 0u;
-                const bool special = r.lim && (prev == 255u || has_ff(r.wd));
-                uint32_t   none    = r.lim >= kShare ? 0u : ~0u << r.lim;
-                if (special) none = find_escapes(g, r).none;
-                const uint32_t size = r.lim ? granule_size(r.wd, none, len) : 0u;
-                if (r.lim) at[r.q0 / kShare] = (uint16_t)(size | (special ? kSpecial : 0u));
-                mine += size;
+            // a wave's granules follow one another, so that what a literal needs to know of the bytes before it is carried
+            // along (a walk back over its run for every granule made a segment of escapes cost the square of its length; a
+            // string of 2 MB of 255 takes 2.2 ms a call)
+            const uint32_t n = (g.n + kShare - 1) / kShare, per = ((n + kWaves - 1) / kWaves + 63) & ~63u;
+            const uint32_t first = __builtin_amdgcn_readfirstlane(tid / 64) * per, stop = first + per < n ? first + per : n;
+            bool           carry = first && first < stop && starts_on_literal(g, first, lane, bits[t / 64]);
+            for (uint32_t i = first; i < stop; i += 64) {
+                const Granule r       = open_granule(g, i * kShare, lane);
+                bool          literal = false;
+                const bool    special = r.lim && has_ff(r.wd);
+                uint32_t      none = r.lim >= kShare ? 0u : ~0u << r.lim, flags = 0;
+                if (__any(special) || carry) {
+                    const Ends     e  = window_ends(g.end, i, lane, bits[t / 64]);
+                    const uint32_t ff = ff_mask(r.wd);
+                    After          a {false, false};
+                    if (r.lim >= kShare) a = after_granule(ff, e);
+                    const uint64_t says = __ballot(!a.keeps), lit = __ballot(a.lit), before = says & ((1ull << lane) - 1);
+                    literal = before ? (lit >> (63 - __builtin_clzll(before))) & 1u : carry;
+                    carry   = says ? (lit >> (63 - __builtin_clzll(says))) & 1u : carry;
+                    if (r.lim && (special || literal)) {
+                        none  = find_escapes(ff, e, r.lim, literal).none;
+                        flags = literal ? kSpecial | kLiteral : kSpecial;
+                    }
+                    if (lane == 0) atomicOr(&escapes, 1u << h);
+                }
+                if (r.lim) {
+                    const uint32_t size = granule_size(r.wd, none, len);
+                    at[i + lane]        = (uint16_t)(size | flags);
+                    own += size;
+                }
             }
         } else {
-            mine = string_length(cb, tid ? end[h * kSeg + tid - 1] + s0 : s0, end[h * kSeg + tid] + s0, len);
+            own = string_length(cb, tid ? end[h * kSeg + tid - 1] + s0 : s0, end[h * kSeg + tid] + s0, len);
         }
+        uint64_t mine = own;
         for (unsigned d = 32; d >= 1; d >>= 1) mine += __shfl_xor((unsigned long long)mine, d, 64);
         if (lane == 0) wsum[h][tid / 64] = mine;
     }
@@ -372,7 +432,7 @@ __global__ __launch_bounds__(kSeg* GROUPS, 8) void k_fsst_count(const uint8_t* _
         for (unsigned k = 0; k < kSegPerV; ++k) {
             uint64_t all = 0;
             for (unsigned w = 0; w < kWaves; ++w) all += wsum[k][w];
-            segs[seg + k] = {all, malformed ? vec | kMalformed : vec, bound(k), span(k) ? bound(k + 1) - bound(k) : 0u};
+            segs[seg + k] = {all, vec | (malformed ? kMalformed : 0) | ((escapes >> k) & 1u ? kEscapes : 0), bound(k), span(k) ? bound(k + 1) - bound(k) : 0u};
             vec += all;
         }
         vecs[seg / kSegPerV] = vec;
@@ -436,6 +496,7 @@ __global__ __launch_bounds__(kSeg, 6) void k_fsst(const uint8_t* __restrict__ pa
     __shared__ uint32_t wsum[kWaves];
     __shared__ uint64_t wsum64[kWaves];
     __shared__ uint32_t window;
+    __shared__ uint32_t ends[kSeg + 1];  // bit j of word i: a string ends right before byte j of the chunk's granule i
     __shared__ __attribute__((aligned(16))) uint8_t image[kOutLds + 32];
     const unsigned  tid = threadIdx.x;
     const uint64_t  seg = seg0 + blockIdx.x;
@@ -454,7 +515,7 @@ __global__ __launch_bounds__(kSeg, 6) void k_fsst(const uint8_t* __restrict__ pa
         seg_base = oseg[0];
         given_ok = oseg[kSeg] >= seg_base && oseg[kSeg] - seg_base == seg_total;
     } else {
-        seg_base = st.before & ~kMalformed;
+        seg_base = st.before & ~(kMalformed | kEscapes);
         if (bases) seg_base += bases[vec];
         else
             for (uint64_t k = tid; k < vec; k += kSeg) before += vecs[k];
@@ -478,8 +539,13 @@ __global__ __launch_bounds__(kSeg, 6) void k_fsst(const uint8_t* __restrict__ pa
         uint32_t end_rel = 0;  // this string's end
         for (uint32_t c0 = 0; c0 < g.n; c0 += kChunk) {
             if (c0) r = open_granule(g, c0, tid), sz = r.lim ? size_at[r.q0 / kShare] : 0u;
-            const uint32_t size = sz & ~kSpecial;
-            uint32_t       total;
+            const uint32_t size = sz & kSize;
+            const bool     esc  = (st.before & kEscapes) != 0;  // uniform
+            if (esc) {
+                ends[tid] = 0u;
+                if (tid == 0) ends[kSeg] = 0u;
+            }
+            uint32_t total;
             const uint32_t at = block_exclusive_scan(size, wsum, &total);
             total             = __builtin_amdgcn_readfirstlane(total);  // the same in every lane: scalar from here on
             if (total > seg_total - done) {  // never more than what the capacity was tested with
@@ -487,8 +553,14 @@ __global__ __launch_bounds__(kSeg, 6) void k_fsst(const uint8_t* __restrict__ pa
                 total = (uint32_t)(seg_total - done);
             }
             if constexpr (MODE != FS_BYTES) sbase[tid] = at;
+            if (esc) {
+                const uint32_t e = end[tid] - c0;
+                if (e <= kChunk) atomicOr(&ends[e / kShare], 1u << (e % kShare));
+                __syncthreads();
+            }
             Escapes es {0, 0};
-            if (sz & kSpecial) es = find_escapes(g, r);
+            if (sz & kSpecial)
+                es = find_escapes(ff_mask(r.wd), Ends {ends[tid], (ends[tid + 1] & 1u) != 0}, r.lim, sz & kLiteral);
             else if (r.lim < kShare) es.none = ~0u << r.lim;
             const bool drops = es.none != 0;
             if (drops) static_for<8>([&](auto d) { r.wd[d] |= spread4(es.none >> (4 * decltype(d)::value)); });

@@ -299,3 +299,66 @@ def test_ends_out_of_order(torch_cuda, ends):
         if ok:
             plan.check()
             np.testing.assert_array_equal(d_bytes.cpu().numpy()[:cap], want)
+
+
+def _string_column(symbols_of, vectors):
+    """A one-page column of given code streams (1024 rows of bytes a vector) under another column's symbol table."""
+    _, page, _ = _string_page(symbols_of)
+    k = np.arange(1024)
+    place = 128 * (k % 8) + 16 * np.array([0, 4, 2, 6, 1, 5, 3, 7])[(k // 8) % 8] + k // 64
+    data, ends, eps = [], [], []
+    for v, rows in enumerate(vectors):
+        if v:
+            eps += [sum(len(d) for d in data), 4096 * v]
+        data.append(b"".join(rows))
+        e = np.zeros(1024, np.uint32)
+        e[place] = np.cumsum([len(r) for r in rows])
+        ends.append(e.tobytes())
+    n, total = len(vectors), sum(len(d) for d in data)
+    head = bytes([7, 1, 0, 0, n & 255, n >> 8, 0, 0]) + np.array([8 + 8 * n, 8 + 8 * n + total, *eps], np.uint32).tobytes()
+    return np.frombuffer(symbols_of[:page].tobytes() + head + b"".join(data) + b"".join(ends), np.uint8).copy()
+
+
+@pytest.mark.parametrize("shape", ["one_run", "dense", "denser", "aligned"])
+def test_escape_runs(torch_cuda, shape):
+    """Whether a 32-byte piece of a segment starts on an escape's literal depends on the run of 255 bytes before it: one run
+    of 200 KB inside a string (and one of odd length), streams of mostly 255 over strings of all lengths, and runs that
+    begin and end at string ends on 32-byte and 2 KiB places. All three call forms against the codes' definition."""
+    torch = torch_cuda
+    g = np.random.default_rng(len(shape))
+    words, _ = wl.vocab_strings(1024, seed=2)
+    table = fa.encode_strings(words.astype(np.uint32), wl.vocab_strings(1024, seed=2)[1])
+    symbols, _, _ = _string_page(table)
+    symbols += [bytes([(32774747032022883 >> (8 * b)) & 255 for b in range(8)])] * (255 - len(symbols))  # codes without one
+
+    def stream(n, p):
+        b = g.integers(0, 255, n, dtype=np.uint8)
+        b[g.random(n) < p] = 255
+        return b.tobytes()
+
+    vectors = []
+    for v in range(2):
+        if shape == "one_run":
+            rows = [stream(int(g.integers(0, 30)), 0.05) for _ in range(1024)]
+            rows[300 + v], rows[700] = stream(37, 0.1) + b"\xff" * 200_000 + b"abc", b"\xff" * 70_001 + stream(50, 0.2)
+        elif shape == "aligned":
+            rows = [(b"\xff" if g.random() < 0.8 else b"a") * int(32 * g.integers(0, 4) * (64 if i % 97 == 0 else 1)) for i in range(1024)]
+        else:
+            p = 0.5 if shape == "dense" else 0.97
+            rows = [stream(int(g.integers(0, 120 if i % 50 else 9000)), p) for i in range(1024)]
+        vectors.append(rows)
+    enc = _string_column(table, vectors)
+    want_off, want = _strs_from([r for rows in vectors for r in _decode_vector(
+        symbols, np.frombuffer(b"".join(rows), np.uint8), np.cumsum([len(r) for r in rows]))])
+    print(f"fsst escape runs {shape}: {enc.size} bytes, {want.size} decoded", flush=True)
+    plan, d_in, n = fa.Plan(enc, "str"), dev(torch, enc), want_off.size - 1
+    got_off, got = _fused(torch, plan, d_in, n, want.size)
+    np.testing.assert_array_equal(got_off, want_off)
+    np.testing.assert_array_equal(got[: want.size], want)
+    d_off = torch.zeros(n + 1, dtype=torch.int64, device="cuda")
+    plan.string_offsets(d_in.data_ptr(), d_off.data_ptr())
+    np.testing.assert_array_equal(d_off.cpu().numpy(), want_off)
+    d_bytes = empty(torch, want.size)
+    plan.decode_strings(d_in.data_ptr(), d_off.data_ptr(), d_bytes.data_ptr(), want.size)
+    plan.check()
+    np.testing.assert_array_equal(d_bytes.cpu().numpy()[: want.size], want)
