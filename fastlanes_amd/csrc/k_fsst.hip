@@ -21,8 +21,9 @@
 // instructions per code, measured 135 us: unaligned LDS writes take about one cycle per lane.) Escapes are found from two
 // 32-bit masks of a granule, its bytes of 255 and the strings' ends in it; while every thread looked its ends up and walked
 // its escapes, a column with 3% of its bytes escaped took 102 us where it now takes 85. 2^21 strings: 151 -> 71 us
-// a call, k_fsst 42, bound by its vector instructions. No variable of k_fsst may spill: a build whose registers did gave
-// wrong bytes in a hundredth of the segments.
+// a call, k_fsst 42, bound by its vector instructions. The build refuses a k_fsst that spills registers: two
+// intermediate forms of it that did (to scratch) gave wrong bytes in a hundredth of the segments, others from run to run; what
+// made the difference is not known.
 // A vector with a malformed segment (non-monotone offsets) takes a per-string path that reads and writes global memory byte
 // by byte, for all four of its segments: the granules' sizes are kept by byte position, which is one segment's own only
 // while no segment of the vector reaches back over another.
