@@ -84,12 +84,6 @@ struct EncSum {
     uint64_t bits, runs;
 };
 
-// Base and bit width of one vector's FFOR (MODE 1: of the values, MODE 2: of their differences from the previous value
-// inside the aligned W-value segment, 0 at a segment start -- the unrsum of the transposed lane order): base = min,
-// bw = bit length of max - min. SGN: min and max of int64 columns compare as signed values
-// (ffor_prm::ResolveAnalyzeFunc, src/cor/prm/ffor/ffor_analyze.cpp:145-160), done here on the values with their sign
-// bit flipped. A wave reads its vector with 1 KiB loads and has the next vector's in flight; a lane's first
-// difference needs its neighbour's last value, which a shuffle brings (a 1 KiB chunk starts a segment in every type).
 // The block's bit widths and run counts summed for the layout; `b` and `r` are lane 0's sums of the wave.
 __device__ __forceinline__ void group_sum(uint32_t b, uint32_t r, EncSum* sums) {
     __shared__ uint32_t wb[kEncMaxWaves], wr[kEncMaxWaves];
@@ -101,6 +95,12 @@ __device__ __forceinline__ void group_sum(uint32_t b, uint32_t r, EncSum* sums) 
         sums[blockIdx.x] = s;
     }
 }
+// Base and bit width of one vector's FFOR (MODE 1: of the values, MODE 2: of their differences from the previous value
+// inside the aligned W-value segment, 0 at a segment start -- the unrsum of the transposed lane order): base = min,
+// bw = bit length of max - min. SGN: min and max of int64 columns compare as signed values
+// (ffor_prm::ResolveAnalyzeFunc, src/cor/prm/ffor/ffor_analyze.cpp:145-160), done here on the values with their sign
+// bit flipped. A wave reads its vector with 1 KiB loads and has the next vector's in flight; a lane's first
+// difference needs its neighbour's last value, which a shuffle brings (a 1 KiB chunk starts a segment in every type).
 template <typename T, int MODE, bool SGN>
 __global__ __launch_bounds__(64 * kEncMaxWaves) void k_enc_analyze(const T* __restrict__ x, uint32_t n_vec,
                                                                 uint8_t* __restrict__ bw, uint64_t* __restrict__ base,

@@ -89,14 +89,17 @@ int fls_gpu_selection_and(const uint64_t* dev_a, const uint64_t* dev_b, uint64_t
  * pool expression 0 (UNCOMPRESSED), 1 (FFOR), 11 (DELTA), 6 or 7 (RLE) into dev_out, the same bytes encode_from_memory writes
  * for those values. *out_size receives the encoded size (also when it exceeds `capacity`, which returns
  * FLS_E_CAPACITY and writes nothing). The pages are laid out on the device and only the size is read back, so it
- * returns after `stream` has completed. */
+ * returns after `stream` has completed. It works on the stream's device, whichever is current; its scratch is one of
+ * four slots there (up to 2^18 vectors a call; a first call on a device pins 64 bytes of host memory) or a stream
+ * allocation. */
 int fls_gpu_encode(const void* dev_values, uint64_t n, enum data_t type, uint8_t expr_id, uint8_t* dev_out,
                    uint64_t capacity, uint64_t* out_size, void* stream);
 /* fls_gpu_encode without device allocation. No counterpart in the reference: it is for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * The encoder's scratch (per-vector bit widths, bases, their sums and the page table) is a fixed device array
  * of about 160 KiB per GPU, kept until the process ends, instead of stream allocations; n is at most 2^24 values
- * (FLS_E_CAPACITY beyond). Every call on one GPU shares that GPU's array: calls that overlap on one GPU race.
+ * (FLS_E_CAPACITY beyond). Every call on one GPU shares that GPU's array: calls that overlap on one GPU race. Host
+ * memory is not allocated or pinned either.
  * Same bytes, errors and synchronization as fls_gpu_encode. */
 int fls_gpu_encode_noalloc(const void* dev_values, uint64_t n, enum data_t type, uint8_t expr_id, uint8_t* dev_out,
                            uint64_t capacity, uint64_t* out_size, void* stream);
@@ -125,6 +128,7 @@ int fls_gpu_unffor_stream(unsigned width, unsigned bw, const void* dev_packed, c
  * nontemporal: bit 0 = non-temporal stores; bit 1 = direct stores of each lane's segment instead of staging the
  * output through LDS (families 1-3 with 32-bit values, family 8 with 64-bit values); bit 2 (family 4, 8/16-bit
  * values) = decode position lanes 2 per thread with staging instead of one per thread with direct stores.
+ * Family 5 caps the grid of 32/64-bit values only where the dictionary goes to LDS (at most 32 KiB).
  * family 6 is the row-group launch: block = KiB of decoded values per tile, max_blocks = blocks per compute unit
  * (0: as many as stay resident at once, each wave then owning one long run of the work list).
  * fls_gpu_tune_get reads the shape in effect for (family, width, bw); any output pointer may be NULL. */

@@ -1,5 +1,4 @@
-"""One-pass FSST decode (offsets and bytes from one launch per page, segment bases by decoupled look-back) against
-the oracle, bit-exact: vocabulary strings, escape runs, empty and long strings, the reference's own FSST table,
+"""FSST decode of offsets and bytes in one call (sizes counted first, then segments joined) against the oracle, bit-exact: vocabulary strings, escape runs, empty and long strings, the reference's own FSST table,
 repeated calls on one plan mixed with the two-step form, and the capacity error."""
 import numpy as np
 import pytest
