@@ -22,7 +22,7 @@ import numpy as np
 import fastlanes_amd as fa
 from fastlanes_amd import workloads as wl
 
-FAM_STREAM, FAM_UNC, FAM_FFOR, FAM_DELTA, FAM_RLE, FAM_DICT, FAM_ROWGROUP, FAM_PATCH, FAM_RLE_POS = range(9)
+FAM_STREAM, FAM_UNC, FAM_FFOR, FAM_DELTA, FAM_RLE, FAM_DICT, FAM_ROWGROUP, FAM_PATCH, FAM_RLE_POS, FAM_PATCH_SB = range(10)
 RG_TILE_KIB = (16, 32, 64, 128)
 RG_CU_BLOCKS = (0, 8, 16, 32, 64, 128)  # 0 = resident blocks only (one long run per wave)
 BLOCKS = (128, 256, 512)
@@ -127,7 +127,8 @@ def main():
                 x = rng.integers(0, 1 << 7, m, dtype=dt)
                 hit = rng.random(m) < 0.01
                 x[hit] = rng.integers(0, np.iinfo(dt).max, int(hit.sum()), dtype=dt)
-                cases[FAM_PATCH] = (2, x)
+                cases[FAM_PATCH] = (5, x)
+                cases[FAM_PATCH_SB] = (2, x)
                 cases[FAM_RLE_POS] = (7, cases[FAM_RLE][1])
             for fam, (eid, x) in cases.items():
                 enc = fa.encode_from_memory(x, eid)

@@ -19,6 +19,16 @@ std::mutex                                          g_tune_mu;
 std::map<std::tuple<int, unsigned, unsigned>, Tune> g_tune;
 std::once_flag                                      g_tune_once;
 
+// The family whose entry serves where `family` has none (-1: no other).
+int general_family(int family) {
+    switch (family) {
+    case FAM_PAGE_PATCH_SB: return FAM_PAGE_PATCH;
+    case FAM_PAGE_PATCH: return FAM_PAGE_FFOR;
+    case FAM_PAGE_RLE_POS: return FAM_PAGE_RLE;
+    default: return -1;
+    }
+}
+
 // The tuning table shipped next to the library (or named by FLS_TUNING) is loaded on first use.
 void load_default_tuning() {
     const char* env = std::getenv("FLS_TUNING");
@@ -42,9 +52,8 @@ Tune tune_for(int family, unsigned W, unsigned bw) {
     if (it != g_tune.end()) return it->second;
     it = g_tune.find({family, W, 255u});
     if (it != g_tune.end()) return it->second;
-    const int general = family == FAM_PAGE_PATCH ? FAM_PAGE_FFOR : family == FAM_PAGE_RLE_POS ? FAM_PAGE_RLE : -1;
-    if (general >= 0) {
-        it = g_tune.find({general, W, 255u});
+    while ((family = general_family(family)) >= 0) {
+        it = g_tune.find({family, W, 255u});
         if (it != g_tune.end()) return it->second;
     }
     return Tune {};
@@ -52,8 +61,9 @@ Tune tune_for(int family, unsigned W, unsigned bw) {
 void tune_set(int family, unsigned W, unsigned bw, Tune t) {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tune[{family, W, bw}] = t;
-    if (family == FAM_PAGE_FFOR) g_tune.erase({FAM_PAGE_PATCH, W, bw});
-    if (family == FAM_PAGE_RLE) g_tune.erase({FAM_PAGE_RLE_POS, W, bw});
+    for (int f = 0; f < FAM_COUNT; ++f)
+        for (int g = general_family(f); g >= 0; g = general_family(g))
+            if (g == family) g_tune.erase({f, W, bw});
 }
 int tune_load(const char* path) {
     FILE* f = std::fopen(path, "r");

@@ -24,6 +24,7 @@ enum Family : int {
     FAM_PAGE_PATCH,   // patched FFOR-shaped pages (without an entry of their own: as FAM_PAGE_FFOR)
     FAM_PAGE_RLE_POS, // RLE pages of 32/64-bit values with plain positions or differences of more than one bit (without an
                       // entry of their own: as FAM_PAGE_RLE)
+    FAM_PAGE_PATCH_SB,// S and B patches of plain FFOR pages, decoded (without an entry of their own: as FAM_PAGE_PATCH)
     FAM_COUNT
 };
 
@@ -35,8 +36,8 @@ struct Tune {
     uint32_t max_blocks = 0;
 };
 Tune tune_for(int family, unsigned W, unsigned bw);
-// Setting FAM_PAGE_FFOR or FAM_PAGE_RLE drops the width's entry of the family that falls back on it: it covers those pages
-// too until theirs is set again.
+// Setting a family that others fall back on drops the width's entries of those: it covers their pages too until they are
+// set again.
 void tune_set(int family, unsigned W, unsigned bw, Tune t);  // bw 255 = every bit width
 int  tune_load(const char* path);                             // returns entries read, <0 on error
 

@@ -123,8 +123,9 @@ int fls_gpu_unffor_stream(unsigned width, unsigned bw, const void* dev_packed, c
  * The decoder reads a table of launch shapes (threads per block, non-temporal stores, grid cap) from tuning.txt
  * next to the library (or the file named by FLS_TUNING) on first use; fastlanes_amd/autotune.py measures and writes
  * it. family: 0 raw streams, 1 UNCOMPRESSED, 2 FFOR, 3 DELTA, 4 RLE, 5 dictionary pages, 7 patched pages, 8 RLE pages of
- * 32/64-bit values with plain positions or differences of more than one bit; bw 255 = all bit widths. 7 and 8 are 2 and 4
- * where they have no entry; setting 2 or 4 for a width drops its entry of 7 or 8.
+ * 32/64-bit values with plain positions or differences of more than one bit, 9 S and B patches of plain FFOR pages
+ * (decoded); bw 255 = all bit widths. Without an entry 9 is as 7, 7 as 2 and 8 as 4; setting one of those for a width
+ * drops the width's entries of the families that fall back on it.
  * nontemporal: bit 0 = non-temporal stores; bit 1 = direct stores of each lane's segment instead of staging the
  * output through LDS (families 1-3 with 32-bit values, family 8 with 64-bit values); bit 2 (family 4, 8/16-bit
  * values) = decode position lanes 2 per thread with staging instead of one per thread with direct stores.

@@ -29,6 +29,10 @@ def grid(e, family=None, cap=0):
     launches()
     plans[e].decode(4096, 4096, x.nbytes)
     return launches()[-1][1:3]
+def select(e):
+    launches()
+    plans[e].select(4096, "<", np.int64(5), 4096, 4096)
+    return launches()[-1][1:3]
 """
 
 
@@ -36,13 +40,15 @@ def test_patched_pages_have_their_own_launch_shape(hip):
     """Patched pages of 64-bit values take the shape that the table or a caller names for them (no cap of their own besides),
     and follow an FFOR setting made after theirs, as before they had an entry."""
     got = host_hip.run(hip, GRIDS.replace("EXPRS", "(1, 2, 4, 5, 12)") + """
-result = {"shipped": [grid(e) for e in (2, 4, 5, 12)], "ffor": grid(1)}
-result["own"] = [grid(e, 7, 0) for e in (2, 4, 5, 12)]
+result = {"shipped": [grid(e) for e in (2, 4, 5, 12)], "predicate": select(2), "ffor": grid(1)}
+result["own"] = [grid(e, 7, 600) for e in (2, 4, 5, 12)]
+result["s and b"] = [grid(2, 9, 300), grid(4), grid(5), grid(12)]
 result["ffor after own"] = grid(1)
 result["by ffor"] = [grid(e, 2, 700) for e in (2, 4, 5, 12)]
 """)
-    assert got["shipped"] == [[1024, 64]] * 4 and got["ffor"] == [2500, 128]
-    assert got["own"] == [[1250, 64]] * 4 and got["ffor after own"] == [2500, 128]
+    assert got["shipped"] == [[1250, 64]] * 2 + [[1024, 64]] * 2 and got["predicate"] == [1024, 64] and got["ffor"] == [2500, 128]
+    assert got["own"] == [[600, 64]] * 4 and got["s and b"] == [[300, 64]] * 2 + [[600, 64]] * 2
+    assert got["ffor after own"] == [2500, 128]
     assert got["by ffor"] == [[700, 64]] * 4
 
 
@@ -52,7 +58,7 @@ def test_plain_position_pages_have_their_own_launch_shape(hip):
 result = {"shipped": [grid(6), grid(7)], "own": grid(7, 8, 300), "rle after own": grid(6), "by rle": grid(7, 4, 200)}
 """)
     rle, pos = got["shipped"]
-    assert pos[0] == 512 and rle == [2500, 128]
+    assert pos == [2500, 64] and rle == [2500, 128]
     assert got["own"][0] == 300 and got["rle after own"] == rle and got["by rle"][0] == 200
 
 
