@@ -702,7 +702,8 @@ int enc_device(int dev, bool noalloc) {
 }
 
 // The stream's device, made current for as long as this lives: the scratch and the kernels belong to it, whichever device
-// the caller has current (the null stream is that one's).
+// the caller has current (the null stream, hipStreamLegacy and hipStreamPerThread are that one's; hipStreamGetDevice takes the
+// second of them for a pointer).
 struct StreamDevice {
     int        dev = 0, before = 0;
     hipError_t err;
@@ -710,7 +711,7 @@ struct StreamDevice {
         if ((err = hipGetDevice(&before)) != hipSuccess) return;
         dev = before;
         hipDevice_t d = (hipDevice_t)before;
-        if (s && hipStreamGetDevice(s, &d) != hipSuccess) (void)hipGetLastError(), d = (hipDevice_t)before;
+        if (s && s != hipStreamLegacy && s != hipStreamPerThread && hipStreamGetDevice(s, &d) != hipSuccess) (void)hipGetLastError(), d = (hipDevice_t)before;
         if ((int)d != before && (err = hipSetDevice((int)d)) == hipSuccess) dev = (int)d;
     }
     ~StreamDevice() {

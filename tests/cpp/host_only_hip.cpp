@@ -1,6 +1,7 @@
 // A HIP runtime without a GPU, for tests of what the host side asks of the device: device memory is host memory, kernels
 // are not run, and every launch and allocation is written down. Preloaded before libfastlanes_amd.so (tests/host_hip.py).
-// Streams are numbers: stream 0x100 * k + n belongs to device k, the null stream to the current device.
+// Streams are numbers: stream 0x100 * k + n belongs to device k; the null stream (0), hipStreamLegacy (1) and
+// hipStreamPerThread (2) to the current device.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
@@ -31,7 +32,7 @@ void                                                  say(const char* what, unsi
     std::snprintf(t, sizeof t, "%s %llu\n", what, a);
     log_ += t;
 }
-int device_of(hipStream_t s) { return s ? (int)((uintptr_t)s >> 8) : current; }
+int device_of(hipStream_t s) { return (uintptr_t)s > 2 ? (int)((uintptr_t)s >> 8) : current; }
 }  // namespace
 
 extern "C" {
@@ -62,7 +63,10 @@ hipError_t hipGetLastError() { return hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "error"; }
 hipError_t hipGetDevice(int* d) { return *d = current, hipSuccess; }
 hipError_t hipSetDevice(int d) { return current = d, hipSuccess; }
-hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) { return *d = device_of(s), hipSuccess; }
+hipError_t hipStreamGetDevice(hipStream_t s, hipDevice_t* d) {
+    if (s == hipStreamLegacy) std::abort();  // the real one takes the handle for a pointer
+    return *d = device_of(s), hipSuccess;
+}
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
     std::memset(p, 0, sizeof *p);
     p->multiProcessorCount = 256, p->sharedMemPerBlock = 160 << 10, p->maxThreadsPerMultiProcessor = 2048;

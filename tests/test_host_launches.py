@@ -95,3 +95,15 @@ for fn, n in (("fls_gpu_encode_noalloc", 64), ("fls_gpu_encode", 64), ("fls_gpu_
     result.append([sorted(where), current()])
 """)
     assert got == [[[2], 0]] * 3
+
+
+def test_encoder_takes_the_special_streams(hip):
+    """The null stream, hipStreamLegacy and hipStreamPerThread are the current device's (1 here)."""
+    got = host_hip.run(hip, ENCODE + """
+_h.hipSetDevice(1)
+result = []
+for s in (0, 1, 2):
+    for fn in ("fls_gpu_encode_noalloc", "fls_gpu_encode"):
+        result.append(sorted({int(x[1].split()[-1]) for x in encode(fn, 64, s) if x[0] == "launch"}) + [current()])
+""")
+    assert got == [[1, 1]] * 6
